@@ -380,13 +380,17 @@ __global__ void k_scan_bsum(int* bsum, const Grid* __restrict__ gp, int* total_o
   b_scan_bsum(bsum, gp, total_out, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-__device__ __forceinline__ void b_scan_add(int* out, const int* bsum, const Grid* __restrict__ gp, VL vl) {
+// block offsets onto the cell starts; clears the cells' largest list radii
+// (raised by k_pack_density)
+__device__ __forceinline__ void b_scan_add(KArgs a, const int* bsum, const Grid* __restrict__ gp, VL vl) {
   const long long n = gp->ncell + 1;
   long long idx = (long long)vl.b * blockDim.x + threadIdx.x;
-  if (idx < n) out[idx] += bsum[idx / (BS * 4)];
+  if (idx >= n) return;
+  a.cstart[idx] += bsum[idx / (BS * 4)];
+  if (a.cellr) a.cellr[idx] = 0.0f;
 }
-__global__ void k_scan_add(int* out, const int* bsum, const Grid* __restrict__ gp) {
-  b_scan_add(out, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ void k_scan_add(KArgs a, const int* bsum, const Grid* __restrict__ gp) {
+  b_scan_add(a, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 __device__ __forceinline__ void b_scatter(KArgs a, VL vl) {
@@ -525,9 +529,13 @@ __device__ __forceinline__ void b_pack_density(KArgs a, Phys p, VL vl) {
   alignas(32) __shared__ float4 stage[BS * dr_bytes<PT>(true) / 16];
   const int rb = dr_bytes<PT>(p.idust != 0);
   const int k0 = vl.b * blockDim.x, k = k0 + threadIdx.x;
+  int cell = -1;
+  float rl = 0.0f;
   if (k < a.n) {
     int i = a.sidx[k];
     double h = a.f[F_H][i];
+    cell = a.cellid[i];
+    rl = (float)(p.radkern * (1.0 + p.skin) * h) * (1.0f + 1.0e-6f);
     const double4 pk = make_double4(a.f[F_X][i], a.f[F_Y][i], a.f[F_Z][i], 1.0 / h);
     a.P4[k] = pk;
     a.dxb[k] = p.radkern * h;
@@ -539,6 +547,18 @@ __device__ __forceinline__ void b_pack_density(KArgs a, Phys p, VL vl) {
     // the density sums read the dust fraction of the last conservative2primitive
     // (dustfrac, src/density_sums.f90:276-278), not the predicted dustevol
     if (p.idust) R[1] = T4{(PT)a.f[F_DUSTFRAC][i], PT(0), PT(0), PT(0)};
+  }
+  if (a.cellr) {
+    // largest list radius of each cell (the list builder's cell test): the
+    // maximum over a wave's run of equal cells, then one atomic per run
+    // (non-negative floats compare as their bits do)
+    const int lane = threadIdx.x & 63;
+    for (int o = 1; o < 64; o <<= 1) {
+      const float y = __shfl_down(rl, o);
+      if (__shfl_down(cell, o) == cell && lane + o < 64) rl = fmaxf(rl, y);
+    }
+    const int prev = __shfl_up(cell, 1);
+    if (cell >= 0 && (lane == 0 || prev != cell)) atomicMax((unsigned*)&a.cellr[cell], __float_as_uint(rl));
   }
   __syncthreads();
   flush_records((char*)a.DR + (size_t)k0 * rb, stage, min((int)blockDim.x, a.n - k0), rb);
@@ -783,20 +803,19 @@ __device__ __forceinline__ void for_each_candidate_rec(const KArgs& a, const Gri
 // sits at nbl[k*maxnb + m] = (sorted index << 7) | image code.  Entries
 // [0, nbc) are the gather list G(k): every image of a particle j with
 // r_kj < radkern*h_k*(1+skin), in the candidate order of the cell scan; then
-// nbx transposed extras: every image of j whose opposite image of k is in
-// G(j) while it is not in G(k) itself.  Together they hold every pair (and
-// pair of periodic images) with r < radkern*max(h_k, h_j) while no h has
-// grown past hcap = h*(1+skin).  Membership uses the separation
-// fl(x_k - x_j) + s L per dimension, the shift s = +1, -1 or 0 given by the
-// image code, summed without contraction: it is exactly antisymmetric in
-// FP64 (fl(a - b) = -fl(b - a), and the shifts of two opposite images are
-// exact negatives), so "k in G(j)" is decided identically from k's and from
-// j's side and no pair is lost or doubled.  Lists need
-// radkern*hmax*(1+skin) < L along periodic dimensions (checked on the device
-// at every binning), so every image within a list radius lies in the image
-// cells one period away; where 2*radkern*hmax*(1+skin) >= L a list can hold
-// two images of one neighbour, or an image of the particle itself, as the
-// reference's ghost copies interact (src/ghostND_mhd.f90:180-200).
+// nbx extras: every image of j with r_kj < radkern*h_j*(1+skin) that is not in
+// G(k).  Together they hold every pair (and pair of periodic images) with
+// r < radkern*max(h_k, h_j) while no h has grown past hcap = h*(1+skin).
+// Membership uses the separation fl(x_k - x_j) + s L per dimension, the shift
+// s = +1, -1 or 0 given by the image code, summed without contraction: it is
+// exactly antisymmetric in FP64 (fl(a - b) = -fl(b - a), and the shifts of two
+// opposite images are exact negatives), so a pair is decided identically from
+// both of its sides.  Lists need radkern*hmax*(1+skin) < L along periodic
+// dimensions (checked on the device at every binning), so every image within
+// a list radius lies in the image cells one period away; where
+// 2*radkern*hmax*(1+skin) >= L a list can hold two images of one neighbour, or
+// an image of the particle itself, as the reference's ghost copies interact
+// (src/ghostND_mhd.f90:180-200).
 template <int NDIM>
 __device__ __forceinline__ double image_r2(const Grid& g, const double* xa, const double* xb, unsigned code) {
 #pragma clang fp contract(off)
@@ -819,46 +838,111 @@ __device__ __forceinline__ void st_stream(double* p, double v) { __builtin_nonte
 
 // a value every lane of the wave holds, moved to scalar registers (frees
 // vector registers in the register-bound list builder)
+__device__ __forceinline__ float wave_uniform(float v) {
+  return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
 __device__ __forceinline__ double wave_uniform(double v) {
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_readfirstlane((int)(unsigned)(b & 0xffffffffll));
   const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
 }
-__device__ __forceinline__ int wave_min_i(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-  return v;
+
+// Scans and folds over a wave with DPP moves (row shifts by 1, 2, 4 and 8, then
+// the two row broadcasts): a few cycles a step where a shuffle through LDS
+// takes about a hundred.  After the steps lane 63 holds the fold of all lanes.
+#define NDSP_DPP_STEPS(STEP)                                                   \
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf)          \
+  STEP(0x142, 0xa) STEP(0x143, 0xc)
+__device__ __forceinline__ int wave_scan_add(int x) {
+#define NDSP_STEP(ctrl, rows) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false);
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  return x;
 }
-__device__ __forceinline__ int wave_max_i(int v) {
-  for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o));
-  return v;
+// largest of the lanes' non-negative values
+__device__ __forceinline__ float wave_max_pos(float v) {
+  int x = __float_as_int(v);
+#define NDSP_STEP(ctrl, rows) x = max(x, __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false));
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  return __int_as_float(__builtin_amdgcn_readlane(x, 63));
+}
+// smallest / largest of the lanes' values
+template <bool MAX>
+__device__ __forceinline__ double wave_extreme(double v) {
+#define NDSP_STEP(ctrl, rows)                                                                          \
+  {                                                                                                    \
+    const long long b = __double_as_longlong(v);                                                       \
+    const int l = (int)(unsigned)(b & 0xffffffffll), h = (int)(b >> 32);                               \
+    const unsigned pl = (unsigned)__builtin_amdgcn_update_dpp(l, l, ctrl, rows, 0xf, false);           \
+    const int ph = __builtin_amdgcn_update_dpp(h, h, ctrl, rows, 0xf, false);                          \
+    const double w = __longlong_as_double(((long long)ph << 32) | (long long)pl);                      \
+    v = MAX ? fmax(v, w) : fmin(v, w);                                                                 \
+  }
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffll), 63);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (long long)lo);
 }
 
-// One wavefront per 64 consecutive sorted particles (a compact group: the
-// order is by Morton cell key).  The wave enumerates the cells of the union
-// of its particles' gather boxes (rows (cy, cz) cut to the union of the
-// particles' chords), in the nested order of for_each_candidate, so each
-// list keeps the scan's candidate order.  For a batch of up to NBL_CELLS
-// cells it loads all cell ranges at once, forms their prefix sums in LDS,
-// and then streams the batch's candidates 64 at a time through LDS (the next
-// 64 are fetched while the current ones are tested): FP64 raw positions for
-// the exact test and FP32 image positions relative to the wave's first
-// particle for a screening test.  A decision of the FP32 test taken outside
-// a narrow band around the radius (its width bounded by the FP32 rounding,
-// see below) is the FP64 test's decision; a candidate inside the band takes
-// the exact FP64 image test.  A pair k-j with j in G(k) and k not in G(j) is
-// appended to the extras of j, which fill j's row from its end
-// (k_nblist_sort moves them into place).
-#define NBL_CELLS 128
+// One wavefront per 64 consecutive sorted particles.  The order is by Morton
+// cell key, so most groups are compact, but a group may straddle a jump of
+// the curve; it is cut there into segments of neighbouring lanes, and each
+// segment builds its lists from its own box.
+//
+// A segment's candidates pass three stages:
+//  1. cells: each lane takes one cell at a time of the box widened by the
+//     largest list radius, in the nested order of for_each_candidate; a cell
+//     is kept when its distance to the box is below the largest list radius of
+//     the segment or of the cell (a.cellr); the kept cells' particles are
+//     queued in LDS as list entries.
+//  2. candidates: the queue, 64 at a time (the next 64 positions are fetched
+//     while the current ones are tested); those within the larger of the
+//     segment's and their own list radius of the box are staged, in order, as
+//     FP32 positions relative to the box centre.
+//  3. test: every 64 staged candidates against every lane's particle, a Gram
+//     product on the matrix cores (v_mfma_f32_16x16x4_f32): candidate rows
+//     (-2c, |c|^2) times particle columns (x, 1) plus |x|^2 - R_k^2 is
+//     r^2 - R_k^2 (negative when k's list radius holds j), rows
+//     (-2c, |c|^2 - R_j^2) plus |x|^2 give r^2 - R_j^2 (when j's holds k).  Their
+//     sign bits are shifted into two masks, four VALU instructions per
+//     candidate with the band test (11 and a broadcast LDS read with separations
+//     formed lane by lane).  The first masks of up to NBL_CAP candidates are kept in LDS and
+//     popped together, when the lanes' hit counts have evened out (per 64
+//     candidates the fullest lane holds about three times the mean); four
+//     entries are stored at a time.
+// Each particle finds both parts of its own list, so nothing is written into
+// another particle's row.
+//
+// FP32 screening: a segment's particles lie within P (half its box's diagonal)
+// of the box centre, its staged candidates within P + Rm (Rm the largest list
+// radius met).  With u = 2^-24 and S = 2P + Rm, rounding the positions, the
+// squares and the product's five terms misses r^2 - R^2 by less than 16u S^2,
+// so outside a band of 33u S^2 the sign is the FP64 test's.  Where some value of
+// the 64 x 64 falls inside the band, every candidate within twice the band
+// of a threshold takes the exact FP64 image test.
+//
+// Bound by VALU issue on large runs and by the latency of one wave on small
+// ones.  128^3, one cell per radius: 1.26 ms; 2.02 ms with a builder that
+// scanned rows of cells lane by lane, wrote the extras into other particles'
+// rows with atomics and sorted them in a launch of its own.  61^3, two cells
+// per radius: 0.29 ms instead of 0.97 (there a group on a jump of the curve
+// walked every row of cells of the box in one wave).  Queue and cap trade LDS
+// (four waves per SIMD need 10 KB a wave) against partly filled rounds: 512 and
+// 384 take 1.26 ms, 256 and 512 1.30, 512 and 256 1.32.
+typedef float nbl_f32x4 __attribute__((ext_vector_type(4)));
+#define NBL_CAP 384    // candidates whose masks are held before they are popped (a multiple of 128)
+#define NBL_QUEUE 512  // list entries expanded at a time
 template <int NDIM>
 __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict__ gp, VL vl) {
-  __shared__ double4 sraw[128];
-  __shared__ float4 srel[128];
-  __shared__ unsigned se[128];
-  __shared__ int ckey[NBL_CELLS];
-  __shared__ int ccode[NBL_CELLS];
-  __shared__ int cbeg[NBL_CELLS];
-  __shared__ int cpre[NBL_CELLS + 1];
+  // staged candidates: -2c, |c|^2, |c|^2 - R_j^2 (a ring over the staged index)
+  __shared__ float sc[5][128];
+  __shared__ unsigned se[NBL_CAP + 64];  // staged entries
+  __shared__ unsigned smask[NBL_CAP / 32][64];
+  __shared__ unsigned sq[NBL_QUEUE];
   const int lane = threadIdx.x;
   const int k = xcd_tile(vl) * 64 + lane;
   const bool act = k < a.n;
@@ -869,330 +953,342 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
   const Grid g = *gp;
   const double s1 = 1.0 + p.skin;
   const double lim2 = p.radkern2 * s1 * s1 * (1.0 + 1.0e-12);
-  const double4 pk = a.P4[act ? k : 0];
-  const double xi[3] = {pk.x, pk.y, pk.z};
-  const double hi21 = pk.w * pk.w;
-  const double rad = act ? p.radkern * s1 * (1.0 + 1.0e-9) / pk.w : 0.0;
-  const double rad2 = rad * rad * (1.0 + 1.0e-12);
-  const double org[3] = {wave_uniform(__shfl(xi[0], 0)), wave_uniform(__shfl(xi[1], 0)),
-                          wave_uniform(__shfl(xi[2], 0))};
-  const float xr0 = (float)(xi[0] - org[0]);
-  const float xr1 = NDIM >= 2 ? (float)(xi[1] - org[1]) : 0.f;
-  const float xr2 = NDIM >= 3 ? (float)(xi[2] - org[2]) : 0.f;
-  unsigned* L = a.nbl + (size_t)(act ? k : 0) * a.maxnb;
-  int cnt = 0;
-  bool over = false;
-  // box of the group's particles and the largest search radius
-  // (candidates are kept within that radius of the box itself, which drops
-  // the corners of the widened box: about a fifth of them)
-  double gbox_lo[3], gbox_hi[3], rw2;
-  {
-    double rw = rad;
-    for (int o = 32; o > 0; o >>= 1) rw = fmax(rw, __shfl_xor(rw, o));
-    rw *= 1.0 + 1.0e-9;
-    rw2 = wave_uniform(rw * rw);
-    for (int d = 0; d < 3; d++) {
-      double lo_ = act ? xi[d] : DBL_MAX, hi_ = act ? xi[d] : -DBL_MAX;
-      for (int o = 32; o > 0; o >>= 1) {
-        lo_ = fmin(lo_, __shfl_xor(lo_, o));
-        hi_ = fmax(hi_, __shfl_xor(hi_, o));
-      }
-      gbox_lo[d] = wave_uniform(lo_);
-      gbox_hi[d] = wave_uniform(hi_);
-    }
-  }
-  int fill = 0;  // staged candidates awaiting the test (wave-uniform)
+  const float limf = (float)sqrt(lim2);
+  // the widest search: the largest h of the binning
+  const double rmax = p.radkern * s1 * (1.0 + 1.0e-6) * a.sc->hmax_bin;
+  const int maxnb = a.maxnb;
+  unsigned* const L = a.nbl + (size_t)(act ? k : 0) * maxnb;
+  int cnt = 0, nx = 0;
+  unsigned b0 = 0u, b1 = 0u, b2 = 0u, b3 = 0u;  // the last entries of the row (stored four at a time)
 
-  // FP32 screening.  Positions are rounded to FP32 relative to the origin
-  // org; every staged candidate (and particle of the group) lies within Mg
-  // of it (the group box's farthest corner plus the largest radius).  With
-  // u = 2^-24, the FP32 squared separation misses r^2 by at most
-  // 5u r^2 + 7u Mg r, i.e. near a radius R by a relative 5u + 7u Mg/R; the
-  // band eps(R) = 4e-6 (4 + Mg/R) is more than twice that, thresholds'
-  // rounding included, so a decision outside the band is the FP64 one.
-  float Mg = 0.0f;
+  // lanes that start a segment: a step along the order of more than two cells
+  // and two list radii (particles of one cell, or of cells next to each other
+  // on the curve, stay together)
+  unsigned long long heads;
   {
-    double m2 = 0.0;
+    const double4 pk = a.P4[act ? k : a.n - 1];
+    const double pk_x[3] = {pk.x, pk.y, pk.z};
+    bool jump = false;
+    const float rl = limf / (float)pk.w;
+    const float rp = __shfl_up(rl, 1);
+    for (int d = 0; d < NDIM; d++)
+      jump = jump || fabs(pk_x[d] - __shfl_up(pk_x[d], 1)) > 2.0 * fmax(g.w[d], (double)fmaxf(rl, rp));
+    heads = __ballot(jump && lane > 0) | 1ull;
+  }
+  unsigned long long todo = __ballot(act);
+  while (todo) {
+    // the next segment: from the first lane left to the next head
+    const int first = __builtin_ctzll(todo);
+    const unsigned long long later = first == 63 ? 0ull : heads & ~((2ull << first) - 1ull);
+    const unsigned long long seg = todo & (later ? (1ull << __builtin_ctzll(later)) - 1ull : ~0ull);
+    todo &= ~seg;
+    const bool in = (seg >> lane) & 1ull;
+    const double4 pk = a.P4[act ? k : a.n - 1];
+    const double pk_x[3] = {pk.x, pk.y, pk.z};
+    const float rl2 = (float)(lim2 / (pk.w * pk.w));
+    double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};
+    const float rw2 = wave_max_pos(in ? rl2 : 0.0f) * (1.0f + 1.0e-5f);
+    double org[3] = {0.0, 0.0, 0.0};
+    float half[3] = {0.0f, 0.0f, 0.0f};
+    int clo[3] = {0, 0, 0}, nc[3] = {1, 1, 1};
+    float diag2 = 0.0f;
     for (int d = 0; d < NDIM; d++) {
-      const double md = fmax(org[d] - gbox_lo[d], gbox_hi[d] - org[d]);
-      m2 += md * md;
+      lo[d] = wave_extreme<false>(in ? pk_x[d] : DBL_MAX);
+      hi[d] = wave_extreme<true>(in ? pk_x[d] : -DBL_MAX);
+      org[d] = wave_uniform(0.5 * (lo[d] + hi[d]));
+      half[d] = wave_uniform((float)(0.5 * (hi[d] - lo[d])) * (1.0f + 1.0e-6f));
+      diag2 += half[d] * half[d];
+      int c1, q;
+      cell_range(g, d, lo[d], rmax, clo[d], q);
+      cell_range(g, d, hi[d], rmax, q, c1);
+      nc[d] = max(c1 - clo[d] + 1, 0);
     }
-    Mg = (float)((sqrt(m2) + sqrt(rw2)) * (1.0 + 1.0e-6));
-  }
-  const double rl2 = act ? lim2 / hi21 : 0.0;  // squared list radius of this particle
-  const float eps_k = act ? 4.0e-6f * (4.0f + Mg / (float)sqrt(rl2)) : 0.0f;
-  const float rl2_out = (float)rl2 * (1.0f + eps_k), rl2_in = (float)rl2 * (1.0f - eps_k);
-  const float lim2_f = (float)lim2;
-  // lim2 * eps(R) for a candidate's radius R = sqrt(lim2) / w: band0 + band1 w
-  const float band0 = lim2_f * 1.6e-5f, band1 = lim2_f * 4.0e-6f * Mg / (float)sqrt(lim2);
-  // test the staged candidates [0, m) against this lane's particle (every
-  // lane of the wave takes part; an idle lane has no candidates)
-  auto test = [&](int m) {
-    unsigned long long mask = 0ull;
-    if (act) {
-#pragma unroll 1
-      for (int t0 = 0; t0 < m; t0 += 8) {
-        // 8 candidates with a constant bit each (entries past m are masked)
-        unsigned m8 = 0u;
+    diag2 = wave_uniform(diag2);
+    float rm2 = rw2;           // largest squared list radius met
+    int fill = 0, tested = 0;  // staged and tested candidates (wave-uniform)
+
+    // the particles' columns of the Gram product: of column block cb, lane l
+    // holds component l / 16 of particle 16 cb + l % 16, and the constants
+    // added to its products (an idle lane's particle is far from everything)
+    float bp[4];
+    nbl_f32x4 ck[4], cj[4];
+    {
+      float xr[3] = {0.0f, 0.0f, 0.0f}, p2 = 0.0f;
+      for (int d = 0; d < NDIM; d++) {
+        xr[d] = in ? (float)(pk_x[d] - org[d]) : 0.0f;
+        p2 += xr[d] * xr[d];
+      }
+      const float pg = in ? p2 - rl2 : 1.0e30f, px = in ? p2 : 1.0e30f;
+      const int q = lane >> 4;
 #pragma unroll
-        for (int u = 0; u < 8; u++) {
-          const float4 c = srel[t0 + u];
-          const float dx = xr0 - c.x, dy = xr1 - c.y, dz = xr2 - c.z;
-          const float r2f = dx * dx + dy * dy + dz * dz;
-          m8 |= r2f < rl2_out ? (1u << u) : 0u;
+      for (int cb = 0; cb < 4; cb++) {
+        const int src = 16 * cb + (lane & 15);
+        const float v0 = __shfl(xr[0], src), v1 = __shfl(xr[1], src), v2 = __shfl(xr[2], src);
+        const float vg = __shfl(pg, src), vx = __shfl(px, src);
+        bp[cb] = q == 0 ? v0 : q == 1 ? v1 : q == 2 ? v2 : 1.0f;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+          ck[cb][v] = vg;
+          cj[cb][v] = vx;
         }
-        mask |= (unsigned long long)m8 << t0;
       }
-      if (m < 64) mask &= (1ull << m) - 1ull;
     }
-    // an extra's slot is reserved when it is found and written when the next
-    // one is found (or after the loop), so the atomic's latency overlaps the
-    // tests in between
-    int pend_row = -1, pend_slot = 0;
-    unsigned pend_ent = 0u;
-    while (mask) {
-      const int t = __builtin_ctzll(mask);
-      mask &= mask - 1ull;
-      const unsigned e = se[t];
-      const float4 cr = srel[t];
-      const float dx = xr0 - cr.x, dy = xr1 - cr.y, dz = xr2 - cr.z;
-      const float r2f = dx * dx + dy * dy + dz * dz;
-      double rr = -1.0;
-      if (!(r2f < rl2_in)) {
-        const double4 c = sraw[t];
-        const double xr[3] = {c.x, c.y, c.z};
-        rr = image_r2<NDIM>(g, xi, xr, e & 63u);
-        if (!(rr * hi21 < lim2)) continue;
-      }
-      if (cnt < a.maxnb) L[cnt] = e;
-      else over = true;
-      cnt++;
-      const int kk = (int)(e >> 7);
-      if (kk != k) {
-        // q - lim2 against the band lim2 * eps(R_kk), R_kk = rlim / w_kk
-        const float dq = r2f * (cr.w * cr.w) - lim2_f;
-        const float band = band0 + band1 * cr.w;
-        int kin = dq < -band ? 1 : dq > band ? 0 : -1;
-        if (kin < 0) {
-          const double4 c = sraw[t];
-          if (rr < 0.0) {
-            const double xr[3] = {c.x, c.y, c.z};
-            rr = image_r2<NDIM>(g, xi, xr, e & 63u);
+    // test of the staged candidates [tested, tested + m), m <= 64
+    auto test = [&](int m) {
+      const int s0 = tested & 127;
+      const unsigned* ec = se + tested;
+      // row r of row block rb is candidate 16 (r / 4) + 4 rb + r % 4: the four
+      // values of a lane's quarter-wave q are then candidates 16 q + 4 rb ...
+      const float* const ak = sc[lane >> 4] + s0 + 16 * ((lane >> 2) & 3) + (lane & 3);
+      const float* const aj = sc[(lane >> 4) == 3 ? 4 : lane >> 4] + s0 + 16 * ((lane >> 2) & 3) + (lane & 3);
+      unsigned hg[4] = {0u, 0u, 0u, 0u}, hx[4] = {0u, 0u, 0u, 0u};
+      const float S = 2.0f * sqrtf(diag2) + sqrtf(rm2);
+      const float band = wave_uniform(2.0e-6f * S * S);
+      bool near = false;
+#pragma unroll
+      for (int rb = 3; rb >= 0; rb--) {
+        const float rk = ak[4 * rb], rj = aj[4 * rb];
+#pragma unroll
+        for (int cb = 0; cb < 4; cb += 2) {
+          const nbl_f32x4 d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(rk, bp[cb], ck[cb], 0, 0, 0);
+          const nbl_f32x4 d2 = __builtin_amdgcn_mfma_f32_16x16x4f32(rj, bp[cb], cj[cb], 0, 0, 0);
+          const nbl_f32x4 d3 = __builtin_amdgcn_mfma_f32_16x16x4f32(rk, bp[cb + 1], ck[cb + 1], 0, 0, 0);
+          const nbl_f32x4 d4 = __builtin_amdgcn_mfma_f32_16x16x4f32(rj, bp[cb + 1], cj[cb + 1], 0, 0, 0);
+          // from the last one down: candidate 16 q + b ends up in bit b
+#pragma unroll
+          for (int v = 3; v >= 0; v--) {
+            hg[cb] = __builtin_amdgcn_alignbit(hg[cb], __float_as_uint(d1[v]), 31);
+            hx[cb] = __builtin_amdgcn_alignbit(hx[cb], __float_as_uint(d2[v]), 31);
+            hg[cb + 1] = __builtin_amdgcn_alignbit(hg[cb + 1], __float_as_uint(d3[v]), 31);
+            hx[cb + 1] = __builtin_amdgcn_alignbit(hx[cb + 1], __float_as_uint(d4[v]), 31);
+            near |= fabsf(d1[v]) < band;
+            near |= fabsf(d2[v]) < band;
+            near |= fabsf(d3[v]) < band;
+            near |= fabsf(d4[v]) < band;
           }
-          kin = rr * (c.w * c.w) < lim2 ? 1 : 0;
-        }
-        if (!kin) {
-          if (pend_row >= 0 && pend_slot < a.maxnb)
-            a.nbl[(size_t)pend_row * a.maxnb + (a.maxnb - 1 - pend_slot)] = pend_ent;
-          pend_slot = atomicAdd(&a.nbx[kk], 1);
-          pend_row = kk;
-          pend_ent = ((unsigned)k << 7) | inverse_code(e & 63u);
+          // the products are used up here (left to itself the compiler keeps
+          // the values of all 32 tiles and spills)
+          unsigned nb = near;
+          asm volatile("" : "+v"(nb), "+v"(hg[cb]), "+v"(hx[cb]), "+v"(hg[cb + 1]), "+v"(hx[cb + 1]));
+          near = nb != 0u;
         }
       }
-    }
-    if (pend_row >= 0 && pend_slot < a.maxnb)
-      a.nbl[(size_t)pend_row * a.maxnb + (a.maxnb - 1 - pend_slot)] = pend_ent;
-  };
-
-  int ncl = 0;  // cells in the current batch (wave-uniform)
-  auto process_batch = [&]() {
-    __syncthreads();
-    for (int c = lane; c < ncl; c += 64) {
-      const int key = ckey[c];
-      const int b = key >= 0 ? a.cstart[key] : 0;
-      const int e = key >= 0 ? a.cstart[key + 1] : 0;
-      cbeg[c] = b;
-      cpre[c] = e - b;
-    }
-    __syncthreads();
-    int run = 0;
-    for (int c0 = 0; c0 < ncl; c0 += 64) {
-      const int v = c0 + lane < ncl ? cpre[c0 + lane] : 0;
-      int x = v;
-      for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (lane >= o) x += y;
+      // quarter-wave q holds candidates 16 q .. of every column block; the
+      // transpose hands quarter-wave cb the whole masks of its particles
+      unsigned mg[2], mx[2];
+      auto gather = [&](unsigned (&h)[4], unsigned (&o)[2]) {
+        const auto e = __builtin_amdgcn_permlane32_swap(h[0], h[2], false, false);
+        const auto f = __builtin_amdgcn_permlane32_swap(h[1], h[3], false, false);
+        const auto u = __builtin_amdgcn_permlane16_swap(e[0], f[0], false, false);
+        const auto v = __builtin_amdgcn_permlane16_swap(e[1], f[1], false, false);
+        o[0] = u[0] | (u[1] << 16);
+        o[1] = v[0] | (v[1] << 16);
+      };
+      gather(hg, mg);
+      gather(hx, mx);
+      if (m < 64) {
+        const unsigned long long valid = (1ull << m) - 1ull;
+        mg[0] &= (unsigned)valid;
+        mx[0] &= (unsigned)valid;
+        mg[1] &= (unsigned)(valid >> 32);
+        mx[1] &= (unsigned)(valid >> 32);
       }
-      if (c0 + lane < ncl) cpre[c0 + lane] = run + x - v;
-      run += __shfl(x, 63);
-    }
-    if (lane == 0) cpre[ncl] = run;
-    __syncthreads();
-    const int T = run;
-    // candidate q of the batch -> (raw record, list entry)
-    auto fetch = [&](int q, double4& pj, unsigned& ent) {
-      int lo = 0, hi = ncl - 1;
-      while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (cpre[mid] <= q) lo = mid;
-        else hi = mid - 1;
+      if (__ballot(near)) {
+        // (rare: the particle is read again rather than held in registers)
+        const double4 pi = a.P4[act ? k : a.n - 1];
+        const double xi[3] = {pi.x, pi.y, pi.z};
+        const double hi21 = pi.w * pi.w;
+        const float rl2 = (float)(lim2 / hi21);
+        float xr[3] = {0.0f, 0.0f, 0.0f};
+        for (int d = 0; d < NDIM; d++) xr[d] = (float)(xi[d] - org[d]);
+        for (int t = 0; t < m; t++) {
+          float r2 = 0.0f;
+          for (int d = 0; d < NDIM; d++) {
+            const float dx = xr[d] + 0.5f * sc[d][s0 + t];
+            r2 += dx * dx;
+          }
+          const float rj2 = sc[3][s0 + t] - sc[4][s0 + t];
+          if (!in || !(fminf(fabsf(r2 - rl2), fabsf(r2 - rj2)) < 2.0f * band)) continue;
+          const unsigned e = ec[t];
+          const double4 pj = a.P4[e >> 7];
+          const double xj[3] = {pj.x, pj.y, pj.z};
+          const double rr = image_r2<NDIM>(g, xi, xj, e & 63u);
+          const unsigned bit = 1u << (t & 31);
+          const bool ig = rr * hi21 < lim2, ix = rr * (pj.w * pj.w) < lim2;
+          if (t < 32) {
+            mg[0] = ig ? mg[0] | bit : mg[0] & ~bit;
+            mx[0] = ix ? mx[0] | bit : mx[0] & ~bit;
+          } else {
+            mg[1] = ig ? mg[1] | bit : mg[1] & ~bit;
+            mx[1] = ix ? mx[1] | bit : mx[1] & ~bit;
+          }
+        }
       }
-      const int kk = cbeg[lo] + (q - cpre[lo]);
-      ent = ((unsigned)kk << 7) | (unsigned)ccode[lo];
-      pj = a.P4[kk];
+#pragma unroll
+      for (int w = 0; w < 2; w++) {
+        smask[(tested >> 5) + w][lane] = mg[w];
+        // the extras go to the end of the row until the gather part is whole
+        unsigned x = mx[w] & ~mg[w];
+        while (x) {
+          const unsigned e = ec[32 * w + __builtin_ctz(x)];
+          x &= x - 1u;
+          if (nx < maxnb) L[maxnb - 1 - nx] = e;
+          nx++;
+        }
+      }
+      tested += m;
     };
-    double4 pj = make_double4(0.0, 0.0, 0.0, 0.0);
-    unsigned ent = 0u;
-    if (lane < T) fetch(lane, pj, ent);
-    for (int q0 = 0; q0 < T; q0 += 64) {
-      // keep the candidates inside the group's box widened by the largest
-      // radius, compacted in order behind the ones already staged
-      const int code = (int)(ent & 63u);
-      double xj[3] = {pj.x, pj.y, pj.z};
-      for (int d = 0; d < NDIM; d++) {
-        const int kd = (code >> (2 * d)) & 3;
-        if (kd) image_coord(g, d, kd, xj[d], 0.0, xj[d]);
-      }
-      bool keep = lane < T - q0;
-      double gd2 = 0.0;
-      for (int d = 0; d < NDIM; d++) {
-        const double e = fmax(fmax(gbox_lo[d] - xj[d], xj[d] - gbox_hi[d]), 0.0);
-        gd2 += e * e;
-      }
-      keep = keep && gd2 <= rw2;
-      const unsigned long long bal = __ballot(keep);
-      if (keep) {
-        const int pos = fill + __popcll(bal & ((1ull << lane) - 1ull));
-        sraw[pos] = pj;
-        srel[pos] = make_float4((float)(xj[0] - org[0]), NDIM >= 2 ? (float)(xj[1] - org[1]) : 0.f,
-                                NDIM >= 3 ? (float)(xj[2] - org[2]) : 0.f, (float)pj.w);
-        se[pos] = ent;
-      }
-      fill += __popcll(bal);
-      if (q0 + 64 + lane < T) fetch(q0 + 64 + lane, pj, ent);  // next 64, in flight during the test
-      if (fill >= 64) {
-        __syncthreads();
-        test(64);
-        __syncthreads();
-        if (lane < fill - 64) {
-          sraw[lane] = sraw[64 + lane];
-          srel[lane] = srel[64 + lane];
-          se[lane] = se[64 + lane];
+    // the gather part of the tested candidates into the rows
+    auto pop = [&]() {
+      __syncthreads();
+      const int nw = (tested + 31) >> 5;
+      int w = 0;
+      unsigned m = nw ? smask[0][lane] : 0u;
+      while (w < nw) {
+        if (m) {
+          const unsigned e = se[32 * w + __builtin_ctz(m)];
+          m &= m - 1u;
+          b0 = b1; b1 = b2; b2 = b3; b3 = e;
+          cnt++;
+          if (!(cnt & 3) && cnt <= maxnb) ((uint4*)L)[(cnt >> 2) - 1] = make_uint4(b0, b1, b2, b3);
         }
-        fill -= 64;
-        __syncthreads();
+        if (!m && ++w < nw) m = smask[w][lane];
       }
-    }
-    ncl = 0;
-  };
+      __syncthreads();
+    };
 
-  int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  for (int d = 1; d < NDIM; d++) {
-    int l = INT_MAX, h = INT_MIN;
-    if (act) cell_range(g, d, xi[d], rad, l, h);
-    lo[d] = wave_min_i(l);
-    hi[d] = wave_max_i(h);
-  }
-  for (int cz = lo[2]; cz <= hi[2]; cz++) {
-    int kz = 0, sz = 0;
-    double gz2 = 0.0;
-    if (NDIM >= 3) {
-      sz = cell_image(g, 2, cz, kz);
-      if (sz < 0) continue;
-      const double gz = cell_gap(g, 2, cz, xi[2]);
-      gz2 = gz * gz;
-    }
-    for (int cy = lo[1]; cy <= hi[1]; cy++) {
-      int ky = 0, sy = 0;
-      double r2 = rad2 - gz2;
-      if (NDIM >= 2) {
-        sy = cell_image(g, 1, cy, ky);
-        if (sy < 0) continue;
-        const double gy = cell_gap(g, 1, cy, xi[1]);
-        r2 -= gy * gy;
-      }
-      int lx = INT_MAX, hx = INT_MIN;
-      if (act && r2 >= 0.0) cell_range(g, 0, xi[0], NDIM >= 2 ? sqrt(r2) : rad, lx, hx);
-      lx = wave_min_i(lx);
-      hx = wave_max_i(hx);
-      // the row's key bits (y and z parts of cell_key)
-      const unsigned kyz = NDIM == 1 ? 0u : key_part(g, 1, sy) | (NDIM == 3 ? key_part(g, 2, sz) : 0u);
-      for (int cx0 = lx; cx0 <= hx; cx0 += 64) {
-        const int nadd = min(64, hx - cx0 + 1);
-        if (ncl + nadd > NBL_CELLS) process_batch();
-        if (lane < nadd) {
-          int kx = 0;
-          const int sx = cell_image(g, 0, cx0 + lane, kx);
-          ckey[ncl + lane] = sx >= 0 ? (int)(key_part(g, 0, sx) | kyz) : -1;
-          ccode[ncl + lane] = (int)list_code(kx, ky, kz);
+    // 64 cells a turn; a last turn without cells tests the candidates left over
+    const int ntot = nc[0] * nc[1] * nc[2];
+    bool more = true;
+    for (int c0 = 0; more; c0 += 64) {
+      more = c0 < ntot;
+      int cb = 0, cn = 0;
+      unsigned code = 0u;
+      float cr2 = 0.0f;
+      const int c = c0 + lane;
+      if (c < ntot) {
+        int cc[3] = {c, 0, 0}, kind[3] = {0, 0, 0}, src[3] = {0, 0, 0};
+        if (NDIM >= 2) {
+          cc[1] = c / nc[0];
+          cc[0] = c - cc[1] * nc[0];
         }
-        ncl += nadd;
+        if (NDIM >= 3) {
+          cc[2] = cc[1] / nc[1];
+          cc[1] = cc[1] - cc[2] * nc[1];
+        }
+        bool ok = true;
+        float d2 = 0.0f;
+        for (int d = 0; d < NDIM; d++) {
+          cc[d] += clo[d];
+          src[d] = cell_image(g, d, cc[d], kind[d]);
+          ok = ok && src[d] >= 0;
+          // distance of the cell (widened a little: a particle may be binned
+          // next door by rounding) from the box
+          const float mid = (float)(g.lo[d] + (cc[d] + 0.5) * g.w[d] - org[d]);
+          const float e = fmaxf(fabsf(mid) - half[d] - 0.50001f * (float)g.w[d], 0.0f);
+          d2 += e * e;
+        }
+        if (ok) {
+          unsigned key = key_part(g, 0, src[0]);
+          if (NDIM >= 2) key |= key_part(g, 1, src[1]);
+          if (NDIM >= 3) key |= key_part(g, 2, src[2]);
+          cb = a.cstart[key];
+          cn = a.cstart[key + 1] - cb;
+          const float cr = a.cellr[key];
+          cr2 = cr * cr * (1.0f + 1.0e-5f);
+          if (d2 * (1.0f - 1.0e-4f) > fmaxf(rw2, cr2)) cn = 0;
+          if (cn == 0) cr2 = 0.0f;
+          code = list_code(kind[0], kind[1], kind[2]);
+        }
+      }
+      int pre = wave_scan_add(cn);
+      const int T = __builtin_amdgcn_readlane(pre, 63);
+      pre -= cn;
+      rm2 = wave_uniform(fmaxf(rm2, wave_max_pos(cr2)));
+      for (int q0 = 0; q0 < T || !more; q0 += NBL_QUEUE) {
+        const int nq = min(NBL_QUEUE, T - q0);
+        __syncthreads();
+        {
+          const int qa = max(0, q0 - pre), qb = min(cn, q0 + nq - pre);
+          for (int q = qa; q < qb; q++) sq[pre - q0 + q] = ((unsigned)(cb + q) << 7) | code;
+        }
+        __syncthreads();
+        auto fetch = [&](int q, double4& pj, unsigned& e) {
+          e = sq[q];
+          pj = a.P4[e >> 7];
+        };
+        double4 pj = make_double4(0.0, 0.0, 0.0, 1.0);
+        unsigned ent = 0u;
+        if (lane < nq) fetch(lane, pj, ent);
+        for (int q = 0; q < nq || !more; q += 64) {
+          const double xj[3] = {pj.x, pj.y, pj.z};
+          float rel[3] = {0.0f, 0.0f, 0.0f}, d2 = 0.0f;
+          for (int d = 0; d < NDIM; d++) {
+            // kind 1: the image left of xmin; kind 2: right of xmax
+            const unsigned kd = (ent >> (2 * d)) & 3u;
+            const double Ld = g.xmax[d] - g.xmin[d];
+            rel[d] = (float)(xj[d] + (kd == 1u ? -Ld : kd == 2u ? Ld : 0.0) - org[d]);
+            const float e = fmaxf(fabsf(rel[d]) - half[d], 0.0f);
+            d2 += e * e;
+          }
+          const float rj = limf * __builtin_amdgcn_rcpf((float)pj.w);
+          const float rj2 = rj * rj;
+          const bool keep = lane < nq - q && d2 * (1.0f - 1.0e-4f) <= fmaxf(rw2, rj2);
+          const unsigned long long bal = __ballot(keep);
+          if (keep) {
+            const int pos = fill + __popcll(bal & ((1ull << lane) - 1ull));
+            float c2 = rel[0] * rel[0];
+            if (NDIM >= 2) c2 += rel[1] * rel[1];
+            if (NDIM >= 3) c2 += rel[2] * rel[2];
+            for (int d = 0; d < 3; d++) sc[d][pos & 127] = -2.0f * rel[d];
+            sc[3][pos & 127] = c2;
+            sc[4][pos & 127] = c2 - rj2;
+            se[pos] = ent;
+          }
+          fill += __popcll(bal);
+          if (q + 64 + lane < nq) fetch(q + 64 + lane, pj, ent);  // in flight during the test
+          const int m = min(fill - tested, 64);
+          if (m == 64 || (!more && m > 0)) {
+            __syncthreads();
+            test(m);
+            __syncthreads();
+          }
+          if (tested == NBL_CAP || !more) {
+            pop();
+            const unsigned t = se[NBL_CAP + lane];
+            __syncthreads();
+            se[lane] = t;
+            fill -= tested;
+            tested = 0;
+          }
+          if (!more) break;
+        }
+        if (!more) break;
       }
     }
   }
-  if (ncl) process_batch();
-  if (fill) {
-    __syncthreads();
-    test(fill);
+  if (!act) return;
+  // the row's open entries, then the extras behind them (the copy is ascending
+  // and its target never above its source)
+  const bool over = cnt + nx > maxnb;
+  if (!over) {
+    const int r = cnt & 3, m0 = cnt - r;
+    if (r == 1) L[m0] = b3;
+    if (r == 2) { L[m0] = b2; L[m0 + 1] = b3; }
+    if (r == 3) { L[m0] = b1; L[m0 + 1] = b2; L[m0 + 2] = b3; }
+    for (int m = 0; m < nx; m++) L[cnt + m] = L[maxnb - nx + m];
+  } else {
+    // the row did not hold the list: this particle scans cells
+    atomicAdd(&a.sc->list_overflow, 1);
   }
-  if (act) {
-    a.nbc[k] = over ? -1 : cnt;
-    a.hcap[k] = s1 / pk.w;
-  }
+  a.nbc[k] = over ? -1 : cnt;
+  a.nbx[k] = nx;
+  a.hcap[k] = s1 / a.P4[k].w;
 }
 template <int NDIM>
-// four waves per SIMD (a few registers spill; the LDS of a wave fits 4.5):
-// the builder waits on its candidate fetches, and 3 -> 4 waves took a
-// 128^3 build from 2.31 to 2.04 ms
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_nblist(KArgs a, Phys p,
                                                                                         const Grid* __restrict__ gp) {
   b_nblist<NDIM>(a, p, gp, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-// nx <= N entries E[0..nx) sorted ascending into D[0..nx) (D may overlap E:
-// every entry is read before any is written)
-template <int N>
-__device__ __forceinline__ void sort_extras(const unsigned* E, unsigned* D, int nx) {
-  unsigned v[N];
-#pragma unroll
-  for (int m = 0; m < N; m++) v[m] = m < nx ? E[m] : 0xffffffffu;
-  sort_regs<N>(v);
-#pragma unroll
-  for (int m = 0; m < N; m++)
-    if (m < nx) D[m] = v[m];
-}
-
-// extras (written from the end of the row) into [nbc, nbc + nbx) in
-// ascending entry order, so sums are deterministic; a row that did not hold
-// the gather list and the extras falls back to the cell scan
-__device__ __forceinline__ void b_nblist_sort(KArgs a, VL vl) {
-  const int k = vl.b * blockDim.x + threadIdx.x;
-  if (k >= a.n || !a.sc->list_on) return;
-  const int c0 = a.nbc[k], nx = a.nbx[k];
-  if (c0 < 0 || c0 + nx > a.maxnb) {
-    if (c0 >= 0) a.nbc[k] = -1;
-    atomicAdd(&a.sc->list_overflow, 1);
-    return;
-  }
-  // extras occupy E = L[maxnb-nx .. maxnb-1]; they end at L[c0 ..] ascending
-  unsigned* E = a.nbl + (size_t)k * a.maxnb + (a.maxnb - nx);
-  unsigned* D = a.nbl + (size_t)k * a.maxnb + c0;
-  if (nx <= 32) {
-    // up to 32 of them sorted in registers (a bitonic network of 8, 16 or
-    // 32, the smallest that holds every such row of the wave; every index a
-    // constant), then stored in place
-    const bool w16 = __ballot(nx > 16) != 0, w8 = __ballot(nx > 8) != 0;
-    if (w16) sort_extras<32>(E, D, nx);
-    else if (w8) sort_extras<16>(E, D, nx);
-    else sort_extras<8>(E, D, nx);
-    return;
-  }
-  // more: insertion sort in place, then move down (ascending copy,
-  // destination not above source)
-  for (int m = 1; m < nx; m++) {
-    const unsigned v = E[m];
-    int q = m - 1;
-    while (q >= 0 && E[q] > v) {
-      E[q + 1] = E[q];
-      q--;
-    }
-    E[q + 1] = v;
-  }
-  if (D != E)
-    for (int m = 0; m < nx; m++) D[m] = E[m];
-}
-__global__ __launch_bounds__(BS) void k_nblist_sort(KArgs a) {
-  b_nblist_sort(a, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // ===========================================================================
@@ -2871,11 +2967,9 @@ NDSP_MK(km_fill_cells) { NDSP_MEMBER b_fill_cells(M.a.cfill, M.gdev, vl); }
 NDSP_MK(km_cellid) { NDSP_MEMBER b_cellid(M.a, M.gdev, vl); }
 NDSP_MK(km_scan_local) { NDSP_MEMBER b_scan_local(M.a.cfill, M.a.cstart, M.bsum, M.gdev, vl); }
 NDSP_MK(km_scan_bsum) { NDSP_MEMBER b_scan_bsum(M.bsum, M.gdev, nullptr, vl); }
-NDSP_MK(km_scan_add) { NDSP_MEMBER b_scan_add(M.a.cstart, M.bsum, M.gdev, vl); }
+NDSP_MK(km_scan_add) { NDSP_MEMBER b_scan_add(M.a, M.bsum, M.gdev, vl); }
 NDSP_MK(km_scatter) { NDSP_MEMBER b_scatter(M.a, vl); }
 NDSP_MK(km_cellsort) { NDSP_MEMBER b_cellsort_wave(M.a, M.gdev, vl); }
-NDSP_MK(km_fill_nbx) { NDSP_MEMBER b_fill_i(M.a.nbx, M.a.n, 0, vl); }
-NDSP_MK(km_nblist_sort) { NDSP_MEMBER b_nblist_sort(M.a, vl); }
 NDSP_MK(km_init_density) { NDSP_MEMBER b_init_density_scalars(M.a.sc, M.bconstmax, M.a.n, vl); }
 NDSP_MK(km_pass_ctl) { NDSP_MEMBER b_pass_ctl(M.a.sc, M.a.n, M.reflect, M.p.maxits, vl); }
 NDSP_MK(km_hmax) { NDSP_MEMBER b_hmax(M.a, M.a.sc, vl); }
@@ -3164,10 +3258,13 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
   if (c->a.cstart) hipFree(c->a.cstart);
   if (c->a.cfill) hipFree(c->a.cfill);
   if (c->bsum) hipFree(c->bsum);
+  if (c->a.cellr) hipFree(c->a.cellr);
   c->a.cstart = c->a.cfill = c->bsum = nullptr;
+  c->a.cellr = nullptr;
   HIPCHK(hipMalloc(&c->a.cstart, sizeof(int) * cap));
   HIPCHK(hipMalloc(&c->a.cfill, sizeof(int) * cap));
   HIPCHK(hipMalloc(&c->bsum, sizeof(int) * (cap / (BS * 4) + 2)));
+  if (c->p.use_list) HIPCHK(hipMalloc(&c->a.cellr, sizeof(float) * cap));
   c->cap_bits = bits;
   invalidate_graphs(c);
   return 0;
@@ -3230,7 +3327,7 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
     hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(BS), 0, c->st, (const int*)a.cfill, a.cstart, c->bsum,
                        (const Grid*)c->gdev);
     hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(BS), 0, c->st, c->bsum, (const Grid*)c->gdev, (int*)nullptr);
-    hipLaunchKernelGGL(k_scan_add, dim3(cap_blocks), dim3(BS), 0, c->st, a.cstart, (const int*)c->bsum,
+    hipLaunchKernelGGL(k_scan_add, dim3(cap_blocks), dim3(BS), 0, c->st, a, (const int*)c->bsum,
                        (const Grid*)c->gdev);
     hipLaunchKernelGGL(k_fill_cells, dim3(std::min(cap_blocks, 4096u)), dim3(BS), 0, c->st, a.cfill,
                        (const Grid*)c->gdev);
@@ -3245,17 +3342,12 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
       hipLaunchKernelGGL(k_pack_density<float>, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
   }
   if (c->p.use_list) {
-    hipLaunchKernelGGL(k_fill_i, dim3(std::min(nblk(n), 4096u)), dim3(BS), 0, c->st, a.nbx, n, 0);
-    {
-      TScope t(c, "nblist");
-      dispatch_ndim(c->p.ndim, [&](auto nd) {
-        constexpr int ND = decltype(nd)::value;
-        hipLaunchKernelGGL((k_nblist<ND>), dim3(nblk(n, 64)), dim3(64), 0, c->st, a, c->p, (const Grid*)c->gdev);
-        return 0;
-      });
-    }
-    TScope t(c, "nblist_sort");
-    hipLaunchKernelGGL(k_nblist_sort, dim3(nblk(n)), dim3(BS), 0, c->st, a);
+    TScope t(c, "nblist");
+    dispatch_ndim(c->p.ndim, [&](auto nd) {
+      constexpr int ND = decltype(nd)::value;
+      hipLaunchKernelGGL((k_nblist<ND>), dim3(nblk(n, 64)), dim3(64), 0, c->st, a, c->p, (const Grid*)c->gdev);
+      return 0;
+    });
   }
   HIPCHK(hipGetLastError());
   c->grid_valid = true;
@@ -3675,7 +3767,7 @@ int ndsp_destroy(ndsp_ctx* c) {
   for (int fi = 0; fi < F_NFIELDS; fi++) if (a.f[fi]) hipFree(a.f[fi]);
   void* ptrs[] = {c->scratch_d, c->scratch_i, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
                   a.DR, a.FR, a.GF, a.sc, (void*)a.tabf, (void*)a.tabd,
-                  c->part, c->cons_out, a.cstart, a.cfill, c->bsum, c->list_a, c->list_b, a.nrflag, c->cmp_bsum,
+                  c->part, c->cons_out, a.cstart, a.cfill, a.cellr, c->bsum, c->list_a, c->list_b, a.nrflag, c->cmp_bsum,
                   a.nbl, a.nbc, a.nbx, a.hcap, a.red, c->gdev};
   for (void* q : ptrs) if (q) hipFree(q);
   if (c->graph_a) hipGraphExecDestroy(c->graph_a);
@@ -4187,13 +4279,11 @@ static int batch_part_a(ndsp_batch* b) {
     if (fp64) BLAUNCH(km_pack_density<double>, g, BGroup::S_256, BS);
     else BLAUNCH(km_pack_density<float>, g, BGroup::S_256, BS);
     if (g.lists) {
-      BLAUNCH(km_fill_nbx, g, BGroup::S_256, BS);
       dispatch_ndim(g.ndim, [&](auto nd) {
         constexpr int ND = decltype(nd)::value;
         BLAUNCH(km_nblist<ND>, g, BGroup::S_64, 64);
         return 0;
       });
-      BLAUNCH(km_nblist_sort, g, BGroup::S_256, BS);
     }
     BLAUNCH(km_init_density, g, BGroup::S_ONE, 64);
     const RedSpec spec = red_spec({RED_Q(RED_MAX, RED_F64, stressmax), RED_Q(RED_MAX, RED_F64, hmax_nr),

@@ -105,6 +105,7 @@ struct KArgs {
   int* cellid;        // per slot
   int* cstart;        // ncell + 1
   int* cfill;         // ncell
+  float* cellr;       // ncell: largest list radius of a cell's particles (null without lists)
   int* nrflag;        // unconverged after a pass, by sorted position (compacted in order; null: appended)
   int* sidx;          // sorted position -> slot
   // packed neighbour views in sorted order
@@ -127,7 +128,7 @@ struct KArgs {
   // nbl[k*maxnb + m] = (sorted index << 7) | image code (kinds kx + 5 ky + 25 kz)
   unsigned* nbl;
   int* nbc;           // gather-list length, -1 when the list overflowed
-  int* nbx;           // transposed extras after the gather list
+  int* nbx;           // extras after the gather list (members by j's list radius only)
   double* hcap;       // the list holds every neighbour while h <= hcap
   int maxnb;
   // per-block partials of the global reductions: quantity q of block b at
