@@ -804,7 +804,7 @@ __device__ __forceinline__ void for_each_candidate_rec(const KArgs& a, const Gri
 // [0, nbc) are the gather list G(k): every image of a particle j with
 // r_kj < radkern*h_k*(1+skin), in the candidate order of the cell scan; then
 // nbx extras: every image of j with r_kj < radkern*h_j*(1+skin) that is not in
-// G(k).  Together they hold every pair (and pair of periodic images) with
+// G(k), ascending.  Together they hold every pair (and pair of periodic images) with
 // r < radkern*max(h_k, h_j) while no h has grown past hcap = h*(1+skin).
 // Membership uses the separation fl(x_k - x_j) + s L per dimension, the shift
 // s = +1, -1 or 0 given by the image code, summed without contraction: it is
@@ -846,6 +846,19 @@ __device__ __forceinline__ double wave_uniform(double v) {
   const int lo = __builtin_amdgcn_readfirstlane((int)(unsigned)(b & 0xffffffffll));
   const int hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
   return __longlong_as_double(((long long)hi << 32) | (long long)(unsigned)lo);
+}
+
+// nx <= N entries E[0..nx) sorted ascending into D[0..nx) (D may overlap E:
+// every entry is read before any is written)
+template <int N>
+__device__ __forceinline__ void sort_extras(const unsigned* E, unsigned* D, int nx) {
+  unsigned v[N];
+#pragma unroll
+  for (int m = 0; m < N; m++) v[m] = m < nx ? E[m] : 0xffffffffu;
+  sort_regs<N>(v);
+#pragma unroll
+  for (int m = 0; m < N; m++)
+    if (m < nx) D[m] = v[m];
 }
 
 // Scans and folds over a wave with DPP moves (row shifts by 1, 2, 4 and 8, then
@@ -1268,15 +1281,37 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
     }
   }
   if (!act) return;
-  // the row's open entries, then the extras behind them (the copy is ascending
-  // and its target never above its source)
+  // the row's open entries, then the extras behind them in ascending order
   const bool over = cnt + nx > maxnb;
   if (!over) {
     const int r = cnt & 3, m0 = cnt - r;
     if (r == 1) L[m0] = b3;
     if (r == 2) { L[m0] = b2; L[m0 + 1] = b3; }
     if (r == 3) { L[m0] = b1; L[m0 + 1] = b2; L[m0 + 2] = b3; }
-    for (int m = 0; m < nx; m++) L[cnt + m] = L[maxnb - nx + m];
+    unsigned* const E = L + (maxnb - nx);
+    unsigned* const D = L + cnt;
+    if (nx <= 32) {
+      // sorted in registers (a bitonic network of 8, 16 or 32, the smallest
+      // that holds every such row of the wave), then stored in place
+      const bool w16 = __ballot(nx > 16) != 0, w8 = __ballot(nx > 8) != 0;
+      if (w16) sort_extras<32>(E, D, nx);
+      else if (w8) sort_extras<16>(E, D, nx);
+      else sort_extras<8>(E, D, nx);
+    } else {
+      // insertion sort in place, then down (ascending copy, the target never
+      // above the source)
+      for (int m = 1; m < nx; m++) {
+        const unsigned v = E[m];
+        int q = m - 1;
+        while (q >= 0 && E[q] > v) {
+          E[q + 1] = E[q];
+          q--;
+        }
+        E[q + 1] = v;
+      }
+      if (D != E)
+        for (int m = 0; m < nx; m++) D[m] = E[m];
+    }
   } else {
     // the row did not hold the list: this particle scans cells
     atomicAdd(&a.sc->list_overflow, 1);
