@@ -2879,6 +2879,61 @@ __global__ void k_copy_set(FieldSet<T> fs, const T* __restrict__ scratch, int n)
 }
 
 // ===========================================================================
+// host arrays in and out.  A caller's array holds w reals per particle in the
+// caller's order; the device holds one array per component in slot order.
+// The arrays cross the bus as they are, and these kernels take them apart or
+// put them together (128^3, ten components read back: 65 ms with the host
+// scattering every component through the particle ids, 15 ms here, the copy
+// into the caller's pageable memory).
+// ===========================================================================
+
+// in[i*w + d] -> component d of slot i (components past w are zero)
+__global__ void k_split3(const double* __restrict__ in, double* __restrict__ o0, double* __restrict__ o1,
+                         double* __restrict__ o2, int w, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const double* r = in + (size_t)i * w;
+  o0[i] = r[0];
+  o1[i] = w > 1 ? r[1] : 0.0;
+  o2[i] = w > 2 ? r[2] : 0.0;
+}
+// what an upload leaves besides the caller's arrays: slots in caller order,
+// no partners yet, Bfield and the dust fraction of the evolved state, every
+// derived field and rate zero
+__global__ void k_upload_rest(KArgs a, int set_itype) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  a.uid[i] = i;
+  a.slot_of[i] = i;
+  a.ireal[i] = -1;
+  if (set_itype) a.itype[i] = 0;
+  const double bx = a.f[F_BX][i], by = a.f[F_BY][i], bz = a.f[F_BZ][i], eps = a.f[F_EPS][i];
+#pragma unroll
+  for (int fi = F_RHO; fi < F_NFIELDS; fi++)
+    a.f[fi][i] = fi == F_BFX ? bx : fi == F_BFY ? by : fi == F_BFZ ? bz : fi == F_DUSTFRAC ? eps : 0.0;
+}
+// components f0.. of slot s -> out[uid[s]*w + d]
+struct CallerFields {
+  const double* f[3];
+  const int* i;  // an integer field instead, when not null
+  int slots;     // or the slots themselves
+};
+__global__ void k_to_caller(CallerFields c, const int* __restrict__ uid, double* __restrict__ out, int w, int n) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;
+  double* r = out + (size_t)uid[s] * w;
+  if (c.slots) {
+    r[0] = s;
+  } else if (c.i) {
+    r[0] = c.i[s];
+  } else {
+    r[0] = c.f[0][s];
+    if (w > 1) r[1] = c.f[1][s];
+    if (w > 2) r[2] = c.f[2][s];
+  }
+}
+
+// ===========================================================================
 // neighbour-set enumeration (test support)
 // ===========================================================================
 
@@ -3154,6 +3209,8 @@ struct ndsp_ctx {
   // (members of a batch, whose argument tables hold the field addresses,
   // copy back instead)
   double* falt[F_NPERSIST] = {};
+  char* fields = nullptr;      // the allocations behind a.f and falt (a reorder swaps their pointers)
+  char* fields_alt = nullptr;
   bool falt_failed = false;
   bool in_batch = false;
   bool alt_graph_valid = false;
@@ -3243,6 +3300,17 @@ static void timing_collect(ndsp_ctx* c) {
   }
   c->pending.clear();
   c->nev = 0;
+}
+
+// nf fields of n doubles in one allocation, each on a 256-byte boundary
+static size_t field_stride(size_t n) { return (sizeof(double) * n + 255) / 256 * 256; }
+static bool alloc_fields(char** slab, double** f, int nf, size_t n) {
+  if (hipMalloc((void**)slab, field_stride(n) * nf) != hipSuccess) {
+    *slab = nullptr;
+    return false;
+  }
+  for (int k = 0; k < nf; k++) f[k] = (double*)(*slab + field_stride(n) * k);
+  return true;
 }
 
 static inline unsigned nblk(long long n, int bs = BS) { return (unsigned)((n + bs - 1) / bs); }
@@ -3536,15 +3604,8 @@ static int reorder(ndsp_ctx* c) {
   const int n = c->n;
   TScope t(c, "reorder");
   if (!c->in_batch && !c->falt_failed && !c->falt[0]) {
-    bool ok = true;
-    for (int fi = 0; fi < F_NPERSIST && ok; fi++) ok = hipMalloc(&c->falt[fi], sizeof(double) * n) == hipSuccess;
-    if (!ok) {
+    if (!alloc_fields(&c->fields_alt, c->falt, F_NPERSIST, n)) {
       (void)hipGetLastError();
-      for (int fi = 0; fi < F_NPERSIST; fi++)
-        if (c->falt[fi]) {
-          (void)hipFree(c->falt[fi]);
-          c->falt[fi] = nullptr;
-        }
       c->falt_failed = true;
     }
   }
@@ -3720,10 +3781,8 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   KArgs& a = c->a;
   memset(&a, 0, sizeof(a));
   const size_t n = (size_t)npart;
-  for (int fi = 0; fi < F_NFIELDS; fi++) {
-    if (hipMalloc(&a.f[fi], sizeof(double) * n) != hipSuccess) return cleanup_fail(set_err(NDSP_ERR_ALLOC, "hipMalloc fields"));
-    hipMemset(a.f[fi], 0, sizeof(double) * n);
-  }
+  if (!alloc_fields(&c->fields, a.f, F_NFIELDS, n)) return cleanup_fail(set_err(NDSP_ERR_ALLOC, "hipMalloc fields"));
+  hipMemset(c->fields, 0, field_stride(n) * F_NFIELDS);
   bool ok = true;
   ok &= hipMalloc(&c->scratch_d, sizeof(double) * n * REORDER_W) == hipSuccess;
   ok &= hipMalloc(&c->scratch_i, sizeof(int) * n) == hipSuccess;
@@ -3799,8 +3858,7 @@ int ndsp_destroy(ndsp_ctx* c) {
   if (!c) return 0;
   if (c->st) hipStreamSynchronize(c->st);
   KArgs& a = c->a;
-  for (int fi = 0; fi < F_NFIELDS; fi++) if (a.f[fi]) hipFree(a.f[fi]);
-  void* ptrs[] = {c->scratch_d, c->scratch_i, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
+  void* ptrs[] = {c->fields, c->fields_alt, c->scratch_d, c->scratch_i, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
                   a.DR, a.FR, a.GF, a.sc, (void*)a.tabf, (void*)a.tabd,
                   c->part, c->cons_out, a.cstart, a.cfill, a.cellr, c->bsum, c->list_a, c->list_b, a.nrflag, c->cmp_bsum,
                   a.nbl, a.nbc, a.nbx, a.hcap, a.red, c->gdev};
@@ -3809,7 +3867,6 @@ int ndsp_destroy(ndsp_ctx* c) {
   if (c->graph_b) hipGraphExecDestroy(c->graph_b);
   if (c->alt_graph_a) hipGraphExecDestroy(c->alt_graph_a);
   if (c->alt_graph_b) hipGraphExecDestroy(c->alt_graph_b);
-  for (int fi = 0; fi < F_NPERSIST; fi++) if (c->falt[fi]) hipFree(c->falt[fi]);
   if (c->mlp_alloced) mlp_free(c->mlp);
   for (auto e : c->ev0) hipEventDestroy(e);
   for (auto e : c->ev1) hipEventDestroy(e);
@@ -3823,56 +3880,45 @@ int ndsp_upload(ndsp_ctx* c, const double* x, const double* vel, const double* p
                 const double* dustevol, const int32_t* itype) {
   if (!c || !x || !vel || !pmass || !hh || !en || !alpha || !psi) return set_err(NDSP_ERR_BAD_ARG, "upload: null array");
   const int n = c->n, nd = c->p.ndim;
-  std::vector<double> buf(n);
-  auto put = [&](int fi) { return hipMemcpyAsync(c->a.f[fi], buf.data(), sizeof(double) * n, hipMemcpyHostToDevice, c->st); };
+  int nfixed = 0;
   for (int i = 0; i < n; i++) {
     if (itype && itype[i] != 0 && itype[i] != 1)
       return set_err(NDSP_ERR_BAD_OPTION, "only gas (itype 0) and fixed boundary (itype 1) particles are supported");
     if (itype && itype[i] == 1 && !c->p.fixed_on)
       return set_err(NDSP_ERR_BAD_OPTION, "fixed particles (itype 1) need a wall of fixed particles (ibound 1)");
     if (!(hh[i] > 0.0)) return set_err(NDSP_ERR_H_NONPOSITIVE, "upload: h <= 0");
+    nfixed += itype && itype[i] == 1;
   }
-  for (int d = 0; d < 3; d++) {
-    for (int i = 0; i < n; i++) buf[i] = d < nd ? x[(size_t)i * nd + d] : 0.0;
-    HIPCHK(put(F_X + d));
-    HIPCHK(hipStreamSynchronize(c->st));
-  }
-  const int vf[3] = {F_VX, F_VY, F_VZ}, bf[3] = {F_BX, F_BY, F_BZ}, af[3] = {F_A0, F_A1, F_A2};
-  for (int d = 0; d < 3; d++) {
-    for (int i = 0; i < n; i++) buf[i] = vel[(size_t)i * 3 + d];
-    HIPCHK(put(vf[d])); HIPCHK(hipStreamSynchronize(c->st));
-    for (int i = 0; i < n; i++) buf[i] = (c->p.imhd && Bevol) ? Bevol[(size_t)i * 3 + d] : 0.0;
-    HIPCHK(put(bf[d])); HIPCHK(hipStreamSynchronize(c->st));
-    for (int i = 0; i < n; i++) buf[i] = alpha[(size_t)i * 3 + d];
-    HIPCHK(put(af[d])); HIPCHK(hipStreamSynchronize(c->st));
-  }
-  const double* one[4] = {pmass, hh, en, psi};
-  const int onef[4] = {F_M, F_H, F_EN, F_PSI};
+  // vectors through the scratch (its two halves in turn: the copies and the
+  // kernels that read them are ordered on the stream), scalars in place
+  double** f = c->a.f;
+  const size_t row = sizeof(double) * (size_t)n;
+  const struct { const double* src; int f0, w; } vec[4] = {
+      {x, F_X, nd}, {vel, F_VX, 3}, {c->p.imhd ? Bevol : nullptr, F_BX, 3}, {alpha, F_A0, 3}};
   for (int q = 0; q < 4; q++) {
-    for (int i = 0; i < n; i++) buf[i] = one[q][i];
-    HIPCHK(put(onef[q])); HIPCHK(hipStreamSynchronize(c->st));
+    const int f0 = vec[q].f0;
+    if (!vec[q].src) {
+      for (int d = 0; d < 3; d++)
+        hipLaunchKernelGGL(k_fill_d, dim3(std::min(nblk(n), 4096u)), dim3(BS), 0, c->st, f[f0 + d], n, 0.0);
+      continue;
+    }
+    double* half = c->scratch_d + (size_t)(q & 1) * (REORDER_W / 2) * n;
+    HIPCHK(hipMemcpyAsync(half, vec[q].src, row * vec[q].w, hipMemcpyHostToDevice, c->st));
+    hipLaunchKernelGGL(k_split3, dim3(nblk(n)), dim3(BS), 0, c->st, (const double*)half, f[f0], f[f0 + 1], f[f0 + 2],
+                       vec[q].w, n);
   }
-  for (int i = 0; i < n; i++) buf[i] = (c->p.idust && dustevol) ? dustevol[i] : 0.0;
-  HIPCHK(put(F_EPS)); HIPCHK(hipStreamSynchronize(c->st));
-  // dustfrac starts equal to the evolved dust fraction
-  HIPCHK(hipMemcpy(c->a.f[F_DUSTFRAC], c->a.f[F_EPS], sizeof(double) * n, hipMemcpyDeviceToDevice));
-  std::vector<int> ids(n);
-  for (int i = 0; i < n; i++) ids[i] = i;
-  HIPCHK(hipMemcpy(c->a.uid, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->a.slot_of, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  for (int i = 0; i < n; i++) ids[i] = itype ? itype[i] : 0;
-  HIPCHK(hipMemcpy(c->a.itype, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  for (int i = 0; i < n; i++) ids[i] = -1;
-  HIPCHK(hipMemcpy(c->a.ireal, ids.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-  c->nfixed = 0;
-  for (int i = 0; i < n; i++) c->nfixed += itype && itype[i] == 1;
-  c->ireal_set = c->nfixed == 0;
-  // derived fields and rates start at zero
-  for (int fi = F_RHO; fi < F_NFIELDS; fi++)
-    if (fi != F_DUSTFRAC) HIPCHK(hipMemsetAsync(c->a.f[fi], 0, sizeof(double) * n, c->st));
+  const struct { const double* src; int f0; } one[5] = {
+      {pmass, F_M}, {hh, F_H}, {en, F_EN}, {psi, F_PSI}, {c->p.idust ? dustevol : nullptr, F_EPS}};
+  for (const auto& o : one) {
+    if (o.src) HIPCHK(hipMemcpyAsync(f[o.f0], o.src, row, hipMemcpyHostToDevice, c->st));
+    else hipLaunchKernelGGL(k_fill_d, dim3(std::min(nblk(n), 4096u)), dim3(BS), 0, c->st, f[o.f0], n, 0.0);
+  }
+  if (itype) HIPCHK(hipMemcpyAsync(c->a.itype, itype, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, c->st));
+  hipLaunchKernelGGL(k_upload_rest, dim3(nblk(n)), dim3(BS), 0, c->st, c->a, itype ? 0 : 1);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->st));
-  for (int d = 0; d < 3; d++)
-    HIPCHK(hipMemcpy(c->a.f[F_BFX + d], c->a.f[F_BX + d], sizeof(double) * n, hipMemcpyDeviceToDevice));
+  c->nfixed = nfixed;
+  c->ireal_set = nfixed == 0;
   c->grid_valid = false;
   c->have_rates = false;
   c->nsteps = 0;
@@ -3893,30 +3939,13 @@ static const struct { const char* name; int f0; int w; } kFieldMap[] = {
 int ndsp_download(ndsp_ctx* c, const char* name, double* out, int32_t* width) {
   if (!c || !name || !out) return set_err(NDSP_ERR_BAD_ARG, "download: null argument");
   const int n = c->n;
-  std::vector<int> uid(n);
-  HIPCHK(hipStreamSynchronize(c->st));
-  HIPCHK(hipMemcpy(uid.data(), c->a.uid, sizeof(int) * n, hipMemcpyDeviceToHost));
-  std::vector<double> buf(n);
-  if (!strcmp(name, "x")) {
-    const int nd = c->p.ndim;
-    for (int d = 0; d < nd; d++) {
-      HIPCHK(hipMemcpy(buf.data(), c->a.f[F_X + d], sizeof(double) * n, hipMemcpyDeviceToHost));
-      for (int s = 0; s < n; s++) out[(size_t)uid[s] * nd + d] = buf[s];
-    }
-    if (width) *width = nd;
-    return 0;
-  }
-  if (!strcmp(name, "slot")) {
-    // where each particle sits in device memory (the cell order of the last reorder)
-    for (int s = 0; s < n; s++) out[uid[s]] = s;
-    if (width) *width = 1;
-    return 0;
-  }
   if (!strcmp(name, "nblist_len")) {
     // entries of each particle's neighbour list at the last binning
     // (gather list + extras); -1 where it scans cells instead (an overflow,
     // or lists off)
-    std::vector<int> nbc(n, -1), nbx(n, 0), sidx(n);
+    HIPCHK(hipStreamSynchronize(c->st));
+    std::vector<int> uid(n), nbc(n, -1), nbx(n, 0), sidx(n);
+    HIPCHK(hipMemcpy(uid.data(), c->a.uid, sizeof(int) * n, hipMemcpyDeviceToHost));
     if (c->p.use_list) {
       HIPCHK(hipMemcpy(nbc.data(), c->a.nbc, sizeof(int) * n, hipMemcpyDeviceToHost));
       HIPCHK(hipMemcpy(nbx.data(), c->a.nbx, sizeof(int) * n, hipMemcpyDeviceToHost));
@@ -3927,21 +3956,32 @@ int ndsp_download(ndsp_ctx* c, const char* name, double* out, int32_t* width) {
     if (width) *width = 1;
     return 0;
   }
-  if (!strcmp(name, "numneigh") || !strcmp(name, "nits")) {
-    std::vector<int> ib(n);
-    HIPCHK(hipMemcpy(ib.data(), !strcmp(name, "nits") ? c->a.nits : c->a.numneigh, sizeof(int) * n,
-                     hipMemcpyDeviceToHost));
-    for (int s = 0; s < n; s++) out[uid[s]] = ib[s];
-    if (width) *width = 1;
-    return 0;
-  }
-  for (const auto& e : kFieldMap) {
-    if (strcmp(name, e.name)) continue;
-    for (int q = 0; q < e.w; q++) {
-      HIPCHK(hipMemcpy(buf.data(), c->a.f[e.f0 + q], sizeof(double) * n, hipMemcpyDeviceToHost));
-      for (int s = 0; s < n; s++) out[(size_t)uid[s] * e.w + q] = buf[s];
+  CallerFields cf{};
+  int w = 0;
+  if (!strcmp(name, "x")) {
+    w = c->p.ndim;
+    for (int d = 0; d < w; d++) cf.f[d] = c->a.f[F_X + d];
+  } else if (!strcmp(name, "slot")) {
+    // where each particle sits in device memory (the cell order of the last reorder)
+    w = 1;
+    cf.slots = 1;
+  } else if (!strcmp(name, "numneigh") || !strcmp(name, "nits")) {
+    w = 1;
+    cf.i = !strcmp(name, "nits") ? c->a.nits : c->a.numneigh;
+  } else {
+    for (const auto& e : kFieldMap) {
+      if (strcmp(name, e.name)) continue;
+      w = e.w;
+      for (int d = 0; d < w; d++) cf.f[d] = c->a.f[e.f0 + d];
+      break;
     }
-    if (width) *width = e.w;
+  }
+  if (w) {
+    hipLaunchKernelGGL(k_to_caller, dim3(nblk(n)), dim3(BS), 0, c->st, cf, (const int*)c->a.uid, c->scratch_d, w, n);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(out, c->scratch_d, sizeof(double) * (size_t)n * w, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    if (width) *width = w;
     return 0;
   }
   return set_err(NDSP_ERR_BAD_ARG, std::string("download: unknown field ") + name);
