@@ -2,22 +2,25 @@
 // include/ndsp.h.  One context holds one simulation resident in HBM.
 //
 // Pipeline of one derivative evaluation (src/derivs.f90:27):
-//   k_boundary      periodic wrap / wall reflection (src/boundaryND.f90:66-160)
-//   k_binstats      max h and bounding box (src/ghostND_mhd.f90:77, linkND.f90:78-90)
-//   k_cellid, scan, k_scatter, k_cellsort_wave
+//   k_binstats      periodic wrap / wall reflection (src/boundaryND.f90:66-160),
+//                   max h and bounding box (src/ghostND_mhd.f90:77,
+//                   linkND.f90:78-90), the cell grid
+//   k_cellid, k_scan_local, k_scatter, k_cellsort_wave
 //                   counting sort of particles by Morton cell key, stable
 //                   by slot: replaces the head/next link lists of
 //                   set_linklist (src/linkND.f90:45-161)
 //   k_pack_density  sorted neighbour view: FP64 (x,y,z,1/h) + payload
+//   k_nblist        per-particle neighbour lists
 //   k_nr_pass       h-rho Newton-Raphson passes, persistent once a pass is partial
 //                   (src/iterate_density.f90:43-360 with density_sums.f90),
 //                   fused conservative->primitive + EOS
-//                   (src/conservative2primitive.f90:42-470, src/eos.f90:40-106)
+//                   (src/conservative2primitive.f90:42-470, src/eos.f90:40-106);
+//                   k_pass_fold and k_pass_next between them
 //   k_pack_force    sorted neighbour view for the force pass
 //   k_force         fused pair sums of get_rates (src/ratesND_mhd.f90:304-467,
 //                   1175-1690, 1700-1894, 2154-2206, 2377-2720, 2813-2878)
 //   k_finalize      per-particle finalisation (src/ratesND_mhd.f90:482-943)
-//   k_dt            timestep (src/stepND_leapfrog_mhd.f90:252)
+//   k_dt_fold       timestep (src/stepND_leapfrog_mhd.f90:252)
 // and of one step: k_predict, derivs with the corrector in the finalize launch
 // (k_finalize_correct) (stepND_leapfrog_mhd.f90:31-275).
 //
@@ -62,15 +65,19 @@ static int set_err(int code, const std::string& m) {
 
 static const int BS = 256;
 
+// A recorded step's second half is launched right behind the first, before the
+// host knows whether the recorded passes finished the h-rho iteration; its
+// kernels do nothing until they have (and nothing again once the step is done,
+// when the half is launched a second time for a batch's late members).
+__device__ __forceinline__ bool held_back(const DScal* sc, int guard) { return guard && sc->phase != 1; }
+
 // ===========================================================================
 // small kernels: boundary, statistics, binning, scan
 // ===========================================================================
 
 // boundary, src/boundaryND.f90:66-160
-__device__ __forceinline__ void b_boundary(KArgs a, Phys p, Grid g, int in_step, VL vl) {
+__device__ __forceinline__ void boundary_one(const KArgs& a, const Phys& p, const Grid& g, int in_step, int i) {
 #pragma clang fp contract(off)
-  int i = vl.b * blockDim.x + threadIdx.x;
-  if (i >= a.n) return;
   double* xs[3] = {a.f[F_X], a.f[F_Y], a.f[F_Z]};
   double* vs[3] = {a.f[F_VX], a.f[F_VY], a.f[F_VZ]};
   double* xins[3] = {a.f[F_XIN], a.f[F_YIN], a.f[F_ZIN]};
@@ -78,10 +85,10 @@ __device__ __forceinline__ void b_boundary(KArgs a, Phys p, Grid g, int in_step,
   double* fs[3] = {a.f[F_FX], a.f[F_FY], a.f[F_FZ]};
   for (int d = 0; d < 3; d++) if (d < p.ndim) {
     if (g.bound[d] != 3) continue;
-    double x = xs[d][i];
-    if (x > g.xmax[d]) x = g.xmin[d] + x - g.xmax[d];
-    else if (x < g.xmin[d]) x = g.xmax[d] - (g.xmin[d] - x);
-    xs[d][i] = x;
+    // (stored only where it moves: few particles do)
+    const double x = xs[d][i];
+    if (x > g.xmax[d]) xs[d][i] = g.xmin[d] + x - g.xmax[d];
+    else if (x < g.xmin[d]) xs[d][i] = g.xmax[d] - (g.xmin[d] - x);
   }
   for (int d = 0; d < 3; d++) if (d < p.ndim) {
     if (g.bound[d] <= 1) continue;
@@ -97,45 +104,38 @@ __device__ __forceinline__ void b_boundary(KArgs a, Phys p, Grid g, int in_step,
     }
   }
 }
-__global__ void k_boundary(KArgs a, Phys p, Grid g, int in_step) {
-  b_boundary(a, p, g, in_step, VL{(int)blockIdx.x, (int)gridDim.x});
+// Whether the calling block is the last of nb to get here.  One thread calls
+// it, after that thread's own stores, which are then visible to the device; a
+// block that is the last makes an agent-scope acquire before it reads the
+// others' (every thread: the launch's stores lie in eight L2 caches).
+__device__ __forceinline__ bool last_block(int* done, int nb) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+  return atomicAdd(done, 1) == nb - 1;
 }
 
-// per-block max h and bounding box -> part[blk*8 + 0..6]
-__device__ __forceinline__ void b_binstats(KArgs a, int ndim, double* part, VL vl) {
-  __shared__ double sm[7][BS];
-  int t = threadIdx.x;
-  double hm = 0.0, lo[3] = {DBL_MAX, DBL_MAX, DBL_MAX}, hi[3] = {-DBL_MAX, -DBL_MAX, -DBL_MAX};
-  const double* xs[3] = {a.f[F_X], a.f[F_Y], a.f[F_Z]};
-  for (int i = vl.b * blockDim.x + t; i < a.n; i += vl.nb * blockDim.x) {
-    hm = fmax(hm, a.f[F_H][i]);
-    for (int d = 0; d < ndim; d++) {
-      lo[d] = fmin(lo[d], xs[d][i]);
-      hi[d] = fmax(hi[d], xs[d][i]);
+// max h and bounding box (v[0]; minima v[1..3]; maxima v[4..6]) of the block's
+// threads, in thread 0
+__device__ __forceinline__ void block_box(double (&v)[7], double (&sm)[7][BS / 64]) {
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  for (int q = 0; q < 7; q++) {
+    const bool mn = q >= 1 && q <= 3;
+    for (int o = 32; o > 0; o >>= 1) {
+      const double y = __shfl_xor(v[q], o);
+      v[q] = mn ? fmin(v[q], y) : fmax(v[q], y);
     }
+    if (lane == 0) sm[q][w] = v[q];
   }
-  sm[0][t] = hm;
-  for (int d = 0; d < 3; d++) { sm[1 + d][t] = lo[d]; sm[4 + d][t] = hi[d]; }
   __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if (t < s) {
-      sm[0][t] = fmax(sm[0][t], sm[0][t + s]);
-      for (int d = 0; d < 3; d++) {
-        sm[1 + d][t] = fmin(sm[1 + d][t], sm[1 + d][t + s]);
-        sm[4 + d][t] = fmax(sm[4 + d][t], sm[4 + d][t + s]);
-      }
+  if (threadIdx.x == 0)
+    for (int q = 0; q < 7; q++) {
+      const bool mn = q >= 1 && q <= 3;
+      for (int u = 1; u < BS / 64; u++) v[q] = mn ? fmin(v[q], sm[q][u]) : fmax(v[q], sm[q][u]);
     }
-    __syncthreads();
-  }
-  if (t < 7) part[vl.b * 8 + t] = sm[t][0];
-}
-__global__ void k_binstats(KArgs a, int ndim, double* part) {
-  b_binstats(a, ndim, part, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-// one block of BS threads folds the per-block partials of k_binstats
-__device__ __forceinline__ void b_binstats_final(DScal* sc, const double* part, int nb, VL vl) {
-  __shared__ double sm[7][BS];
+// the fold of k_binstats' per-block partials, by one block of BS threads
+__device__ __forceinline__ void fold_binstats(DScal* sc, const double* part, int nb) {
+  __shared__ double sm[7][BS / 64];
   double v[7] = {0.0, DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX};
   for (int b = threadIdx.x; b < nb; b += blockDim.x) {
     v[0] = fmax(v[0], part[b * 8]);
@@ -144,26 +144,11 @@ __device__ __forceinline__ void b_binstats_final(DScal* sc, const double* part, 
       v[4 + d] = fmax(v[4 + d], part[b * 8 + 4 + d]);
     }
   }
-  for (int q = 0; q < 7; q++) sm[q][threadIdx.x] = v[q];
-  __syncthreads();
-  for (int st = BS / 2; st > 0; st >>= 1) {
-    if ((int)threadIdx.x < st) {
-      const int t = threadIdx.x;
-      sm[0][t] = fmax(sm[0][t], sm[0][t + st]);
-      for (int d = 0; d < 3; d++) {
-        sm[1 + d][t] = fmin(sm[1 + d][t], sm[1 + d][t + st]);
-        sm[4 + d][t] = fmax(sm[4 + d][t], sm[4 + d][t + st]);
-      }
-    }
-    __syncthreads();
-  }
+  block_box(v, sm);
   if (threadIdx.x == 0) {
-    sc->hmax_bin = sm[0][0];
-    for (int d = 0; d < 3; d++) { sc->bbox_lo[d] = sm[1 + d][0]; sc->bbox_hi[d] = sm[4 + d][0]; }
+    sc->hmax_bin = v[0];
+    for (int d = 0; d < 3; d++) { sc->bbox_lo[d] = v[1 + d]; sc->bbox_hi[d] = v[4 + d]; }
   }
-}
-__global__ __launch_bounds__(BS) void k_binstats_final(DScal* sc, const double* part, int nb) {
-  b_binstats_final(sc, part, nb, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // Cell grid of this binning, on the device (no host round trip): cells of
@@ -173,8 +158,8 @@ __global__ __launch_bounds__(BS) void k_binstats_final(DScal* sc, const double* 
 // 2^cap_bits.  Also decides whether neighbour lists can be used
 // (radkern*hmax*(1+skin) below every periodic length, so every image within
 // a list radius lies in the image cells one period away).
-__device__ __forceinline__ void b_grid_setup(DScal* sc, Grid* gd, Grid box, Phys p, int cap_bits, VL vl) {
-  if (threadIdx.x | vl.b) return;
+__device__ __forceinline__ void grid_setup(DScal* sc, Grid* gd, const Grid& box, const Phys& p, int cap_bits, int n) {
+  sc->err = 0;
   Grid g = box;
   const double hmax = sc->hmax_bin;
   const double rmax = p.radkern * hmax;
@@ -255,24 +240,56 @@ __device__ __forceinline__ void b_grid_setup(DScal* sc, Grid* gd, Grid box, Phys
   sc->list_overflow = 0;
   *gd = g;
 }
-__global__ void k_grid_setup(DScal* sc, Grid* gd, Grid box, Phys p, int cap_bits) {
-  b_grid_setup(sc, gd, box, p, cap_bits, VL{(int)blockIdx.x, (int)gridDim.x});
-}
+__device__ __forceinline__ void init_density_scalars(DScal* sc, const Phys& p, int n);
 
-__device__ __forceinline__ void b_fill_cells(int* __restrict__ a, const Grid* __restrict__ gd, VL vl) {
-  const long long m = gd->ncell + 1;
-  for (long long i = (long long)vl.b * blockDim.x + threadIdx.x; i < m; i += (long long)vl.nb * blockDim.x)
-    a[i] = 0;
+// The first launch of a binning: the boundary of every particle (wrap >= 0, its
+// in_step), max h and the bounding box, and in the last block to finish the
+// fold over the blocks, the cell grid (gd not null) and the scalars of the
+// h-rho iteration that follows.  One launch for six (wrap, statistics, their
+// fold, grid, error reset, scalar set-up: each 2-5 us and a gap of its own on
+// a small simulation).
+__device__ __forceinline__ void b_binstats(KArgs a, const Phys& p, const Grid& box, Grid* gd, int wrap, int cap_bits,
+                                           double* part, VL vl) {
+  __shared__ double sm[7][BS / 64];
+  __shared__ int last;
+  const int t = threadIdx.x;
+  double v[7] = {0.0, DBL_MAX, DBL_MAX, DBL_MAX, -DBL_MAX, -DBL_MAX, -DBL_MAX};
+  const double* xs[3] = {a.f[F_X], a.f[F_Y], a.f[F_Z]};
+  for (int i = vl.b * blockDim.x + t; i < a.n; i += vl.nb * blockDim.x) {
+    if (wrap >= 0) boundary_one(a, p, box, wrap, i);
+    v[0] = fmax(v[0], a.f[F_H][i]);
+    for (int d = 0; d < 3; d++)
+      if (d < p.ndim) {
+        const double x = xs[d][i];
+        v[1 + d] = fmin(v[1 + d], x);
+        v[4 + d] = fmax(v[4 + d], x);
+      }
+  }
+  block_box(v, sm);
+  if (t == 0) {
+    for (int q = 0; q < 7; q++) part[vl.b * 8 + q] = v[q];
+    last = last_block(&a.sc->bin_done, vl.nb);
+  }
+  __syncthreads();
+  if (!last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  fold_binstats(a.sc, part, vl.nb);
+  if (t) return;
+  a.sc->bin_done = 0;
+  if (!gd) return;
+  grid_setup(a.sc, gd, box, p, cap_bits, a.n);
+  init_density_scalars(a.sc, p, a.n);
 }
-__global__ void k_fill_cells(int* __restrict__ a, const Grid* __restrict__ gd) {
-  b_fill_cells(a, gd, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ __launch_bounds__(BS) void k_binstats(KArgs a, Phys p, Grid box, Grid* gd, int wrap, int cap_bits,
+                                                 double* part) {
+  b_binstats(a, p, box, gd, wrap, cap_bits, part, VL{(int)blockIdx.x, (int)gridDim.x});
 }
-
-__device__ __forceinline__ void b_fill_i(int* __restrict__ a, int n, int v, VL vl) {
-  for (int i = vl.b * blockDim.x + threadIdx.x; i < n; i += vl.nb * blockDim.x) a[i] = v;
-}
-__global__ void k_fill_i(int* __restrict__ a, int n, int v) {
-  b_fill_i(a, n, v, VL{(int)blockIdx.x, (int)gridDim.x});
+// grid and scalars alone (the first binning, whose key space the host sizes
+// from the statistics)
+__global__ void k_grid_setup(DScal* sc, Grid* gd, Grid box, Phys p, int cap_bits, int n) {
+  if (threadIdx.x | blockIdx.x) return;
+  grid_setup(sc, gd, box, p, cap_bits, n);
+  init_density_scalars(sc, p, n);
 }
 
 __device__ __forceinline__ int cell_coord(const Grid& g, int d, double x) {
@@ -280,6 +297,46 @@ __device__ __forceinline__ int cell_coord(const Grid& g, int d, double x) {
   if (c < 0) c = 0;
   if (c > g.nc[d] - 1) c = g.nc[d] - 1;
   return c;
+}
+
+// Scans and folds over a wave with DPP moves (row shifts by 1, 2, 4 and 8, then
+// the two row broadcasts): a few cycles a step where a shuffle through LDS
+// takes about a hundred.  After the steps lane 63 holds the fold of all lanes.
+#define NDSP_DPP_STEPS(STEP)                                                   \
+  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf)          \
+  STEP(0x142, 0xa) STEP(0x143, 0xc)
+__device__ __forceinline__ int wave_scan_add(int x) {
+#define NDSP_STEP(ctrl, rows) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false);
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  return x;
+}
+// largest of the lanes' non-negative values
+__device__ __forceinline__ float wave_max_pos(float v) {
+  int x = __float_as_int(v);
+#define NDSP_STEP(ctrl, rows) x = max(x, __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false));
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  return __int_as_float(__builtin_amdgcn_readlane(x, 63));
+}
+// smallest / largest of the lanes' values
+template <bool MAX>
+__device__ __forceinline__ double wave_extreme(double v) {
+#define NDSP_STEP(ctrl, rows)                                                                          \
+  {                                                                                                    \
+    const long long b = __double_as_longlong(v);                                                       \
+    const int l = (int)(unsigned)(b & 0xffffffffll), h = (int)(b >> 32);                               \
+    const unsigned pl = (unsigned)__builtin_amdgcn_update_dpp(l, l, ctrl, rows, 0xf, false);           \
+    const int ph = __builtin_amdgcn_update_dpp(h, h, ctrl, rows, 0xf, false);                          \
+    const double w = __longlong_as_double(((long long)ph << 32) | (long long)pl);                      \
+    v = MAX ? fmax(v, w) : fmin(v, w);                                                                 \
+  }
+  NDSP_DPP_STEPS(NDSP_STEP)
+#undef NDSP_STEP
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffll), 63);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
+  return __longlong_as_double(((long long)hi << 32) | (long long)lo);
 }
 
 // Consecutive lanes of a wave holding the same key (-1: none) form a run; the
@@ -312,95 +369,90 @@ __device__ __forceinline__ void b_cellid(KArgs a, const Grid* __restrict__ gp, V
     c = cell_key(g, cx, cy, cz);
     a.cellid[i] = c;
   }
-  run_atomic_add(a.cfill, c);
+  // its place among the cell's particles in the order of arrival
+  const int r = run_atomic_add(a.cfill, c);
+  if (c >= 0) a.rank[i] = r;
 }
 __global__ void k_cellid(KArgs a, const Grid* __restrict__ gp) {
   b_cellid(a, gp, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-// exclusive scan, 3 phases (1024 elements per block)
-__device__ __forceinline__ void b_scan_local(const int* in, int* out, int* bsum, const Grid* __restrict__ gp, VL vl) {
-  __shared__ int sm[BS];
+// Exclusive scan of the cells' counts, 1024 per block: places within the block
+// into cpart, the block's total into bsum, whose own scan the last block to
+// finish makes.  The counts are cleared as they are read: every binning finds
+// them zero.
+__device__ __forceinline__ void b_scan_local(KArgs a, int* bsum, const Grid* __restrict__ gp, VL vl) {
+  __shared__ int sm[BS / 64];
+  __shared__ int last;
   const long long n = gp->ncell + 1;
-  if ((long long)vl.b * BS * 4 >= n) return;
-  const int ITEMS = 4;
-  long long base = (long long)vl.b * BS * ITEMS + (long long)threadIdx.x * ITEMS;
-  int v[ITEMS];
+  const int nb = (int)((n + BS * 4 - 1) / (BS * 4));  // the blocks with work
+  if (vl.b >= nb) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const long long base = (long long)vl.b * BS * 4 + (long long)threadIdx.x * 4;
+  int v[4];
   int tot = 0;
-  for (int k = 0; k < ITEMS; k++) {
-    long long idx = base + k;
-    v[k] = idx < n ? in[idx] : 0;
+  for (int k = 0; k < 4; k++) {
+    const long long idx = base + k;
+    v[k] = idx < n ? a.cfill[idx] : 0;
+    if (v[k]) a.cfill[idx] = 0;
     tot += v[k];
   }
-  sm[threadIdx.x] = tot;
+  const int inc = wave_scan_add(tot);
+  if (lane == 63) sm[w] = inc;
   __syncthreads();
-  for (int s = 1; s < BS; s <<= 1) {
-    int x = threadIdx.x >= s ? sm[threadIdx.x - s] : 0;
-    __syncthreads();
-    sm[threadIdx.x] += x;
-    __syncthreads();
+  int run = inc - tot, all = 0;
+  for (int u = 0; u < BS / 64; u++) {
+    if (u < w) run += sm[u];
+    all += sm[u];
   }
-  int run = sm[threadIdx.x] - tot;
-  for (int k = 0; k < ITEMS; k++) {
-    long long idx = base + k;
-    if (idx < n) out[idx] = run;
+  for (int k = 0; k < 4; k++) {
+    const long long idx = base + k;
+    if (idx < n) a.cpart[idx] = run;
     run += v[k];
   }
-  if (threadIdx.x == BS - 1) bsum[vl.b] = sm[BS - 1];
-}
-__global__ void k_scan_local(const int* in, int* out, int* bsum, const Grid* __restrict__ gp) {
-  b_scan_local(in, out, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-__device__ __forceinline__ void b_scan_bsum(int* bsum, const Grid* __restrict__ gp, int* total_out, VL vl) {
-  __shared__ int sm[BS];
-  const int nb = (int)((gp->ncell + 1 + BS * 4 - 1) / (BS * 4));
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nb; base += BS) {
-    int idx = base + threadIdx.x;
-    int v = idx < nb ? bsum[idx] : 0;
-    sm[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = 1; s < BS; s <<= 1) {
-      int x = threadIdx.x >= s ? sm[threadIdx.x - s] : 0;
-      __syncthreads();
-      sm[threadIdx.x] += x;
-      __syncthreads();
-    }
-    if (idx < nb) bsum[idx] = carry + sm[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == BS - 1) carry += sm[BS - 1];
-    __syncthreads();
+  if (threadIdx.x == 0) {
+    bsum[vl.b] = all;
+    last = last_block(&a.sc->scan_done, nb);
   }
-  if (threadIdx.x == 0 && total_out) *total_out = carry;
+  __syncthreads();
+  if (!last) return;
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  int carry = 0;
+  for (int b0 = 0; b0 < nb; b0 += BS) {
+    const int idx = b0 + threadIdx.x;
+    const int x = idx < nb ? bsum[idx] : 0;
+    const int xi = wave_scan_add(x);
+    __syncthreads();
+    if (lane == 63) sm[w] = xi;
+    __syncthreads();
+    int off = carry;
+    for (int u = 0; u < BS / 64; u++) {
+      if (u < w) off += sm[u];
+      carry += sm[u];
+    }
+    if (idx < nb) bsum[idx] = off + xi - x;
+  }
+  if (threadIdx.x == 0) a.sc->scan_done = 0;
 }
-__global__ void k_scan_bsum(int* bsum, const Grid* __restrict__ gp, int* total_out) {
-  b_scan_bsum(bsum, gp, total_out, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ __launch_bounds__(BS) void k_scan_local(KArgs a, int* bsum, const Grid* __restrict__ gp) {
+  b_scan_local(a, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-// block offsets onto the cell starts; clears the cells' largest list radii
-// (raised by k_pack_density)
-__device__ __forceinline__ void b_scan_add(KArgs a, const int* bsum, const Grid* __restrict__ gp, VL vl) {
-  const long long n = gp->ncell + 1;
-  long long idx = (long long)vl.b * blockDim.x + threadIdx.x;
-  if (idx >= n) return;
-  a.cstart[idx] += bsum[idx / (BS * 4)];
-  if (a.cellr) a.cellr[idx] = 0.0f;
-}
-__global__ void k_scan_add(KArgs a, const int* bsum, const Grid* __restrict__ gp) {
-  b_scan_add(a, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-__device__ __forceinline__ void b_scatter(KArgs a, VL vl) {
+// the cells' starts (block offsets onto the places), their largest list radii
+// cleared (raised by k_pack_density), and every particle's slot to its place
+__device__ __forceinline__ void b_scatter(KArgs a, const int* __restrict__ bsum, const Grid* __restrict__ gp, VL vl) {
+  const long long n = gp->ncell + 1, step = (long long)vl.nb * blockDim.x;
+  for (long long idx = (long long)vl.b * blockDim.x + threadIdx.x; idx < n; idx += step) {
+    a.cstart[idx] = a.cpart[idx] + bsum[idx / (BS * 4)];
+    if (a.cellr) a.cellr[idx] = 0.0f;
+  }
   const int i = vl.b * blockDim.x + threadIdx.x;
-  const int c = i < a.n ? a.cellid[i] : -1;
-  const int r = run_atomic_add(a.cfill, c);
-  if (c >= 0) a.sidx[a.cstart[c] + r] = i;
+  if (i >= a.n) return;
+  const int c = a.cellid[i];
+  a.sidx[a.cpart[c] + bsum[c / (BS * 4)] + a.rank[i]] = i;
 }
-__global__ void k_scatter(KArgs a) {
-  b_scatter(a, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ void k_scatter(KArgs a, const int* __restrict__ bsum, const Grid* __restrict__ gp) {
+  b_scatter(a, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // ascending order of N values held in registers (bitonic network; every
@@ -614,7 +666,8 @@ __device__ __forceinline__ void pack_force_one(KArgs& a, const Phys& p, int k, c
   }
 }
 template <typename PT>
-__device__ __forceinline__ void b_pack_force(KArgs a, Phys p, VL vl) {
+__device__ __forceinline__ void b_pack_force(KArgs a, Phys p, int guard, VL vl) {
+  if (held_back(a.sc, guard)) return;
   alignas(32) __shared__ float4 stage[BS * fr_bytes<PT>(2) / 16];
   const int phys = fr_phys(p);
   const int rb = (int)fr_bytes<PT>(phys);
@@ -625,8 +678,8 @@ __device__ __forceinline__ void b_pack_force(KArgs a, Phys p, VL vl) {
 }
 
 template <typename PT>
-__global__ void k_pack_force(KArgs a, Phys p) {
-  b_pack_force<PT>(a, p, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ void k_pack_force(KArgs a, Phys p, int guard) {
+  b_pack_force<PT>(a, p, guard, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // ===========================================================================
@@ -859,46 +912,6 @@ __device__ __forceinline__ void sort_extras(const unsigned* E, unsigned* D, int 
 #pragma unroll
   for (int m = 0; m < N; m++)
     if (m < nx) D[m] = v[m];
-}
-
-// Scans and folds over a wave with DPP moves (row shifts by 1, 2, 4 and 8, then
-// the two row broadcasts): a few cycles a step where a shuffle through LDS
-// takes about a hundred.  After the steps lane 63 holds the fold of all lanes.
-#define NDSP_DPP_STEPS(STEP)                                                   \
-  STEP(0x111, 0xf) STEP(0x112, 0xf) STEP(0x114, 0xf) STEP(0x118, 0xf)          \
-  STEP(0x142, 0xa) STEP(0x143, 0xc)
-__device__ __forceinline__ int wave_scan_add(int x) {
-#define NDSP_STEP(ctrl, rows) x += __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false);
-  NDSP_DPP_STEPS(NDSP_STEP)
-#undef NDSP_STEP
-  return x;
-}
-// largest of the lanes' non-negative values
-__device__ __forceinline__ float wave_max_pos(float v) {
-  int x = __float_as_int(v);
-#define NDSP_STEP(ctrl, rows) x = max(x, __builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xf, false));
-  NDSP_DPP_STEPS(NDSP_STEP)
-#undef NDSP_STEP
-  return __int_as_float(__builtin_amdgcn_readlane(x, 63));
-}
-// smallest / largest of the lanes' values
-template <bool MAX>
-__device__ __forceinline__ double wave_extreme(double v) {
-#define NDSP_STEP(ctrl, rows)                                                                          \
-  {                                                                                                    \
-    const long long b = __double_as_longlong(v);                                                       \
-    const int l = (int)(unsigned)(b & 0xffffffffll), h = (int)(b >> 32);                               \
-    const unsigned pl = (unsigned)__builtin_amdgcn_update_dpp(l, l, ctrl, rows, 0xf, false);           \
-    const int ph = __builtin_amdgcn_update_dpp(h, h, ctrl, rows, 0xf, false);                          \
-    const double w = __longlong_as_double(((long long)ph << 32) | (long long)pl);                      \
-    v = MAX ? fmax(v, w) : fmin(v, w);                                                                 \
-  }
-  NDSP_DPP_STEPS(NDSP_STEP)
-#undef NDSP_STEP
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(b & 0xffffffffll), 63);
-  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), 63);
-  return __longlong_as_double(((long long)hi << 32) | (long long)lo);
 }
 
 // One wavefront per 64 consecutive sorted particles.  The order is by Morton
@@ -1329,7 +1342,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_
 // ===========================================================================
 // global reductions without contended atomics: every block reduces its
 // values (wave shuffles, then LDS across waves) and writes one partial per
-// quantity; k_red_final folds the partials into the scalar record.
+// quantity; red_fold folds the partials into the scalar record.
 // ===========================================================================
 
 __device__ __forceinline__ double red_combine(int kind, double a, double b) {
@@ -1358,56 +1371,56 @@ __device__ __forceinline__ void block_partials(double (&v)[NQ], const int (&kind
   }
 }
 
-__device__ __forceinline__ void b_red_final(const double* __restrict__ red, int rcap, int nblocks,
-                                                  RedSpec spec, DScal* sc, const int* skip, VL vl) {
-  if (skip && *skip) return;
-  // every quantity at once: each thread folds its blocks for all of them
-  // (eight blocks a step, so that up to 8 x nq loads are in flight), then a
-  // butterfly per wave and the waves in order (every fold here is a min, a
-  // max or a sum of integers: exact in any order)
-  __shared__ double sw[BS / 64][RED_MAXQ];
-  const int nq = spec.nq;
-  int kind[RED_MAXQ];
-  double acc[RED_MAXQ];
+// Folds the NQ quantities of spec over the partials of nblocks blocks into the
+// scalar record, by one block of up to FOLD_B threads (every fold here is a min,
+// a max or a sum of integers: exact in any order).  Eight blocks a step and
+// thread, so that 8 x NQ loads are in flight; then a butterfly per wave and the
+// waves in order.
+#define FOLD_B 1024
+template <int NQ>
+__device__ __forceinline__ void red_fold(const double* __restrict__ red, int rcap, int nblocks, const RedSpec& spec,
+                                         DScal* sc) {
+  __shared__ double sw[FOLD_B / 64][NQ];
+  const int nt = blockDim.x;
+  int kind[NQ];
+  double acc[NQ];
 #pragma unroll
-  for (int q = 0; q < RED_MAXQ; q++) {
-    kind[q] = q < nq ? (spec.op[q] & 15) : RED_SUM;
+  for (int q = 0; q < NQ; q++) {
+    kind[q] = spec.op[q] & 15;
     acc[q] = kind[q] == RED_SUM ? 0.0 : kind[q] == RED_MAX ? -DBL_MAX : DBL_MAX;
   }
   int b = threadIdx.x;
-  for (; b + 7 * BS < nblocks; b += 8 * BS) {
+  for (; b + 7 * nt < nblocks; b += 8 * nt) {
 #pragma unroll
-    for (int q = 0; q < RED_MAXQ; q++) {
-      if (q >= nq) continue;
+    for (int q = 0; q < NQ; q++) {
       const double* __restrict__ rq = red + (size_t)q * rcap + b;
       double v[8];
 #pragma unroll
-      for (int u = 0; u < 8; u++) v[u] = rq[u * BS];
+      for (int u = 0; u < 8; u++) v[u] = rq[u * nt];
 #pragma unroll
       for (int u = 0; u < 8; u++) acc[q] = red_combine(kind[q], acc[q], v[u]);
     }
   }
-  for (; b < nblocks; b += BS) {
+  for (; b < nblocks; b += nt) {
 #pragma unroll
-    for (int q = 0; q < RED_MAXQ; q++)
-      if (q < nq) acc[q] = red_combine(kind[q], acc[q], red[(size_t)q * rcap + b]);
+    for (int q = 0; q < NQ; q++) acc[q] = red_combine(kind[q], acc[q], red[(size_t)q * rcap + b]);
   }
 #pragma unroll
-  for (int q = 0; q < RED_MAXQ; q++) {
+  for (int q = 0; q < NQ; q++) {
     double x = acc[q];
     for (int o = 32; o > 0; o >>= 1) x = red_combine(kind[q], x, __shfl_xor(x, o, 64));
     acc[q] = x;
   }
   if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-    for (int q = 0; q < RED_MAXQ; q++) sw[threadIdx.x >> 6][q] = acc[q];
+    for (int q = 0; q < NQ; q++) sw[threadIdx.x >> 6][q] = acc[q];
   }
   __syncthreads();
-  if ((int)threadIdx.x < nq) {
+  if ((int)threadIdx.x < NQ) {
     const int q = threadIdx.x;
     const int kq = spec.op[q] & 15, type = spec.op[q] >> 4;
     double r = sw[0][q];
-    for (int w = 1; w < BS / 64; w++) r = red_combine(kq, r, sw[w][q]);
+    for (int w = 1; w < (nt >> 6); w++) r = red_combine(kq, r, sw[w][q]);
     char* base = (char*)sc + spec.off[q];
     if (type == RED_F64) {
       double* d = (double*)base;
@@ -1420,10 +1433,14 @@ __device__ __forceinline__ void b_red_final(const double* __restrict__ red, int 
       *d = kq == RED_SUM ? *d + (unsigned long long)r : (unsigned long long)red_combine(kq, (double)*d, r);
     }
   }
+  __syncthreads();
 }
-__global__ __launch_bounds__(BS) void k_red_final(const double* __restrict__ red, int rcap, int nblocks,
-                                                  RedSpec spec, DScal* sc, const int* skip) {
-  b_red_final(red, rcap, nblocks, spec, sc, skip, VL{(int)blockIdx.x, (int)gridDim.x});
+// the scalar record to the host's copy (pinned memory), by the whole block
+__device__ __forceinline__ void scalars_out(const DScal* sc, DScal* out) {
+  __threadfence();
+  __syncthreads();
+  const int* src = (const int*)sc;
+  for (int w = threadIdx.x; w < (int)(sizeof(DScal) / sizeof(int)); w += blockDim.x) ((int*)out)[w] = src[w];
 }
 
 static RedSpec red_spec(std::initializer_list<std::pair<int, int>> q) {
@@ -1492,15 +1509,13 @@ __device__ __forceinline__ void nr_update(const Phys& p, double hh, double hin, 
 template <int NDIM, typename PT, bool DUST, int TB>
 __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restrict__ gp, int* __restrict__ list_a,
                                                 int* __restrict__ list_b, VL vl) {
-  // pass parameters from the device-side control (k_pass_ctl): pass its0
-  // reads the active list written by the previous pass (list_a after odd
-  // passes, list_b after even ones) and appends its unconverged particles to
-  // the other one
+  // pass parameters from the device-side control (pass_ctl): pass its0
+  // reads the active list made after the previous pass (list_a after odd
+  // passes, list_b after even ones)
   if (a.sc->pc_done) return;
   const int nlist = a.sc->pc_nlist, its0 = a.sc->pc_its, sym = a.sc->pc_sym;
   const int persistent = a.sc->pc_persistent;
   const int* __restrict__ list = its0 == 1 ? nullptr : ((its0 & 1) ? list_b : list_a);
-  int* __restrict__ next_list = (its0 & 1) ? list_a : list_b;
   // a workgroup with no particle of this pass skips loading the tables (a
   // later pass holds only the particles still iterating); it still writes
   // its neutral reduction partials, which the final fold reads
@@ -1723,19 +1738,21 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
     const int rk[7] = {RED_MAX, RED_MAX, RED_MAX, RED_MIN, RED_MAX, RED_SUM, RED_SUM};
     block_partials<7>(rv, rk, a.red, a.rcap, vl);
   }
-  // unconverged particles form the next pass's list: flagged here and
-  // compacted in sorted order afterwards (k_cmp_*), so that the next pass's
-  // workgroups keep the spatial order, or appended one atomic per wave
-  if (!persistent && a.nrflag) {
-    if (active) a.nrflag[k] = unconverged ? 1 : 0;
-  } else if (!persistent) {
-    const unsigned long long m = __ballot(unconverged);
-    const int lane = threadIdx.x & 63;
-    const int cnt = __popcll(m);
-    int base = 0;
-    if (lane == 0 && cnt) base = atomicAdd(&a.sc->ncalc_next, cnt);
-    base = __shfl(base, 0);
-    if (unconverged) next_list[base + __popcll(m & ((1ull << lane) - 1ull))] = k;
+  // unconverged particles form the next pass's list: flagged by their place in
+  // this one and counted per tile; k_pass_fold scans the counts and
+  // k_pass_next moves them up in order, so that the next pass's workgroups keep
+  // the spatial order
+  if (!persistent && !idle) {
+    __shared__ int wcnt[TB / 64];
+    if (active) a.nrflag[tid] = unconverged ? 1 : 0;
+    const int cnt = __popcll(__ballot(unconverged));
+    if ((threadIdx.x & 63) == 0) wcnt[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int tot = 0;
+      for (int w = 0; w < TB / 64; w++) tot += wcnt[w];
+      a.nrcnt[tile] = tot;
+    }
   }
 }
 // three waves per SIMD (an occupancy attribute): with one record in flight
@@ -1746,149 +1763,120 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_
   b_nr_pass<NDIM, PT, DUST, TB>(a, p, gp, list_a, list_b, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-// P4.w = 1/h of every particle before a symmetric pass after the first, and
-// the reflecting ghost extents after a relink (as decided by k_pass_ctl)
-__device__ __forceinline__ void b_refresh_hinv(KArgs a, Phys p, VL vl) {
-  if (a.sc->pc_done || !a.sc->pc_refresh) return;
-  const int refresh_dxb = a.sc->pc_relink;
-  int k = vl.b * blockDim.x + threadIdx.x;
-  if (k >= a.n) return;
-  const double h = a.f[F_H][a.sidx[k]];
-  a.P4[k].w = 1.0 / h;
-  ((double4*)((char*)a.DR + (size_t)k * a.dr_stride))->w = 1.0 / h;
-  if (refresh_dxb) a.dxb[k] = p.radkern * h;
-}
-__global__ void k_refresh_hinv(KArgs a, Phys p) {
-  b_refresh_hinv(a, p, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-// max h over all particles -> hmax_cur (and the ghost extent on a relink)
-__device__ __forceinline__ void b_hmax(KArgs a, DScal* sc, VL vl) {
-  if (sc->pc_done) return;
-  const int relink = sc->pc_relink;
-  __shared__ double sm[BS];
-  double hm = 0.0;
-  for (int i = vl.b * blockDim.x + threadIdx.x; i < a.n; i += vl.nb * blockDim.x)
-    hm = fmax(hm, a.f[F_H][i]);
-  sm[threadIdx.x] = hm;
-  __syncthreads();
-  for (int s = BS / 2; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sm[threadIdx.x] = fmax(sm[threadIdx.x], sm[threadIdx.x + s]);
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    atomic_max_pos(&sc->hmax_cur, sm[0]);
-    if (relink) atomic_max_pos(&sc->hhmax_ghost, sm[0]);
-  }
-}
-__global__ void k_hmax(KArgs a, DScal* sc) {
-  b_hmax(a, sc, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-// After a pass (src/iterate_density.f90:280-300): finished when the pass was
-// the persistent one, failed, or left no particle unconverged; otherwise the
-// unconverged ones form the next pass, symmetric if they are all particles
+// The pass control (src/iterate_density.f90:280-300): finished when the pass
+// was the persistent one, failed, or left no particle unconverged; otherwise
+// the unconverged ones form the next pass, symmetric if they are all particles
 // (:131-135), synchronous while walls reflect (a relink, :260-262, rebuilds
 // the ghosts with every particle's current h).
-__device__ __forceinline__ void b_pass_ctl(DScal* sc, int n, int reflect, int maxits, VL vl) {
-  if (threadIdx.x | vl.b) return;
-  if (sc->pc_done) return;
-  if (sc->pc_persistent || sc->err || sc->ncalc_next == 0 || sc->pc_its > maxits) {
+__device__ __forceinline__ void pass_ctl(DScal* sc, int n, int reflect, int maxits) {
+  const int nl = sc->ncalc_next;
+  sc->ncalc_next = 0;
+  sc->pc_nprev = sc->pc_nlist;
+  if (sc->pc_persistent || sc->err || nl == 0 || sc->pc_its > maxits) {
     sc->pc_done = 1;
+    sc->phase = 1;
     return;
   }
   const int relink = reflect && sc->relink;
-  const int nl = sc->ncalc_next;
   sc->pc_nlist = nl;
   sc->pc_its = sc->pc_its + 1;
   sc->pc_sym = nl == n;
   sc->pc_persistent = !reflect && nl != n;
   sc->pc_relink = relink;
   sc->pc_refresh = nl == n || relink;
-  sc->ncalc_next = 0;
   sc->relink = 0;
   sc->hmax_cur = 0.0;
   if (relink) sc->hhmax_ghost = 0.0;
 }
-__global__ void k_pass_ctl(DScal* sc, int n, int reflect, int maxits) {
-  b_pass_ctl(sc, n, reflect, maxits, VL{(int)blockIdx.x, (int)gridDim.x});
+// After a pass, one block of up to FOLD_B threads: the pass's reductions, the scan
+// of the tiles' unconverged counts (their total is the next pass's size), the
+// control, and (out not null) the scalars to the host.  One launch for three
+// and a copy.
+__device__ __forceinline__ void b_pass_fold(KArgs a, const RedSpec& spec, int nblocks, int tb, int reflect, int maxits,
+                                            DScal* out) {
+  __shared__ int ws[FOLD_B / 64];
+  DScal* sc = a.sc;
+  if (!sc->pc_done) {
+    red_fold<7>(a.red, a.rcap, nblocks, spec, sc);
+    if (!sc->pc_persistent) {
+      const int nt = (sc->pc_nlist + tb - 1) / tb;
+      const int per = (nt + (int)blockDim.x - 1) / (int)blockDim.x;
+      const int t0 = min(nt, (int)threadIdx.x * per), t1 = min(nt, t0 + per);
+      int tot = 0;
+      for (int t = t0; t < t1; t++) tot += a.nrcnt[t];
+      const int inc = wave_scan_add(tot), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+      if (lane == 63) ws[w] = inc;
+      __syncthreads();
+      int run = inc - tot, all = 0;
+      for (int u = 0; u < ((int)blockDim.x >> 6); u++) {
+        if (u < w) run += ws[u];
+        all += ws[u];
+      }
+      for (int t = t0; t < t1; t++) {
+        const int c = a.nrcnt[t];
+        a.nrcnt[t] = run;
+        run += c;
+      }
+      if (threadIdx.x == 0) sc->ncalc_next = all;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) pass_ctl(sc, a.n, reflect, maxits);
+  }
+  if (out) scalars_out(sc, out);
+}
+__global__ __launch_bounds__(FOLD_B) void k_pass_fold(KArgs a, RedSpec spec, int nblocks, int tb, int reflect,
+                                                      int maxits, DScal* out) {
+  b_pass_fold(a, spec, nblocks, tb, reflect, maxits, out);
 }
 
-// Ordered compaction of the flags a pass left (sorted positions of the
-// unconverged particles) into the next pass's list, in three launches over
-// blocks of CMP_ITEMS*BS flags: per-block counts, their exclusive scan (and
-// the total, the next pass's size), and the scatter, which also clears the
-// flags it reads.
-#define CMP_ITEMS 4
-__global__ __launch_bounds__(BS) void k_cmp_count(const int* __restrict__ flag, int n, int* __restrict__ bsum) {
-  __shared__ int ws[BS / 64];
-  const long long base = (long long)blockIdx.x * BS * CMP_ITEMS;
-  int c = 0;
-  for (int q = 0; q < CMP_ITEMS; q++) {
-    const long long i = base + (long long)q * BS + threadIdx.x;
-    if (i < n) c += flag[i];
+// What the next pass needs (as pass_ctl decided): its list, the flagged places
+// of the last one moved up in order; before a symmetric pass after the first,
+// P4.w = 1/h and max h of every particle; after a relink the reflecting ghost
+// extents and hhmax.
+__device__ __forceinline__ void b_pass_next(KArgs a, const Phys& p, int tb, int* __restrict__ list_a,
+                                            int* __restrict__ list_b, VL vl) {
+  DScal* sc = a.sc;
+  if (sc->pc_done) return;
+  __shared__ int wc[BS / 64];
+  __shared__ double sm[BS / 64];
+  const int k = vl.b * blockDim.x + threadIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int its0 = sc->pc_its - 1, nprev = sc->pc_nprev;
+  if (vl.b * (int)blockDim.x < nprev) {
+    const int* __restrict__ from = its0 == 1 ? nullptr : ((its0 & 1) ? list_b : list_a);
+    int* __restrict__ to = (its0 & 1) ? list_a : list_b;
+    const bool f = k < nprev && a.nrflag[k] != 0;
+    const unsigned long long m = __ballot(f);
+    if (lane == 0) wc[w] = __popcll(m);
+    __syncthreads();
+    if (f) {
+      int at = a.nrcnt[k / tb] + __popcll(m & ((1ull << lane) - 1ull));
+      // the earlier waves of the same tile
+      for (int u = w - 1; u >= 0 && (vl.b * (int)blockDim.x + 64 * u) / tb == k / tb; u--) at += wc[u];
+      to[at] = from ? from[k] : k;
+    }
   }
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if ((threadIdx.x & 63) == 0) ws[threadIdx.x >> 6] = c;
+  if (!sc->pc_refresh) return;
+  const int relink = sc->pc_relink;
+  double h = 0.0;
+  if (k < a.n) {
+    h = a.f[F_H][a.sidx[k]];
+    a.P4[k].w = 1.0 / h;
+    ((double4*)((char*)a.DR + (size_t)k * a.dr_stride))->w = 1.0 / h;
+    if (relink) a.dxb[k] = p.radkern * h;
+  }
+  for (int o = 32; o > 0; o >>= 1) h = fmax(h, __shfl_xor(h, o));
+  if (lane == 0) sm[w] = h;
   __syncthreads();
   if (threadIdx.x == 0) {
-    int t = 0;
-    for (int w = 0; w < BS / 64; w++) t += ws[w];
-    bsum[blockIdx.x] = t;
+    for (int u = 1; u < BS / 64; u++) h = fmax(h, sm[u]);
+    atomic_max_pos(&sc->hmax_cur, h);
+    if (relink) atomic_max_pos(&sc->hhmax_ghost, h);
   }
 }
-__global__ __launch_bounds__(BS) void k_cmp_scan(int* __restrict__ bsum, int nb, DScal* sc) {
-  __shared__ int sm[BS];
-  __shared__ int carry;
-  if (threadIdx.x == 0) carry = 0;
-  __syncthreads();
-  for (int base = 0; base < nb; base += BS) {
-    const int idx = base + threadIdx.x;
-    const int v = idx < nb ? bsum[idx] : 0;
-    sm[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = 1; s < BS; s <<= 1) {
-      const int x = (int)threadIdx.x >= s ? sm[threadIdx.x - s] : 0;
-      __syncthreads();
-      sm[threadIdx.x] += x;
-      __syncthreads();
-    }
-    if (idx < nb) bsum[idx] = carry + sm[threadIdx.x] - v;
-    __syncthreads();
-    if (threadIdx.x == BS - 1) carry += sm[BS - 1];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) sc->ncalc_next = carry;
+__global__ __launch_bounds__(BS) void k_pass_next(KArgs a, Phys p, int tb, int* __restrict__ list_a,
+                                                  int* __restrict__ list_b) {
+  b_pass_next(a, p, tb, list_a, list_b, VL{(int)blockIdx.x, (int)gridDim.x});
 }
-__global__ __launch_bounds__(BS) void k_cmp_scatter(int* __restrict__ flag, int n, const int* __restrict__ bsum,
-                                                    const DScal* __restrict__ sc, int* __restrict__ list_a,
-                                                    int* __restrict__ list_b) {
-  __shared__ int ws[BS / 64];
-  // the list the pass that set the flags names as its next (b_nr_pass)
-  int* __restrict__ out = (sc->pc_its & 1) ? list_a : list_b;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const long long base = (long long)blockIdx.x * BS * CMP_ITEMS;
-  int run = bsum[blockIdx.x];
-  for (int q = 0; q < CMP_ITEMS; q++) {
-    const long long i = base + (long long)q * BS + threadIdx.x;
-    const int f = i < n ? flag[i] : 0;
-    const unsigned long long m = __ballot(f != 0);
-    if (lane == 0) ws[w] = __popcll(m);
-    __syncthreads();
-    int off = run, tot = 0;
-    for (int u = 0; u < BS / 64; u++) {
-      if (u < w) off += ws[u];
-      tot += ws[u];
-    }
-    if (f) {
-      out[off + __popcll(m & ((1ull << lane) - 1ull))] = (int)i;
-      flag[i] = 0;
-    }
-    run += tot;
-    __syncthreads();
-  }
-}
-
 
 // ===========================================================================
 // force: fused pair sums of get_rates
@@ -1897,7 +1885,8 @@ __global__ __launch_bounds__(BS) void k_cmp_scatter(int* __restrict__ flag, int 
 // PHYS: 0 hydro, 1 MHD (imhd 11), 2 one-fluid dust (idust 4); TB threads
 // per workgroup (chosen by the autotuner)
 template <int NDIM, typename PT, int PHYS, int TB>
-__device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict__ gp, VL vl) {
+__device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict__ gp, int guard, VL vl) {
+  if (held_back(a.sc, guard)) return;
   __shared__ PT tg[NDSP_IKERN + 1];
   {
     const PT* src = sizeof(PT) == 4 ? (const PT*)a.tabf : (const PT*)a.tabd;
@@ -2216,8 +2205,8 @@ __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict_
   }
 }
 template <int NDIM, typename PT, int PHYS, int TB>
-__global__ __launch_bounds__(TB) void k_force(KArgs a, Phys p, const Grid* __restrict__ gp) {
-  b_force<NDIM, PT, PHYS, TB>(a, p, gp, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ __launch_bounds__(TB) void k_force(KArgs a, Phys p, const Grid* __restrict__ gp, int guard) {
+  b_force<NDIM, PT, PHYS, TB>(a, p, gp, guard, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // per-particle finalisation, src/ratesND_mhd.f90:482-943 (FP64)
@@ -2318,32 +2307,55 @@ __global__ void k_finalize(KArgs a, Phys p) {
   b_finalize(a, p, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
-// timestep, src/ratesND_mhd.f90:938-943 and src/stepND_leapfrog_mhd.f90:252
-__device__ __forceinline__ void b_dt(DScal* sc, Phys p, VL vl) {
-  if (threadIdx.x | vl.b) return;
-  double dtforce = DBL_MAX;
-  if (sc->fhmax > 0.0) dtforce = fmin(dtforce, sqrt(1.0 / sc->fhmax));
-  sc->dtforce = dtforce;
-  sc->dt = fmin(fmin(fmin(p.C_force * dtforce, p.C_cour * sc->dtcourant), 0.9 * sc->dtdrag),
-                p.C_force * DBL_MAX);
+// The force pass's reductions, by one block: they start from the values the
+// scalars have without any pair.
+__device__ __forceinline__ void b_force_fold(KArgs a, const RedSpec& spec, int nblocks, int guard) {
+  DScal* sc = a.sc;
+  if (held_back(sc, guard)) return;
+  if (threadIdx.x == 0) {
+    sc->vsigmax = 0.0;
+    sc->dtcourant = 1.0e6;
+    sc->fhmax = 0.0;
+    sc->dtdrag = DBL_MAX;
+    sc->pairs_force = 0;
+  }
+  __syncthreads();
+  red_fold<3>(a.red, a.rcap, nblocks, spec, sc);
 }
-__global__ void k_dt(DScal* sc, Phys p) {
-  b_dt(sc, p, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ __launch_bounds__(FOLD_B) void k_force_fold(KArgs a, RedSpec spec, int nblocks, int guard) {
+  b_force_fold(a, spec, nblocks, guard);
+}
+// The finalisation's reductions and the timestep (src/ratesND_mhd.f90:938-943,
+// src/stepND_leapfrog_mhd.f90:252), by one block; at the end of a leapfrog step
+// (end) the time advances by the step's dt and the next one takes the dt just
+// chosen (src/evolve.f90:106-110); out: the scalars to the host.
+__device__ __forceinline__ void b_dt_fold(KArgs a, const Phys& p, const RedSpec& spec, int nblocks, int guard, int end,
+                                          DScal* out) {
+  DScal* sc = a.sc;
+  if (!held_back(sc, guard)) {
+    red_fold<2>(a.red, a.rcap, nblocks, spec, sc);
+    if (threadIdx.x == 0) {
+      double dtforce = DBL_MAX;
+      if (sc->fhmax > 0.0) dtforce = fmin(dtforce, sqrt(1.0 / sc->fhmax));
+      sc->dtforce = dtforce;
+      sc->dt = fmin(fmin(fmin(p.C_force * dtforce, p.C_cour * sc->dtcourant), 0.9 * sc->dtdrag),
+                    p.C_force * DBL_MAX);
+      if (end) {
+        sc->time = sc->time + sc->dt_cur;
+        sc->dt_cur = sc->dt;
+        sc->phase = 0;
+      }
+    }
+  }
+  if (out) scalars_out(sc, out);
+}
+__global__ __launch_bounds__(FOLD_B) void k_dt_fold(KArgs a, Phys p, RedSpec spec, int nblocks, int guard, int end,
+                                                    DScal* out) {
+  b_dt_fold(a, p, spec, nblocks, guard, end, out);
 }
 
-// end of a leapfrog step: advance the time by the step's dt and take the dt
-// chosen by this step's rates for the next one (src/evolve.f90:106-110)
-__device__ __forceinline__ void b_step_end(DScal* sc, VL vl) {
-  if (threadIdx.x | vl.b) return;
-  sc->time = sc->time + sc->dt_cur;
-  sc->dt_cur = sc->dt;
-}
-__global__ void k_step_end(DScal* sc) {
-  b_step_end(sc, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-__device__ __forceinline__ void b_init_density_scalars(DScal* sc, double bconstmax, int n, VL vl) {
-  if (threadIdx.x | vl.b) return;
+__device__ __forceinline__ void init_density_scalars(DScal* sc, const Phys& p, int n) {
+  sc->phase = 0;
   sc->pc_nlist = n;
   sc->pc_its = 1;
   sc->pc_sym = 1;
@@ -2357,27 +2369,16 @@ __device__ __forceinline__ void b_init_density_scalars(DScal* sc, double bconstm
   sc->ncalc_next = 0;
   sc->relink = 0;
   sc->list_invalid = 0;
-  sc->stressmax = fmax(0.0, bconstmax);
+  sc->stressmax = fmax(0.0, p.Bconstmax);
   sc->itsmax = 0;
   sc->nmin = INT_MAX;
   sc->nmax = 0;
   sc->pairs_density = 0;
   sc->ncalc_total = 0;
 }
-__global__ void k_init_density_scalars(DScal* sc, double bconstmax, int n) {
-  b_init_density_scalars(sc, bconstmax, n, VL{(int)blockIdx.x, (int)gridDim.x});
-}
-
-__device__ __forceinline__ void b_init_force_scalars(DScal* sc, VL vl) {
-  if (threadIdx.x | vl.b) return;
-  sc->vsigmax = 0.0;
-  sc->dtcourant = 1.0e6;
-  sc->fhmax = 0.0;
-  sc->dtdrag = DBL_MAX;
-  sc->pairs_force = 0;
-}
-__global__ void k_init_force_scalars(DScal* sc) {
-  b_init_force_scalars(sc, VL{(int)blockIdx.x, (int)gridDim.x});
+// (an iteration that does not follow a binning directly)
+__global__ void k_init_density_scalars(DScal* sc, Phys p, int n) {
+  if (!(threadIdx.x | blockIdx.x)) init_density_scalars(sc, p, n);
 }
 
 // ===========================================================================
@@ -2474,7 +2475,8 @@ __global__ void k_predict_fixed(KArgs a, Phys p) {
 // conservative2primitive.f90:425-432): mass, density, h, energies, B,
 // switches, psi, the h terms, pressure and sound speed, and the dust
 // fields; position and velocity stay its own.  Rates are formed afterwards.
-__device__ __forceinline__ void b_fixed_copy(KArgs a, Phys p, VL vl) {
+__device__ __forceinline__ void b_fixed_copy(KArgs a, Phys p, int guard, VL vl) {
+  if (held_back(a.sc, guard)) return;
   const int i = vl.b * blockDim.x + threadIdx.x;
   if (!p.fixed_on || i >= a.n || a.itype[i] != 1) return;
   const int j = a.slot_of[a.ireal[i]];
@@ -2487,8 +2489,8 @@ __device__ __forceinline__ void b_fixed_copy(KArgs a, Phys p, VL vl) {
                            F_EPS, F_RHOGAS, F_RHODUST, F_DVX, F_DVY, F_DVZ};
   for (int q = 0; q < (int)(sizeof cf / sizeof cf[0]); q++) a.f[cf[q]][i] = a.f[cf[q]][j];
 }
-__global__ void k_fixed_copy(KArgs a, Phys p) {
-  b_fixed_copy(a, p, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ void k_fixed_copy(KArgs a, Phys p, int guard) {
+  b_fixed_copy(a, p, guard, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // slot of every caller index (after uploads and reorders)
@@ -2536,13 +2538,18 @@ __device__ __forceinline__ void b_correct(KArgs a, Phys p, VL vl) {
   if (p.idivbzero >= 2) f[F_PSI][i] = f[F_PSIIN][i] + hdt * (f[F_DPSIDT][i] + f[F_DPSIDTIN][i]);
   if (p.idust) f[F_EPS][i] = f[F_EPSIN][i] + hdt * (f[F_DEPS][i] + f[F_DEPSIN][i]);
 }
-// finalize, then the corrector, particle by particle: neither reads another
-// particle's fields, and the rates the corrector reads were just written by
-// the same thread (no second pass over them from HBM)
-__global__ void k_finalize_correct(KArgs a, Phys p) {
-  const VL vl{(int)blockIdx.x, (int)gridDim.x};
+// finalize, then the corrector and the boundary, particle by particle: none
+// reads another particle's fields, and the rates the corrector reads were just
+// written by the same thread (no second pass over them from HBM)
+__device__ __forceinline__ void b_finalize_correct(KArgs a, const Phys& p, const Grid& box, int guard, VL vl) {
+  if (held_back(a.sc, guard)) return;
   b_finalize(a, p, vl);
   b_correct(a, p, vl);
+  const int i = vl.b * blockDim.x + threadIdx.x;
+  if (i < a.n) boundary_one(a, p, box, 1, i);
+}
+__global__ void k_finalize_correct(KArgs a, Phys p, Grid box, int guard) {
+  b_finalize_correct(a, p, box, guard, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // ===========================================================================
@@ -2912,16 +2919,18 @@ __global__ void k_upload_rest(KArgs a, int set_itype) {
   for (int fi = F_RHO; fi < F_NFIELDS; fi++)
     a.f[fi][i] = fi == F_BFX ? bx : fi == F_BFY ? by : fi == F_BFZ ? bz : fi == F_DUSTFRAC ? eps : 0.0;
 }
-// components f0.. of slot s -> out[uid[s]*w + d]
+// component d of caller index i -> out[i*w + d] (written in order: out may be
+// host memory)
 struct CallerFields {
   const double* f[3];
   const int* i;  // an integer field instead, when not null
   int slots;     // or the slots themselves
 };
-__global__ void k_to_caller(CallerFields c, const int* __restrict__ uid, double* __restrict__ out, int w, int n) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  double* r = out + (size_t)uid[s] * w;
+__global__ void k_to_caller(CallerFields c, const int* __restrict__ slot_of, double* __restrict__ out, int w, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int s = slot_of[i];
+  double* r = out + (size_t)i * w;
   if (c.slots) {
     r[0] = s;
   } else if (c.i) {
@@ -3017,8 +3026,7 @@ struct MArgs {
   int* bsum;      // scan block sums
   int* list_a;
   int* list_b;
-  DScal* out;     // slot of this member in the batch's scalar array
-  double bconstmax;
+  DScal* out;     // this member's scalars on the host (pinned)
   int cap_bits;
   int reflect;
   int nbp;        // binning-statistics blocks
@@ -3045,35 +3053,31 @@ __device__ __forceinline__ int member_of(const int* __restrict__ off, int nm, in
 
 NDSP_MK(km_predict) { NDSP_MEMBER b_predict(M.a, M.p, vl); }
 NDSP_MK(km_predict_fixed) { NDSP_MEMBER b_predict_fixed(M.a, M.p, vl); }
-NDSP_MK(km_fixed_copy) { NDSP_MEMBER b_fixed_copy(M.a, M.p, vl); }
 NDSP_MK(km_slot_of) { NDSP_MEMBER b_slot_of(M.a, vl); }
-NDSP_MK(km_correct) { NDSP_MEMBER b_correct(M.a, M.p, vl); }
-NDSP_MK(km_boundary_step) { NDSP_MEMBER b_boundary(M.a, M.p, M.box, 1, vl); }
-NDSP_MK(km_err_reset) { NDSP_MEMBER if (threadIdx.x == 0) M.a.sc->err = 0; }
-NDSP_MK(km_binstats) { NDSP_MEMBER b_binstats(M.a, M.p.ndim, M.part, vl); }
-NDSP_MK(km_binstats_final) { NDSP_MEMBER b_binstats_final(M.a.sc, M.part, M.nbp, vl); }
-NDSP_MK(km_grid_setup) { NDSP_MEMBER b_grid_setup(M.a.sc, M.gdev, M.box, M.p, M.cap_bits, vl); }
-NDSP_MK(km_fill_cells) { NDSP_MEMBER b_fill_cells(M.a.cfill, M.gdev, vl); }
 NDSP_MK(km_cellid) { NDSP_MEMBER b_cellid(M.a, M.gdev, vl); }
-NDSP_MK(km_scan_local) { NDSP_MEMBER b_scan_local(M.a.cfill, M.a.cstart, M.bsum, M.gdev, vl); }
-NDSP_MK(km_scan_bsum) { NDSP_MEMBER b_scan_bsum(M.bsum, M.gdev, nullptr, vl); }
-NDSP_MK(km_scan_add) { NDSP_MEMBER b_scan_add(M.a, M.bsum, M.gdev, vl); }
-NDSP_MK(km_scatter) { NDSP_MEMBER b_scatter(M.a, vl); }
 NDSP_MK(km_cellsort) { NDSP_MEMBER b_cellsort_wave(M.a, M.gdev, vl); }
-NDSP_MK(km_init_density) { NDSP_MEMBER b_init_density_scalars(M.a.sc, M.bconstmax, M.a.n, vl); }
-NDSP_MK(km_pass_ctl) { NDSP_MEMBER b_pass_ctl(M.a.sc, M.a.n, M.reflect, M.p.maxits, vl); }
-NDSP_MK(km_hmax) { NDSP_MEMBER b_hmax(M.a, M.a.sc, vl); }
-NDSP_MK(km_refresh_hinv) { NDSP_MEMBER b_refresh_hinv(M.a, M.p, vl); }
-NDSP_MK(km_init_force) { NDSP_MEMBER b_init_force_scalars(M.a.sc, vl); }
-NDSP_MK(km_finalize) { NDSP_MEMBER b_finalize(M.a, M.p, vl); }
-NDSP_MK(km_dt) { NDSP_MEMBER b_dt(M.a.sc, M.p, vl); }
-NDSP_MK(km_step_end) { NDSP_MEMBER b_step_end(M.a.sc, vl); }
-// every member's scalars into the batch's contiguous array (one copy to the host)
-NDSP_MK(km_gather_scalars) {
+NDSP_MK(km_fixed_copy) { NDSP_MEMBER b_fixed_copy(M.a, M.p, 1, vl); }
+NDSP_MK(km_binstats) { NDSP_MEMBER b_binstats(M.a, M.p, M.box, M.gdev, 1, M.cap_bits, M.part, vl); }
+NDSP_MK(km_scan_local) { NDSP_MEMBER b_scan_local(M.a, M.bsum, M.gdev, vl); }
+NDSP_MK(km_scatter) { NDSP_MEMBER b_scatter(M.a, M.bsum, M.gdev, vl); }
+NDSP_MK(km_finalize_correct) { NDSP_MEMBER b_finalize_correct(M.a, M.p, M.box, 1, vl); }
+// after a pass, the force pass and the finalisation: one block per member
+__global__ __launch_bounds__(FOLD_B) void km_pass_fold(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm,
+                                                       RedSpec spec, int tb, int last) {
   NDSP_MEMBER
-  const int* src = (const int*)M.a.sc;
-  int* dst = (int*)M.out;
-  for (int w = threadIdx.x; w < (int)(sizeof(DScal) / sizeof(int)); w += blockDim.x) dst[w] = src[w];
+  b_pass_fold(M.a, spec, M.nb_nr, tb, M.reflect, M.p.maxits, last ? M.out : nullptr);
+}
+NDSP_MK(km_pass_next_64) { NDSP_MEMBER b_pass_next(M.a, M.p, 64, M.list_a, M.list_b, vl); }
+NDSP_MK(km_pass_next_256) { NDSP_MEMBER b_pass_next(M.a, M.p, 256, M.list_a, M.list_b, vl); }
+__global__ __launch_bounds__(FOLD_B) void km_force_fold(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm,
+                                                        RedSpec spec) {
+  NDSP_MEMBER
+  b_force_fold(M.a, spec, M.nb_force, 1);
+}
+__global__ __launch_bounds__(FOLD_B) void km_dt_fold(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm,
+                                                     RedSpec spec) {
+  NDSP_MEMBER
+  b_dt_fold(M.a, M.p, spec, M.nb_256, 1, 1, M.out);
 }
 // a block of fields of the periodic reorder (slot k <- sorted position k) of
 // the members flagged in due: phase 0 gathers fields f0 .. f0+REORDER_W-1
@@ -3104,17 +3108,10 @@ __global__ void km_reorder(const MArgs* __restrict__ ma, const int* __restrict__
     }
   }
 }
-// reductions: which[0] = h-rho pass (skipped once finished), 1 = force, 2 = finalize
-__global__ void km_red_final(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm, RedSpec spec,
-                             int which) {
-  NDSP_MEMBER
-  const int nb = which == 0 ? M.nb_nr : which == 1 ? M.nb_force : M.nb_256;
-  b_red_final(M.a.red, M.a.rcap, nb, spec, M.a.sc, which == 0 ? (const int*)&M.a.sc->pc_done : nullptr, vl);
-}
 template <typename PT>
 NDSP_MK(km_pack_density) { NDSP_MEMBER b_pack_density<PT>(M.a, M.p, vl); }
 template <typename PT>
-NDSP_MK(km_pack_force) { NDSP_MEMBER b_pack_force<PT>(M.a, M.p, vl); }
+NDSP_MK(km_pack_force) { NDSP_MEMBER b_pack_force<PT>(M.a, M.p, 1, vl); }
 template <int NDIM>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void km_nblist(const MArgs* __restrict__ ma,
                                                                                          const int* __restrict__ off,
@@ -3127,7 +3124,7 @@ __global__ __launch_bounds__(TB) void km_nr_pass(const MArgs* __restrict__ ma, c
 }
 template <int NDIM, typename PT, int PHYS, int TB>
 __global__ __launch_bounds__(TB) void km_force(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm) {
-  NDSP_MEMBER b_force<NDIM, PT, PHYS, TB>(M.a, M.p, M.gdev, vl);
+  NDSP_MEMBER b_force<NDIM, PT, PHYS, TB>(M.a, M.p, M.gdev, 1, vl);
 }
 
 static int make_tables(int ikernel, int ndim, std::vector<double>& tab, double& radkern, double& dq2) {
@@ -3191,6 +3188,10 @@ static double nexp_of(const Phys& p) {
   return 4.0 / 3.0 * M_PI * r * r * r;
 }
 
+// (33000 reals take 23 us this way and 200 with a copy command, 50000 take 250
+// and 42)
+static const size_t PIN_REALS = 40960;
+
 struct ndsp_ctx {
   int device = 0;           // HIP device current at creation (holds every buffer)
   int tb_force = 256, tb_nr = 256;  // workgroup sizes of the pair kernels (autotuned)
@@ -3220,17 +3221,18 @@ struct ndsp_ctx {
   int n;
   int ibound[3];
   double xmin[3], xmax[3];
-  double bconstmax;
   hipStream_t st = nullptr;
   KArgs a;
   double* scratch_d = nullptr;  // REORDER_W fields of n doubles for reorders
   int* scratch_i = nullptr;
   int* bsum = nullptr;
-  int* cmp_bsum = nullptr;      // block offsets of the compaction of unconverged flags
   int* list_a = nullptr;        // active lists of the h-rho passes
   int* list_b = nullptr;
   double* part = nullptr;       // reduction partials
-  double* cons_out = nullptr;
+  double* cons_out = nullptr;   // pinned host memory: the kernels write their results there
+  DScal* hs = nullptr;          // pinned host copy of the scalars
+  double* pin = nullptr;        // pinned staging of small downloads (PIN_REALS reals at most)
+  bool density_ready = false;   // the binning has just set the scalars of the h-rho iteration
   int nb_part = 0;
   Grid g;
   bool grid_valid = false;
@@ -3302,6 +3304,11 @@ static void timing_collect(ndsp_ctx* c) {
   c->nev = 0;
 }
 
+__global__ void k_zero_i(int* __restrict__ a, long long n) {
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+    a[i] = 0;
+}
+
 // nf fields of n doubles in one allocation, each on a 256-byte boundary
 static size_t field_stride(size_t n) { return (sizeof(double) * n + 255) / 256 * 256; }
 static bool alloc_fields(char** slab, double** f, int nf, size_t n) {
@@ -3315,6 +3322,18 @@ static bool alloc_fields(char** slab, double** f, int nf, size_t n) {
 
 static inline unsigned nblk(long long n, int bs = BS) { return (unsigned)((n + bs - 1) / bs); }
 
+// blocks of k_binstats: four particles a thread up to 1024 blocks (every block
+// publishes its partials to the other XCDs before the last one folds them:
+// 512^2 takes 27 us with 256 blocks and 41 with 1024, 128^3 111 with 256 and 75
+// with 1024)
+static inline unsigned bin_blocks(long long n) { return std::min(1024u, nblk(n, 4 * BS)); }
+
+// threads of the fold over n/tb blocks (the smallest block that keeps eight
+// loads a thread in flight: the fold after a pass takes 5.6 us at 800 particles
+// and 7.0 with 1024 threads; at 128^3 it takes 16.5 us with 1024, where the
+// reductions alone took 17.2 with 256)
+static inline unsigned fold_threads(long long n, int tb) { return nblk(n, tb) > 1024 ? FOLD_B : BS; }
+
 template <typename F>
 static int dispatch_ndim(int ndim, F&& f) {
   if (ndim == 1) return f(std::integral_constant<int, 1>());
@@ -3323,8 +3342,9 @@ static int dispatch_ndim(int ndim, F&& f) {
 }
 
 static int sync_scalars(ndsp_ctx* c, DScal& h) {
-  HIPCHK(hipMemcpyAsync(&h, c->a.sc, sizeof(DScal), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipMemcpyAsync(c->hs, c->a.sc, sizeof(DScal), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
+  h = *c->hs;
   return 0;
 }
 
@@ -3362,10 +3382,14 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
   if (c->a.cfill) hipFree(c->a.cfill);
   if (c->bsum) hipFree(c->bsum);
   if (c->a.cellr) hipFree(c->a.cellr);
-  c->a.cstart = c->a.cfill = c->bsum = nullptr;
+  if (c->a.cpart) hipFree(c->a.cpart);
+  c->a.cstart = c->a.cfill = c->a.cpart = c->bsum = nullptr;
   c->a.cellr = nullptr;
   HIPCHK(hipMalloc(&c->a.cstart, sizeof(int) * cap));
   HIPCHK(hipMalloc(&c->a.cfill, sizeof(int) * cap));
+  HIPCHK(hipMalloc(&c->a.cpart, sizeof(int) * cap));
+  // every binning finds the counts zero and leaves them so
+  hipLaunchKernelGGL(k_zero_i, dim3(1024), dim3(BS), 0, c->st, c->a.cfill, cap);
   HIPCHK(hipMalloc(&c->bsum, sizeof(int) * (cap / (BS * 4) + 2)));
   if (c->p.use_list) HIPCHK(hipMalloc(&c->a.cellr, sizeof(float) * cap));
   c->cap_bits = bits;
@@ -3402,39 +3426,30 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
   KArgs& a = c->a;
   const int n = c->n;
   if (!c->ireal_set) return set_err(NDSP_ERR_BAD_ARG, "fixed particles need their partners: call ndsp_set_ireal");
-  hipLaunchKernelGGL(k_fill_i, dim3(1), dim3(64), 0, c->st, &a.sc->err, 1, 0);
   {
-    TScope t(c, "boundary");
-    hipLaunchKernelGGL(k_boundary, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, c->g, in_step);
-  }
-  {
+    // wrap, statistics, grid and the iteration's scalars in one launch; the
+    // first binning sizes the key space from the statistics in between
     TScope t(c, "binstats");
-    hipLaunchKernelGGL(k_binstats, dim3(c->nb_part), dim3(BS), 0, c->st, a, c->p.ndim, c->part);
-    hipLaunchKernelGGL(k_binstats_final, dim3(1), dim3(BS), 0, c->st, a.sc, c->part, c->nb_part);
-  }
-  if (c->cap_bits == 0) {
-    if (c->capturing) return set_err(NDSP_ERR_BAD_ARG, "capture before the first binning");
-    DScal hs;
-    if (int e = sync_scalars(c, hs)) return e;
-    if (int e = size_key_space(c, hs, 1)) return e;
+    const bool sized = c->cap_bits > 0;
+    hipLaunchKernelGGL(k_binstats, dim3(bin_blocks(n)), dim3(BS), 0, c->st, a, c->p, c->g,
+                       sized ? c->gdev : (Grid*)nullptr, in_step, c->cap_bits, c->part);
+    if (!sized) {
+      if (c->capturing) return set_err(NDSP_ERR_BAD_ARG, "capture before the first binning");
+      DScal hs;
+      if (int e = sync_scalars(c, hs)) return e;
+      if (int e = size_key_space(c, hs, 1)) return e;
+      hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(64), 0, c->st, a.sc, c->gdev, c->g, c->p, c->cap_bits, n);
+    }
+    c->density_ready = true;
   }
   const long long cap = (1LL << c->cap_bits) + 1;
   const unsigned cap_blocks = (unsigned)std::min<long long>(nblk(cap), 1 << 20);
   {
     TScope t(c, "cellsort");
-    hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(64), 0, c->st, a.sc, c->gdev, c->g, c->p, c->cap_bits);
-    hipLaunchKernelGGL(k_fill_cells, dim3(std::min(cap_blocks, 4096u)), dim3(BS), 0, c->st, a.cfill,
-                       (const Grid*)c->gdev);
-    hipLaunchKernelGGL(k_cellid, dim3(nblk(n)), dim3(BS), 0, c->st, a, (const Grid*)c->gdev);
     const unsigned nbs = (unsigned)((cap + BS * 4 - 1) / (BS * 4));
-    hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(BS), 0, c->st, (const int*)a.cfill, a.cstart, c->bsum,
-                       (const Grid*)c->gdev);
-    hipLaunchKernelGGL(k_scan_bsum, dim3(1), dim3(BS), 0, c->st, c->bsum, (const Grid*)c->gdev, (int*)nullptr);
-    hipLaunchKernelGGL(k_scan_add, dim3(cap_blocks), dim3(BS), 0, c->st, a, (const int*)c->bsum,
-                       (const Grid*)c->gdev);
-    hipLaunchKernelGGL(k_fill_cells, dim3(std::min(cap_blocks, 4096u)), dim3(BS), 0, c->st, a.cfill,
-                       (const Grid*)c->gdev);
-    hipLaunchKernelGGL(k_scatter, dim3(nblk(n)), dim3(BS), 0, c->st, a);
+    hipLaunchKernelGGL(k_cellid, dim3(nblk(n)), dim3(BS), 0, c->st, a, (const Grid*)c->gdev);
+    hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(BS), 0, c->st, a, c->bsum, (const Grid*)c->gdev);
+    hipLaunchKernelGGL(k_scatter, dim3(nblk(n)), dim3(BS), 0, c->st, a, (const int*)c->bsum, (const Grid*)c->gdev);
     hipLaunchKernelGGL(k_cellsort_wave, dim3(cap_blocks), dim3(BS), 0, c->st, a, (const Grid*)c->gdev);
   }
   {
@@ -3459,6 +3474,18 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
 
 // K pass launches of the h-rho iteration; each reads its parameters from the
 // device-side control and does nothing once the iteration has finished
+static RedSpec spec_pass() {
+  return red_spec({RED_Q(RED_MAX, RED_F64, stressmax), RED_Q(RED_MAX, RED_F64, hmax_nr),
+                   RED_Q(RED_MAX, RED_I32, itsmax), RED_Q(RED_MIN, RED_I32, nmin), RED_Q(RED_MAX, RED_I32, nmax),
+                   RED_Q(RED_SUM, RED_U64, pairs_density), RED_Q(RED_SUM, RED_U64, ncalc_total)});
+}
+static RedSpec spec_force() {
+  return red_spec({RED_Q(RED_MAX, RED_F64, vsigmax), RED_Q(RED_MIN, RED_F64, dtcourant),
+                   RED_Q(RED_SUM, RED_U64, pairs_force)});
+}
+static RedSpec spec_dt() {
+  return red_spec({RED_Q(RED_MAX, RED_F64, fhmax), RED_Q(RED_MIN, RED_F64, dtdrag)});
+}
 static void launch_passes(ndsp_ctx* c, int K) {
   KArgs& a = c->a;
   const int n = c->n;
@@ -3476,22 +3503,9 @@ static void launch_passes(ndsp_ctx* c, int K) {
                          c->list_a, c->list_b);
       return 0;
     });
-    {
-      const unsigned nb = (unsigned)((n + BS * CMP_ITEMS - 1) / (BS * CMP_ITEMS));
-      hipLaunchKernelGGL(k_cmp_count, dim3(nb), dim3(BS), 0, c->st, (const int*)a.nrflag, n, c->cmp_bsum);
-      hipLaunchKernelGGL(k_cmp_scan, dim3(1), dim3(BS), 0, c->st, c->cmp_bsum, (int)nb, a.sc);
-      hipLaunchKernelGGL(k_cmp_scatter, dim3(nb), dim3(BS), 0, c->st, a.nrflag, n, (const int*)c->cmp_bsum,
-                         (const DScal*)a.sc, c->list_a, c->list_b);
-    }
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(BS), 0, c->st, (const double*)a.red, a.rcap, (int)nblk(n, c->tb_nr),
-                       red_spec({RED_Q(RED_MAX, RED_F64, stressmax), RED_Q(RED_MAX, RED_F64, hmax_nr),
-                                 RED_Q(RED_MAX, RED_I32, itsmax), RED_Q(RED_MIN, RED_I32, nmin),
-                                 RED_Q(RED_MAX, RED_I32, nmax), RED_Q(RED_SUM, RED_U64, pairs_density),
-                                 RED_Q(RED_SUM, RED_U64, ncalc_total)}),
-                       a.sc, (const int*)&a.sc->pc_done);
-    hipLaunchKernelGGL(k_pass_ctl, dim3(1), dim3(64), 0, c->st, a.sc, n, reflect ? 1 : 0, c->p.maxits);
-    hipLaunchKernelGGL(k_hmax, dim3(std::min(1024u, nblk(n))), dim3(BS), 0, c->st, a, a.sc);
-    hipLaunchKernelGGL(k_refresh_hinv, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
+    hipLaunchKernelGGL(k_pass_fold, dim3(1), dim3(fold_threads(n, c->tb_nr)), 0, c->st, a, spec_pass(), (int)nblk(n, c->tb_nr), c->tb_nr,
+                       reflect ? 1 : 0, c->p.maxits, q == K - 1 ? c->hs : (DScal*)nullptr);
+    hipLaunchKernelGGL(k_pass_next, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, c->tb_nr, c->list_a, c->list_b);
   }
 }
 
@@ -3503,7 +3517,8 @@ static int pass_chunk(const ndsp_ctx* c) { return c->reflect ? 4 : 3; }
 
 static int do_density(ndsp_ctx* c) {
   KArgs& a = c->a;
-  hipLaunchKernelGGL(k_init_density_scalars, dim3(1), dim3(1), 0, c->st, a.sc, c->bconstmax, c->n);
+  if (!c->density_ready) hipLaunchKernelGGL(k_init_density_scalars, dim3(1), dim3(1), 0, c->st, a.sc, c->p, c->n);
+  c->density_ready = false;
   TScope t(c, "density");
   launch_passes(c, pass_chunk(c));
   HIPCHK(hipGetLastError());
@@ -3513,9 +3528,9 @@ static int do_density(ndsp_ctx* c) {
 // until the device control reports the iteration finished: more passes
 static int density_finish(ndsp_ctx* c) {
   for (int guard = 0; guard < 1000; guard++) {
-    DScal hs;
-    if (int e = sync_scalars(c, hs)) return e;
-    if (hs.pc_done) return 0;
+    // (the last fold of every chunk of passes writes the scalars to the host)
+    HIPCHK(hipStreamSynchronize(c->st));
+    if (c->hs->pc_done) return 0;
     TScope t(c, "density");
     launch_passes(c, pass_chunk(c));
     HIPCHK(hipGetLastError());
@@ -3523,26 +3538,26 @@ static int density_finish(ndsp_ctx* c) {
   return set_err(NDSP_ERR_NOT_CONVERGED, "h-rho iteration did not finish");
 }
 
-// with_correct: the step's corrector runs in the finalize launch (each
-// particle's final rates, then its corrected state)
-static int do_rates(ndsp_ctx* c, bool with_correct = false) {
+// with_correct: the step's corrector and boundary run in the finalize launch,
+// its end in the last fold; guard: kernels hold back until the h-rho iteration
+// has finished (recorded steps)
+static int do_rates(ndsp_ctx* c, bool with_correct = false, int guard = 0) {
   KArgs& a = c->a;
   const int n = c->n;
-  if (c->p.fixed_on) hipLaunchKernelGGL(k_fixed_copy, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
+  if (c->p.fixed_on) hipLaunchKernelGGL(k_fixed_copy, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, guard);
   {
     TScope t(c, "pack_force");
     if (c->prec == NDSP_PREC_FP64)
-      hipLaunchKernelGGL(k_pack_force<double>, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
+      hipLaunchKernelGGL(k_pack_force<double>, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, guard);
     else
-      hipLaunchKernelGGL(k_pack_force<float>, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
+      hipLaunchKernelGGL(k_pack_force<float>, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, guard);
   }
-  hipLaunchKernelGGL(k_init_force_scalars, dim3(1), dim3(1), 0, c->st, a.sc);
   {
     TScope t(c, "force");
     dispatch_ndim(c->p.ndim, [&](auto nd) {
       constexpr int ND = decltype(nd)::value;
       const int phys = c->p.imhd ? 1 : c->p.idust ? 2 : 0;
-      void (*kern)(KArgs, Phys, const Grid* __restrict__);
+      void (*kern)(KArgs, Phys, const Grid* __restrict__, int);
       const bool small = c->tb_force == 64;
       if (c->prec == NDSP_PREC_FP64) {
         if (small) kern = phys == 1 ? k_force<ND, double, 1, 64> : phys == 2 ? k_force<ND, double, 2, 64> : k_force<ND, double, 0, 64>;
@@ -3551,25 +3566,28 @@ static int do_rates(ndsp_ctx* c, bool with_correct = false) {
         if (small) kern = phys == 1 ? k_force<ND, float, 1, 64> : phys == 2 ? k_force<ND, float, 2, 64> : k_force<ND, float, 0, 64>;
         else kern = phys == 1 ? k_force<ND, float, 1, 256> : phys == 2 ? k_force<ND, float, 2, 256> : k_force<ND, float, 0, 256>;
       }
-      hipLaunchKernelGGL(kern, dim3(nblk(n, c->tb_force)), dim3(c->tb_force), 0, c->st, a, c->p, (const Grid*)c->gdev);
+      hipLaunchKernelGGL(kern, dim3(nblk(n, c->tb_force)), dim3(c->tb_force), 0, c->st, a, c->p, (const Grid*)c->gdev,
+                         guard);
       return 0;
     });
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(BS), 0, c->st, (const double*)a.red, a.rcap, (int)nblk(n, c->tb_force),
-                       red_spec({RED_Q(RED_MAX, RED_F64, vsigmax), RED_Q(RED_MIN, RED_F64, dtcourant),
-                                 RED_Q(RED_SUM, RED_U64, pairs_force)}),
-                       a.sc, (const int*)nullptr);
+    hipLaunchKernelGGL(k_force_fold, dim3(1), dim3(fold_threads(n, c->tb_force)), 0, c->st, a, spec_force(), (int)nblk(n, c->tb_force), guard);
   }
   {
     TScope t(c, "finalize");
-    if (with_correct) hipLaunchKernelGGL(k_finalize_correct, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
+    if (with_correct) hipLaunchKernelGGL(k_finalize_correct, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, c->g, guard);
     else hipLaunchKernelGGL(k_finalize, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p);
-    hipLaunchKernelGGL(k_red_final, dim3(1), dim3(BS), 0, c->st, (const double*)a.red, a.rcap, (int)nblk(n),
-                       red_spec({RED_Q(RED_MAX, RED_F64, fhmax), RED_Q(RED_MIN, RED_F64, dtdrag)}), a.sc,
-                       (const int*)nullptr);
-    hipLaunchKernelGGL(k_dt, dim3(1), dim3(1), 0, c->st, a.sc, c->p);
+    hipLaunchKernelGGL(k_dt_fold, dim3(1), dim3(fold_threads(n, BS)), 0, c->st, a, c->p, spec_dt(), (int)nblk(n), guard,
+                       with_correct ? 1 : 0, c->hs);
   }
   HIPCHK(hipGetLastError());
   c->have_rates = true;
+  return 0;
+}
+// waits for the scalars that the last fold of a density chunk or of the rates
+// wrote to the host
+static int wait_scalars(ndsp_ctx* c, DScal& h) {
+  HIPCHK(hipStreamSynchronize(c->st));
+  h = *c->hs;
   return 0;
 }
 
@@ -3761,7 +3779,7 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   c->p = p;
   c->prec = precision;
   c->n = (int)npart;
-  c->bconstmax = std::max(std::max(dopt[20], dopt[21]), dopt[22]);
+  c->p.Bconstmax = std::max(std::max(dopt[20], dopt[21]), dopt[22]);
   for (int d = 0; d < 3; d++) {
     c->ibound[d] = d < p.ndim ? ib[d] : 0;
     c->xmin[d] = dopt[13 + d];
@@ -3797,7 +3815,8 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   ok &= hipMalloc(&c->list_a, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&c->list_b, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.nrflag, sizeof(int) * n) == hipSuccess;
-  ok &= hipMalloc(&c->cmp_bsum, sizeof(int) * ((size_t)n / (BS * CMP_ITEMS) + 2)) == hipSuccess;
+  ok &= hipMalloc(&a.nrcnt, sizeof(int) * (size_t)nblk(n, 64)) == hipSuccess;
+  a.rank = c->list_a;  // free during a binning: the h-rho passes come after it
   if (ok) ok &= hipMemset(a.nrflag, 0, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.P4, sizeof(double4) * n) == hipSuccess;
   ok &= hipMalloc(&a.dxb, sizeof(double) * n) == hipSuccess;
@@ -3831,7 +3850,9 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   ok &= hipMalloc(&tabd, sizeof(double) * tab.size()) == hipSuccess;
   c->nb_part = 1024;
   ok &= hipMalloc(&c->part, sizeof(double) * 32 * c->nb_part) == hipSuccess;
-  ok &= hipMalloc(&c->cons_out, sizeof(double) * 32) == hipSuccess;
+  ok &= hipHostMalloc((void**)&c->cons_out, sizeof(double) * 32, hipHostMallocDefault) == hipSuccess;
+  ok &= hipHostMalloc((void**)&c->hs, sizeof(DScal), hipHostMallocDefault) == hipSuccess;
+  ok &= hipHostMalloc((void**)&c->pin, sizeof(double) * std::min<size_t>(3 * n, PIN_REALS), hipHostMallocDefault) == hipSuccess;
   ok &= hipMalloc((void**)&c->gdev, sizeof(Grid)) == hipSuccess;
   if (!ok) return cleanup_fail(set_err(NDSP_ERR_ALLOC, "hipMalloc buffers"));
   hipMemcpy(c->gdev, &c->g, sizeof(Grid), hipMemcpyHostToDevice);
@@ -3860,9 +3881,12 @@ int ndsp_destroy(ndsp_ctx* c) {
   KArgs& a = c->a;
   void* ptrs[] = {c->fields, c->fields_alt, c->scratch_d, c->scratch_i, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
                   a.DR, a.FR, a.GF, a.sc, (void*)a.tabf, (void*)a.tabd,
-                  c->part, c->cons_out, a.cstart, a.cfill, a.cellr, c->bsum, c->list_a, c->list_b, a.nrflag, c->cmp_bsum,
+                  c->part, a.cstart, a.cfill, a.cpart, a.cellr, c->bsum, c->list_a, c->list_b, a.nrflag, a.nrcnt,
                   a.nbl, a.nbc, a.nbx, a.hcap, a.red, c->gdev};
   for (void* q : ptrs) if (q) hipFree(q);
+  if (c->cons_out) hipHostFree(c->cons_out);
+  if (c->hs) hipHostFree(c->hs);
+  if (c->pin) hipHostFree(c->pin);
   if (c->graph_a) hipGraphExecDestroy(c->graph_a);
   if (c->graph_b) hipGraphExecDestroy(c->graph_b);
   if (c->alt_graph_a) hipGraphExecDestroy(c->alt_graph_a);
@@ -3977,10 +4001,16 @@ int ndsp_download(ndsp_ctx* c, const char* name, double* out, int32_t* width) {
     }
   }
   if (w) {
-    hipLaunchKernelGGL(k_to_caller, dim3(nblk(n)), dim3(BS), 0, c->st, cf, (const int*)c->a.uid, c->scratch_d, w, n);
+    // small fields straight into pinned host memory (no copy command), larger
+    // ones through the scratch (800 particles: 15 us instead of 29)
+    const size_t len = (size_t)n * w;
+    const bool direct = len <= PIN_REALS;
+    hipLaunchKernelGGL(k_to_caller, dim3(nblk(n)), dim3(BS), 0, c->st, cf, (const int*)c->a.slot_of,
+                       direct ? c->pin : c->scratch_d, w, n);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(out, c->scratch_d, sizeof(double) * (size_t)n * w, hipMemcpyDeviceToHost, c->st));
+    if (!direct) HIPCHK(hipMemcpyAsync(out, c->scratch_d, sizeof(double) * len, hipMemcpyDeviceToHost, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
+    if (direct) memcpy(out, c->pin, sizeof(double) * len);
     if (width) *width = w;
     return 0;
   }
@@ -3998,7 +4028,7 @@ int ndsp_iterate_density(ndsp_ctx* c, ndsp_stats* stats) {
   if (int e = do_density(c)) return e;
   if (int e = density_finish(c)) return e;
   DScal hs;
-  if (int e = sync_scalars(c, hs)) return e;
+  if (int e = wait_scalars(c, hs)) return e;
   timing_collect(c);
   fill_outputs(c, hs, stats, nullptr);
   return check_err(c, hs);
@@ -4009,7 +4039,7 @@ int ndsp_get_rates(ndsp_ctx* c, ndsp_dt* dt) {
   if (!c->grid_valid) return set_err(NDSP_ERR_BAD_ARG, "get_rates: call set_linklist and iterate_density first");
   if (int e = do_rates(c)) return e;
   DScal hs;
-  if (int e = sync_scalars(c, hs)) return e;
+  if (int e = wait_scalars(c, hs)) return e;
   timing_collect(c);
   fill_outputs(c, hs, nullptr, dt);
   return check_err(c, hs);
@@ -4022,7 +4052,7 @@ int ndsp_derivs(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dt) {
   if (int e = density_finish(c)) return e;
   if (int e = do_rates(c)) return e;
   DScal hs;
-  if (int e = sync_scalars(c, hs)) return e;
+  if (int e = wait_scalars(c, hs)) return e;
   timing_collect(c);
   fill_outputs(c, hs, stats, dt);
   return check_err(c, hs);
@@ -4083,16 +4113,12 @@ static int step_part_a(ndsp_ctx* c) {
 // wrap, next dt; online training of the h predictor when enabled.
 static int step_part_b(ndsp_ctx* c) {
   MlpState& ml = c->mlp;
+  const int guard = c->capturing ? 1 : 0;
   if (ml.enabled) {
     TScope t(c, "mlp_target");
     hipLaunchKernelGGL(k_mlp_target, dim3(nblk(c->n)), dim3(BS), 0, c->st, c->a, ml.X);
   }
-  if (int e = do_rates(c, true)) return e;
-  {
-    TScope t(c, "correct");
-    hipLaunchKernelGGL(k_boundary, dim3(nblk(c->n)), dim3(BS), 0, c->st, c->a, c->p, c->g, 1);
-    hipLaunchKernelGGL(k_step_end, dim3(1), dim3(64), 0, c->st, c->a.sc);
-  }
+  if (int e = do_rates(c, true, guard)) return e;
   if (ml.enabled && ml.train) {
     TScope t(c, "mlp_train");
     // online training on this step's (features, converged h): Adam steps on
@@ -4154,16 +4180,23 @@ int ndsp_step(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dtout) {
       if (int e = capture(c, c->graph_b, step_part_b)) return e;
       c->graph_valid = true;
     }
+    // both halves at once: the second holds back while the iteration is
+    // unfinished, and is then launched again once the host has finished it (one
+    // wait a step instead of two)
     HIPCHK(hipGraphLaunch(c->graph_a, c->st));
-    if (int e = density_finish(c)) return e;
     HIPCHK(hipGraphLaunch(c->graph_b, c->st));
+    HIPCHK(hipStreamSynchronize(c->st));
+    if (!c->hs->pc_done) {
+      if (int e = density_finish(c)) return e;
+      HIPCHK(hipGraphLaunch(c->graph_b, c->st));
+    }
   } else {
     if (int e = step_part_a(c)) return e;
     if (int e = density_finish(c)) return e;
     if (int e = step_part_b(c)) return e;
   }
   DScal hs;
-  if (int e = sync_scalars(c, hs)) return e;
+  if (int e = wait_scalars(c, hs)) return e;
   timing_collect(c);
   c->time = hs.time;
   c->dt = hs.dt_cur;
@@ -4204,7 +4237,6 @@ struct ndsp_batch {
   hipGraphExec_t ga = nullptr, gb = nullptr;
   bool valid = false;
   DScal* hs = nullptr;               // pinned host copies of every member's scalars
-  DScal* dsc = nullptr;              // the members' scalars gathered on the device
   std::vector<int> caps;             // members' key-space sizes at recording
   std::vector<int> nbcaps;           // members' list capacities at recording
   std::vector<hipStream_t> gst;      // streams of the groups after the first (recording only)
@@ -4270,7 +4302,6 @@ static int batch_build(ndsp_batch* b) {
       MArgs& M = ma[q];
       memset(&M, 0, sizeof(M));
       M.a = c->a;
-      M.a.nrflag = nullptr;  // batched passes append their unconverged particles
       M.p = c->p;
       M.gdev = c->gdev;
       M.box = c->g;
@@ -4278,11 +4309,10 @@ static int batch_build(ndsp_batch* b) {
       M.bsum = c->bsum;
       M.list_a = c->list_a;
       M.list_b = c->list_b;
-      M.out = b->dsc + g.mem[q];
-      M.bconstmax = c->bconstmax;
+      M.out = b->hs + g.mem[q];
       M.cap_bits = c->cap_bits;
       M.reflect = c->reflect;
-      M.nbp = (int)std::min<unsigned>(c->nb_part, nblk(n));
+      M.nbp = (int)bin_blocks(n);
       M.nb_nr = (int)nblk(n, b->tb);
       M.nb_force = (int)nblk(n, b->tb);
       M.nb_256 = (int)nblk(n);
@@ -4338,17 +4368,9 @@ static int batch_part_a(ndsp_batch* b) {
     const hipStream_t bst = batch_group_stream(b, gi);
     BLAUNCH(km_predict, g, BGroup::S_256, BS);
     if (g.fixed) BLAUNCH(km_predict_fixed, g, BGroup::S_256, BS);
-    BLAUNCH(km_err_reset, g, BGroup::S_ONE, 64);
-    BLAUNCH(km_boundary_step, g, BGroup::S_256, BS);
     BLAUNCH(km_binstats, g, BGroup::S_BIN, BS);
-    BLAUNCH(km_binstats_final, g, BGroup::S_ONE, BS);
-    BLAUNCH(km_grid_setup, g, BGroup::S_ONE, 64);
-    BLAUNCH(km_fill_cells, g, BGroup::S_FILL, BS);
     BLAUNCH(km_cellid, g, BGroup::S_256, BS);
     BLAUNCH(km_scan_local, g, BGroup::S_SCAN, BS);
-    BLAUNCH(km_scan_bsum, g, BGroup::S_ONE, BS);
-    BLAUNCH(km_scan_add, g, BGroup::S_CAP, BS);
-    BLAUNCH(km_fill_cells, g, BGroup::S_FILL, BS);
     BLAUNCH(km_scatter, g, BGroup::S_256, BS);
     BLAUNCH(km_cellsort, g, BGroup::S_CAP, BS);
     if (fp64) BLAUNCH(km_pack_density<double>, g, BGroup::S_256, BS);
@@ -4360,11 +4382,6 @@ static int batch_part_a(ndsp_batch* b) {
         return 0;
       });
     }
-    BLAUNCH(km_init_density, g, BGroup::S_ONE, 64);
-    const RedSpec spec = red_spec({RED_Q(RED_MAX, RED_F64, stressmax), RED_Q(RED_MAX, RED_F64, hmax_nr),
-                                   RED_Q(RED_MAX, RED_I32, itsmax), RED_Q(RED_MIN, RED_I32, nmin),
-                                   RED_Q(RED_MAX, RED_I32, nmax), RED_Q(RED_SUM, RED_U64, pairs_density),
-                                   RED_Q(RED_SUM, RED_U64, ncalc_total)});
     const int K = g.reflect ? 4 : 3;
     for (int q = 0; q < K; q++) {
       dispatch_ndim(g.ndim, [&](auto nd) {
@@ -4378,15 +4395,12 @@ static int batch_part_a(ndsp_batch* b) {
         }
         return 0;
       });
-      BLAUNCH(km_red_final, g, BGroup::S_ONE, BS, spec, 0);
-      BLAUNCH(km_pass_ctl, g, BGroup::S_ONE, 64);
-      BLAUNCH(km_hmax, g, BGroup::S_HMAX, BS);
-      BLAUNCH(km_refresh_hinv, g, BGroup::S_256, BS);
+      BLAUNCH(km_pass_fold, g, BGroup::S_ONE, BS, spec_pass(), b->tb, q == K - 1 ? 1 : 0);
+      if (b->tb == 64) BLAUNCH(km_pass_next_64, g, BGroup::S_256, BS);
+      else BLAUNCH(km_pass_next_256, g, BGroup::S_256, BS);
     }
-    BLAUNCH(km_gather_scalars, g, BGroup::S_ONE, 64);
   }
   if (int e = batch_join(b)) return e;
-  HIPCHK(hipMemcpyAsync(b->hs, b->dsc, sizeof(DScal) * b->sims.size(), hipMemcpyDeviceToHost, b->st));
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -4401,7 +4415,6 @@ static int batch_part_b(ndsp_batch* b) {
     if (g.fixed) BLAUNCH(km_fixed_copy, g, BGroup::S_256, BS);
     if (fp64) BLAUNCH(km_pack_force<double>, g, BGroup::S_256, BS);
     else BLAUNCH(km_pack_force<float>, g, BGroup::S_256, BS);
-    BLAUNCH(km_init_force, g, BGroup::S_ONE, 64);
     dispatch_ndim(g.ndim, [&](auto nd) {
       constexpr int ND = decltype(nd)::value;
 #define NDSP_FORCE_B(PTT, TBB)                                                                        \
@@ -4415,20 +4428,11 @@ static int batch_part_b(ndsp_batch* b) {
 #undef NDSP_FORCE_B
       return 0;
     });
-    BLAUNCH(km_red_final, g, BGroup::S_ONE, BS,
-            red_spec({RED_Q(RED_MAX, RED_F64, vsigmax), RED_Q(RED_MIN, RED_F64, dtcourant),
-                      RED_Q(RED_SUM, RED_U64, pairs_force)}), 1);
-    BLAUNCH(km_finalize, g, BGroup::S_256, BS);
-    BLAUNCH(km_red_final, g, BGroup::S_ONE, BS,
-            red_spec({RED_Q(RED_MAX, RED_F64, fhmax), RED_Q(RED_MIN, RED_F64, dtdrag)}), 2);
-    BLAUNCH(km_dt, g, BGroup::S_ONE, 64);
-    BLAUNCH(km_correct, g, BGroup::S_256, BS);
-    BLAUNCH(km_boundary_step, g, BGroup::S_256, BS);
-    BLAUNCH(km_step_end, g, BGroup::S_ONE, 64);
-    BLAUNCH(km_gather_scalars, g, BGroup::S_ONE, 64);
+    BLAUNCH(km_force_fold, g, BGroup::S_ONE, BS, spec_force());
+    BLAUNCH(km_finalize_correct, g, BGroup::S_256, BS);
+    BLAUNCH(km_dt_fold, g, BGroup::S_ONE, BS, spec_dt());
   }
   if (int e = batch_join(b)) return e;
-  HIPCHK(hipMemcpyAsync(b->hs, b->dsc, sizeof(DScal) * b->sims.size(), hipMemcpyDeviceToHost, b->st));
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -4494,7 +4498,6 @@ int ndsp_batch_create(ndsp_ctx* const* ctxs, int32_t nsim, ndsp_batch** out) {
   b->prec = ctxs[0]->prec;
   bool ok = hipStreamCreate(&b->st) == hipSuccess;
   ok &= hipHostMalloc((void**)&b->hs, sizeof(DScal) * nsim, hipHostMallocDefault) == hipSuccess;
-  ok &= hipMalloc((void**)&b->dsc, sizeof(DScal) * nsim) == hipSuccess;
   if (!ok) {
     ndsp_batch_destroy(b);
     return set_err(NDSP_ERR_ALLOC, "batch_create: stream or scalar buffers");
@@ -4515,7 +4518,6 @@ int ndsp_batch_destroy(ndsp_batch* b) {
   }
   for (hipEvent_t ev : b->gev) hipEventDestroy(ev);
   if (b->hs) hipHostFree(b->hs);
-  if (b->dsc) hipFree(b->dsc);
   if (b->st) hipStreamDestroy(b->st);
   delete b;
   return 0;
@@ -4555,17 +4557,26 @@ int ndsp_batch_step(ndsp_batch* b, ndsp_stats* stats, ndsp_dt* dt) {
   }
   if (std::find(due.begin(), due.end(), 1) != due.end())
     if (int e = batch_reorder(b, due)) return e;
+  // both halves at once: members whose iteration needs more passes than
+  // recorded hold back in the second, which is launched again once the host
+  // has finished them (the others have ended their step and do nothing then)
   HIPCHK(hipGraphLaunch(b->ga, b->st));
+  HIPCHK(hipGraphLaunch(b->gb, b->st));
   HIPCHK(hipStreamSynchronize(b->st));
+  bool late = false;
   for (int s = 0; s < ns; s++) {
     // every member has been binned (as do_linklist leaves it): the next
     // periodic reorder is due by the member's own step count
     b->sims[s]->grid_valid = true;
-    if (!b->hs[s].pc_done)
-      if (int e = density_finish(b->sims[s])) return e;
+    if (b->hs[s].pc_done) continue;
+    late = true;
+    *b->sims[s]->hs = b->hs[s];
+    if (int e = density_finish(b->sims[s])) return e;
   }
-  HIPCHK(hipGraphLaunch(b->gb, b->st));
-  HIPCHK(hipStreamSynchronize(b->st));
+  if (late) {
+    HIPCHK(hipGraphLaunch(b->gb, b->st));
+    HIPCHK(hipStreamSynchronize(b->st));
+  }
   int first_err = 0;
   for (int s = 0; s < ns; s++) {
     ndsp_ctx* c = b->sims[s];
@@ -4651,8 +4662,8 @@ static void free_state(SavedState& S) {
 // statistics of the current positions, as the first binning would size it.
 static int ensure_key_space(ndsp_ctx* c) {
   if (c->cap_bits > 0) return 0;
-  hipLaunchKernelGGL(k_binstats, dim3(c->nb_part), dim3(BS), 0, c->st, c->a, c->p.ndim, c->part);
-  hipLaunchKernelGGL(k_binstats_final, dim3(1), dim3(BS), 0, c->st, c->a.sc, c->part, c->nb_part);
+  hipLaunchKernelGGL(k_binstats, dim3(bin_blocks(c->n)), dim3(BS), 0, c->st, c->a, c->p, c->g,
+                     (Grid*)nullptr, -1, 0, c->part);
   DScal hs;
   if (int e = sync_scalars(c, hs)) return e;
   return size_key_space(c, hs, 1);
@@ -4866,8 +4877,8 @@ int ndsp_conserved(ndsp_ctx* c, double* out) {
   hipLaunchKernelGGL(k_conserved, dim3(nb), dim3(BS), 0, c->st, c->a, c->p, c->part);
   hipLaunchKernelGGL(k_conserved_final, dim3(1), dim3(FOLD_T), 0, c->st, (const double*)c->part, nb, c->cons_out, c->n);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, c->cons_out, sizeof(double) * NCONS, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
+  memcpy(out, c->cons_out, sizeof(double) * NCONS);
   return 0;
 }
 
@@ -4880,8 +4891,8 @@ int ndsp_ev_columns(ndsp_ctx* c, double t, double dt, double* cols, int32_t* nco
   hipLaunchKernelGGL(k_ev_final, dim3(1), dim3(FOLD_T), 0, c->st, (const double*)c->part, nb, c->n, c->p, t, dt,
                      c->cons_out);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(cols, c->cons_out, sizeof(double) * nc, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
+  memcpy(cols, c->cons_out, sizeof(double) * nc);
   if (ncols) *ncols = nc;
   return 0;
 }

@@ -75,7 +75,7 @@ struct DScal {
   int list_on;         // lists built by the last binning (images one period away)
   int grid_clamped;    // cells were widened to fit the key-space capacity
   double dt_cur;       // dt of the step in progress / the next step
-  // h-rho pass control, advanced on the device by k_pass_ctl
+  // h-rho pass control, advanced on the device by pass_ctl
   int pc_nlist;        // particles in the next pass
   int pc_its;          // its of the next pass (1 = first)
   int pc_sym;          // next pass is the symmetric routine
@@ -83,6 +83,10 @@ struct DScal {
   int pc_done;         // the iteration has finished (or failed)
   int pc_relink;       // ghost extents were rebuilt before the next pass
   int pc_refresh;      // 1/h of the packed view must be refreshed
+  int pc_nprev;        // particles in the last pass
+  int phase;           // 1 from the end of a step's h-rho iteration to the end of the step
+  // blocks finished so far of the launches whose last block goes on alone
+  int bin_done, scan_done;
 };
 
 template <typename PT>
@@ -106,7 +110,10 @@ struct KArgs {
   int* cstart;        // ncell + 1
   int* cfill;         // ncell
   float* cellr;       // ncell: largest list radius of a cell's particles (null without lists)
-  int* nrflag;        // unconverged after a pass, by sorted position (compacted in order; null: appended)
+  int* rank;          // per slot: place among its cell's particles, in order of arrival
+  int* cpart;         // ncell + 1: the cells' starts within their scan block
+  int* nrflag;        // unconverged after a pass, by place in the pass's list
+  int* nrcnt;         // per tile of a pass: unconverged particles, then their offset
   int* sidx;          // sorted position -> slot
   // packed neighbour views in sorted order
   double4* P4;        // x, y, z, 1/h
@@ -132,7 +139,7 @@ struct KArgs {
   double* hcap;       // the list holds every neighbour while h <= hcap
   int maxnb;
   // per-block partials of the global reductions: quantity q of block b at
-  // red[q * rcap + b] (combined into sc by k_red_final)
+  // red[q * rcap + b] (combined into sc by red_fold)
   double* red;
   int rcap;
   DScal* sc;
