@@ -691,9 +691,11 @@ __global__ void k_pack_force(KArgs a, Phys p, int guard) {
 // coordinates (ghost arithmetic of src/ghostND_mhd.f90:180-200), flip[d] = 1
 // where the image's velocity component is reversed (image_flip), code = the image
 // kinds kx + 5 ky + 25 kz (0 for a particle seen in place).
-template <int NDIM, typename F>
+// With Q = 4 the lanes of a quad (sub 0..3) take four consecutive particles of a
+// cell at a time, and flush() follows every four.
+template <int NDIM, int Q = 1, typename F, typename FL>
 __device__ __forceinline__ void for_each_candidate(const KArgs& a, const Grid& g, const double* xi,
-                                                   double rad, F&& body) {
+                                                   double rad, int sub, F&& body, FL&& flush) {
   // rows (cy, cz) whose cells lie wholly outside the sphere are skipped and
   // each row is cut to the chord of the sphere; cell faces are widened by a
   // relative margin so that a particle binned by rounding into a cell is
@@ -733,15 +735,19 @@ __device__ __forceinline__ void for_each_candidate(const KArgs& a, const Grid& g
         image_flip(kind, fl);
         const int key = cell_key(g, sx, sy, sz);
         const int b = a.cstart[key], e = a.cstart[key + 1];
-        for (int kk = b; kk < e; kk++) {
-          const double4 pj = a.P4[kk];
-          double xj[3] = {pj.x, pj.y, pj.z};
-          bool ok = true;
-          if (code) {
-            for (int d = 0; d < NDIM; d++)
-              if (kind[d]) ok = ok && image_coord(g, d, kind[d], xj[d], a.dxb[kk], xj[d]);
+        for (int k0 = b; k0 < e; k0 += Q) {
+          const int kk = Q == 1 ? k0 : k0 + sub;
+          if (Q == 1 || kk < e) {
+            const double4 pj = a.P4[kk];
+            double xj[3] = {pj.x, pj.y, pj.z};
+            bool ok = true;
+            if (code) {
+              for (int d = 0; d < NDIM; d++)
+                if (kind[d]) ok = ok && image_coord(g, d, kind[d], xj[d], a.dxb[kk], xj[d]);
+            }
+            if (ok) body(kk, xj, fl, code);
           }
-          if (ok) body(kk, xj, fl, code);
+          flush();
         }
       }
     }
@@ -754,9 +760,25 @@ __device__ __forceinline__ void for_each_candidate(const KArgs& a, const Grid& g
 __device__ __forceinline__ unsigned list_code(int kx, int ky, int kz) {
   return (unsigned)(kx | (ky << 2) | (kz << 4));
 }
-// the code of k seen from j, given the code of j seen from k (1 <-> 2)
-__device__ __forceinline__ unsigned inverse_code(unsigned code) {
-  return ((code & 0x15u) << 1) | ((code & 0x2Au) >> 1);
+// image coordinates of a list entry's particle; a periodic image of a particle
+// exactly on the wall does not exist (src/ghostND_mhd.f90:172,180-200)
+template <int NDIM>
+__device__ __forceinline__ bool list_image(const Grid& g, int code, double* xj) {
+  bool ok = true;
+  if (code) {
+    for (int d = 0; d < NDIM; d++) {
+      const int kd = (code >> (2 * d)) & 3;
+      const double x0 = xj[d];
+      if (kd == 1) {
+        ok = ok && g.xmax[d] - x0 > 0.0;
+        xj[d] = g.xmin[d] + (x0 - g.xmax[d]);
+      } else if (kd == 2) {
+        ok = ok && x0 - g.xmin[d] > 0.0;
+        xj[d] = g.xmax[d] + (x0 - g.xmin[d]);
+      }
+    }
+  }
+  return ok;
 }
 
 // Iterates the first cnt entries of the neighbour list of sorted particle k,
@@ -793,22 +815,7 @@ __device__ __forceinline__ void for_each_listed_pf(const KArgs& a, const Grid& g
     const int code = (int)(e & 63u);
     double xj[3] = {cur.p.x, cur.p.y, cur.p.z};
     const int flip[3] = {0, 0, 0};
-    bool ok = true;
-    if (code) {
-      // ghost arithmetic of src/ghostND_mhd.f90:180-200; a periodic image
-      // of a particle exactly on the wall does not exist (:172)
-      for (int d = 0; d < NDIM; d++) {
-        const int kd = (code >> (2 * d)) & 3;
-        const double x0 = xj[d];
-        if (kd == 1) {
-          ok = ok && g.xmax[d] - x0 > 0.0;
-          xj[d] = g.xmin[d] + (x0 - g.xmax[d]);
-        } else if (kd == 2) {
-          ok = ok && x0 - g.xmin[d] > 0.0;
-          xj[d] = g.xmax[d] + (x0 - g.xmin[d]);
-        }
-      }
-    }
+    const bool ok = list_image<NDIM>(g, code, xj);
     if (ok) body(kk, cur, xj, flip, code);
     c0 = c1; c1 = c2; c2 = c3; c3 = n0; n0 = n1; n1 = n2; n2 = n3;
     if ((m & 3) == 3) {
@@ -842,14 +849,51 @@ __device__ __forceinline__ void for_each_listed_pf(const KArgs& a, const Grid& g
   }
 }
 
-// cell-scan counterpart of for_each_listed_pf (record loaded in place)
-template <int NDIM, typename LOAD, typename F>
+// The same by a quad: lane sub takes entries sub, sub + 4, ..; flush() follows
+// every four entries.  The next record is fetched while the current one is
+// processed, its entry one turn earlier.
+template <int NDIM, typename LOAD, typename F, typename FL>
+__device__ __forceinline__ void for_each_listed_quad(const KArgs& a, const Grid& g, int k, int cnt, int sub, LOAD&& load,
+                                                     F&& body, FL&& flush) {
+  if (cnt <= 0) return;
+  const unsigned* L = a.nbl + (size_t)k * a.maxnb;
+  unsigned e = L[min(sub, cnt - 1)], en = L[min(sub + 4, cnt - 1)];
+  auto cur = load((int)(e >> 7));
+  for (int m = sub; m - sub < cnt; m += 4) {
+    const auto nxt = load((int)(en >> 7));
+    const unsigned e2 = L[min(m + 8, cnt - 1)];
+    if (m < cnt) {
+      double xj[3] = {cur.p.x, cur.p.y, cur.p.z};
+      const int flip[3] = {0, 0, 0};
+      const int code = (int)(e & 63u);
+      if (list_image<NDIM>(g, code, xj)) body((int)(e >> 7), cur, xj, flip, code);
+    }
+    flush();
+    cur = nxt;
+    e = en;
+    en = e2;
+  }
+}
+
+// cell-scan counterpart of the list walks (record loaded in place)
+template <int NDIM, int Q, typename LOAD, typename F, typename FL>
 __device__ __forceinline__ void for_each_candidate_rec(const KArgs& a, const Grid& g, const double* xi,
-                                                       double rad, LOAD&& load, F&& body) {
-  for_each_candidate<NDIM>(a, g, xi, rad, [&](int kk, const double* xj, const int* flip, int code) {
+                                                       double rad, int sub, LOAD&& load, F&& body, FL&& flush) {
+  for_each_candidate<NDIM, Q>(a, g, xi, rad, sub, [&](int kk, const double* xj, const int* flip, int code) {
     const auto r = load(kk);
     body(kk, r, xj, flip, code);
-  });
+  }, flush);
+}
+
+// a kernel table from memory into LDS, 16 bytes at a time (every thread of the
+// block; the caller synchronises)
+template <typename T>
+__device__ __forceinline__ void load_table(T* dst, const T* __restrict__ src) {
+  constexpr int NV = NDSP_TAB * (int)sizeof(T) / 16;
+  const float4* s4 = (const float4*)src;
+  float4* d4 = (float4*)dst;
+#pragma unroll 4
+  for (int t = threadIdx.x; t < NV; t += blockDim.x) d4[t] = s4[t];
 }
 
 // Neighbour lists (periodic or open domains).  Entry m of sorted particle k
@@ -1506,7 +1550,7 @@ __device__ __forceinline__ void nr_update(const Phys& p, double hh, double hin, 
   r.dhdrho = dhdrhoi;
 }
 
-template <int NDIM, typename PT, bool DUST, int TB>
+template <int NDIM, typename PT, bool DUST, int TB, int Q>
 __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restrict__ gp, int* __restrict__ list_a,
                                                 int* __restrict__ list_b, VL vl) {
   // pass parameters from the device-side control (pass_ctl): pass its0
@@ -1519,22 +1563,22 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
   // a workgroup with no particle of this pass skips loading the tables (a
   // later pass holds only the particles still iterating); it still writes
   // its neutral reduction partials, which the final fold reads
-  const int tile = xcd_tile_n(vl, (nlist + (int)blockDim.x - 1) / (int)blockDim.x);
-  const bool idle = tile * (int)blockDim.x >= nlist;
-  __shared__ PT tw[NDSP_IKERN + 1];
-  __shared__ PT tg[NDSP_IKERN + 1];
-  __shared__ PT tgg[NDSP_IKERN + 1];
+  constexpr int PB = TB / Q;  // particles of a workgroup
+  const int tile = xcd_tile_n(vl, (nlist + PB - 1) / PB);
+  const bool idle = tile * PB >= nlist;
+  __shared__ __align__(16) PT tw[NDSP_TAB];
+  __shared__ __align__(16) PT tg[NDSP_TAB];
+  __shared__ __align__(16) PT tgg[NDSP_TAB];
   if (!idle) {
     const PT* src = sizeof(PT) == 4 ? (const PT*)a.tabf : (const PT*)a.tabd;
-    for (int t = threadIdx.x; t <= NDSP_IKERN; t += blockDim.x) {
-      tw[t] = src[t];
-      tg[t] = src[NDSP_IKERN + 1 + t];
-      tgg[t] = src[2 * (NDSP_IKERN + 1) + t];
-    }
+    load_table(tw, src);
+    load_table(tg, src + NDSP_TAB);
+    load_table(tgg, src + 2 * NDSP_TAB);
   }
   __syncthreads();
   const Grid g = *gp;
-  const int tid = tile * (int)blockDim.x + (int)threadIdx.x;
+  const int tid = tile * PB + (int)threadIdx.x / Q;
+  const int sub = (int)threadIdx.x % Q;  // the lane's place among the particle's
   const bool active = tid < nlist;
   bool unconverged = false;
   const int k = active ? (list ? list[tid] : tid) : 0;
@@ -1593,7 +1637,7 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
       const PT hfacwabi = pown_t<NDIM>(hi1p);
       const PT hfacgrkerni = hfacwabi * hi1p;
       const PT hi1s = hi1p * hi1p;
-      Acc<PT> rho, drhodt, gradh, ggh, rhog, rhod;
+      PSum<PT, Q> rho, drhodt, gradh, ggh, rhog, rhod;
       rho.zero(); drhodt.zero(); gradh.zero(); ggh.zero(); rhog.zero(); rhod.zero();
       int nsym = 0, ngat = 0;
       const double rad = p.radkern * (symp ? fmax(h, hmaxc) : h);
@@ -1640,10 +1684,36 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
           drhodt.add(mj * dvdotr * grkerni);
         }
       };
-      if (uselist) for_each_listed_pf<NDIM, 1>(a, g, k, nlisted, loadj, body);
-      else for_each_candidate_rec<NDIM>(a, g, xi, rad, loadj, body);
+      double s0 = 0.0, s1 = 0.0;  // Q = 4: lane j's sums (quantity j of each four)
+      auto flush = [&] {
+        if constexpr (Q == 4) {
+          quad_fold4(sub, rho.t, gradh.t, ggh.t, drhodt.t, s0);
+          rho.zero(); gradh.zero(); ggh.zero(); drhodt.zero();
+          if (dust) {
+            quad_fold4(sub, rhog.t, rhod.t, PT(0), PT(0), s1);
+            rhog.zero(); rhod.zero();
+          }
+        }
+      };
+      if (!uselist) for_each_candidate_rec<NDIM, Q>(a, g, xi, rad, sub, loadj, body, flush);
+      else if constexpr (Q == 4) for_each_listed_quad<NDIM>(a, g, k, nlisted, sub, loadj, body, flush);
+      else for_each_listed_pf<NDIM, 1>(a, g, k, nlisted, loadj, body);
       npairs += (unsigned long long)ngat;
       nn = symp ? nsym : ngat;
+      double sum[6];
+      if constexpr (Q == 4) {
+        nn += quad_move<QUAD_XOR1>(nn);
+        nn += quad_move<QUAD_XOR2>(nn);
+        sum[0] = quad_lane<0>(s0);
+        sum[1] = quad_lane<1>(s0);
+        sum[2] = quad_lane<2>(s0);
+        sum[3] = quad_lane<3>(s0);
+        sum[4] = dust ? quad_lane<0>(s1) : 0.0;
+        sum[5] = dust ? quad_lane<1>(s1) : 0.0;
+      } else {
+        sum[0] = rho.value(); sum[1] = gradh.value(); sum[2] = ggh.value(); sum[3] = drhodt.value();
+        sum[4] = rhog.value(); sum[5] = rhod.value();
+      }
       if (fixedp) {
         a.numneigh[i] = nn;
         r_nmin = nn;
@@ -1651,12 +1721,12 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
         break;
       }
       // Newton-Raphson update, src/iterate_density.f90:162-278 (FP64)
-      rho_v = rho.value();
-      drhodt_v = drhodt.value();
-      if (dust) { rhog_v = rhog.value(); rhod_v = rhod.value(); }
+      rho_v = sum[0];
+      drhodt_v = sum[3];
+      if (dust) { rhog_v = sum[4]; rhod_v = sum[5]; }
       if (rho_v <= 0.0) { err = NDSP_ERR_RHO_NONPOSITIVE; done = true; break; }
       NRStep r;
-      nr_update<NDIM>(p, h, hin, mi, rho_v, gradh.value(), ggh.value(), nn, its, r);
+      nr_update<NDIM>(p, h, hin, mi, rho_v, sum[1], sum[2], nn, its, r);
       gradh_v = r.gradh;
       ggh_v = r.ggh;
       const double hnew = r.hnew;
@@ -1677,7 +1747,8 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
         break;
       }
     }
-    if (done) {
+    // (a quad's lanes hold the same results; the first one hands them on)
+    if (done && sub == 0) {
       // ---- results, then conservative->primitive and EOS for this particle ----
       a.f[F_H][i] = h;
       st_stream(&a.f[F_RHO][i], rho_v);
@@ -1730,7 +1801,7 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
       r_nmax = nn;
     }
     r_pairs = (double)npairs;
-    r_ncalc = its - its0 + 1;
+    if (sub == 0) r_ncalc = its - its0 + 1;
     if (err) atomicCAS(&a.sc->err, 0, err);
   }
   {
@@ -1744,7 +1815,8 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
   // the spatial order
   if (!persistent && !idle) {
     __shared__ int wcnt[TB / 64];
-    if (active) a.nrflag[tid] = unconverged ? 1 : 0;
+    unconverged = unconverged && sub == 0;
+    if (active && sub == 0) a.nrflag[tid] = unconverged ? 1 : 0;
     const int cnt = __popcll(__ballot(unconverged));
     if ((threadIdx.x & 63) == 0) wcnt[threadIdx.x >> 6] = cnt;
     __syncthreads();
@@ -1757,10 +1829,10 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
 }
 // three waves per SIMD (an occupancy attribute): with one record in flight
 // the FP32 pass fits in 168 registers, spilling two outside the pair loop
-template <int NDIM, typename PT, bool DUST, int TB>
+template <int NDIM, typename PT, bool DUST, int TB, int Q>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(3))) void k_nr_pass(
     KArgs a, Phys p, const Grid* __restrict__ gp, int* __restrict__ list_a, int* __restrict__ list_b) {
-  b_nr_pass<NDIM, PT, DUST, TB>(a, p, gp, list_a, list_b, VL{(int)blockIdx.x, (int)gridDim.x});
+  b_nr_pass<NDIM, PT, DUST, TB, Q>(a, p, gp, list_a, list_b, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // The pass control (src/iterate_density.f90:280-300): finished when the pass
@@ -1849,8 +1921,10 @@ __device__ __forceinline__ void b_pass_next(KArgs a, const Phys& p, int tb, int*
     if (lane == 0) wc[w] = __popcll(m);
     __syncthreads();
     if (f) {
-      int at = a.nrcnt[k / tb] + __popcll(m & ((1ull << lane) - 1ull));
-      // the earlier waves of the same tile
+      // those before it in its wave and tile
+      const int t0 = max(0, k / tb * tb - (k - lane));
+      int at = a.nrcnt[k / tb] + __popcll(m & ((1ull << lane) - 1ull) & ~((1ull << t0) - 1ull));
+      // and in the tile's earlier waves
       for (int u = w - 1; u >= 0 && (vl.b * (int)blockDim.x + 64 * u) / tb == k / tb; u--) at += wc[u];
       to[at] = from ? from[k] : k;
     }
@@ -1884,17 +1958,15 @@ __global__ __launch_bounds__(BS) void k_pass_next(KArgs a, Phys p, int tb, int* 
 
 // PHYS: 0 hydro, 1 MHD (imhd 11), 2 one-fluid dust (idust 4); TB threads
 // per workgroup (chosen by the autotuner)
-template <int NDIM, typename PT, int PHYS, int TB>
+template <int NDIM, typename PT, int PHYS, int TB, int Q>
 __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict__ gp, int guard, VL vl) {
   if (held_back(a.sc, guard)) return;
-  __shared__ PT tg[NDSP_IKERN + 1];
-  {
-    const PT* src = sizeof(PT) == 4 ? (const PT*)a.tabf : (const PT*)a.tabd;
-    for (int t = threadIdx.x; t <= NDSP_IKERN; t += blockDim.x) tg[t] = src[NDSP_IKERN + 1 + t];
-  }
+  __shared__ __align__(16) PT tg[NDSP_TAB];
+  load_table(tg, (sizeof(PT) == 4 ? (const PT*)a.tabf : (const PT*)a.tabd) + NDSP_TAB);
   __syncthreads();
   const Grid g = *gp;
-  const int k = xcd_tile(vl) * blockDim.x + threadIdx.x;
+  const int k = xcd_tile(vl) * (TB / Q) + (int)threadIdx.x / Q;
+  const int sub = (int)threadIdx.x % Q;  // the lane's place among the particle's
   const bool active = k < a.n;
   typedef typename V4<PT>::type T4;
   constexpr bool mhd = PHYS == 1;
@@ -1948,7 +2020,7 @@ __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict_
     const double rad = p.radkern * a.sc->hmax_nr;
     if (!(rad < p.boxmin)) err = NDSP_ERR_CELLS;
 
-    Acc<PT> fx, fy, fz, dudt, dbx, dby, dbz, divb, cbx, cby, cbz, gpx, gpy, gpz, del2u, deps, gdx, gdy, gdz;
+    PSum<PT, Q> fx, fy, fz, dudt, dbx, dby, dbz, divb, cbx, cby, cbz, gpx, gpy, gpz, del2u, deps, gdx, gdy, gdz;
     fx.zero(); fy.zero(); fz.zero(); dudt.zero(); dbx.zero(); dby.zero(); dbz.zero();
     divb.zero(); cbx.zero(); cby.zero(); cbz.zero(); gpx.zero(); gpy.zero(); gpz.zero();
     del2u.zero(); deps.zero(); gdx.zero(); gdy.zero(); gdz.zero();
@@ -2168,32 +2240,64 @@ __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict_
         gdz.add(mj * (dvel[2] - dvdotr) * grkerni);
       }
     };
+    double s[4] = {0.0, 0.0, 0.0, 0.0};  // Q = 4: lane j's sums (quantity j of each four)
+    auto flush = [&] {
+      if constexpr (Q == 4) {
+        quad_fold4(sub, fx.t, fy.t, fz.t, dudt.t, s[0]);
+        fx.zero(); fy.zero(); fz.zero(); dudt.zero();
+        if (mhd) {
+          quad_fold4(sub, dbx.t, dby.t, dbz.t, divb.t, s[1]);
+          quad_fold4(sub, cbx.t, cby.t, cbz.t, del2u.t, s[2]);
+          quad_fold4(sub, gpx.t, gpy.t, gpz.t, PT(0), s[3]);
+          dbx.zero(); dby.zero(); dbz.zero(); divb.zero(); cbx.zero(); cby.zero(); cbz.zero();
+          gpx.zero(); gpy.zero(); gpz.zero();
+        } else {
+          quad_fold4(sub, gdx.t, gdy.t, gdz.t, del2u.t, s[1]);
+          if (dust) quad_fold4(sub, deps.t, PT(0), PT(0), PT(0), s[2]);
+          gdx.zero(); gdy.zero(); gdz.zero(); deps.zero();
+        }
+        del2u.zero();
+      }
+    };
     if (!err) {
       // one record ahead: a second 96-byte record in flight would cost the
       // third wave per SIMD (162 registers with one, 180 with two)
-      if (uselist) for_each_listed_pf<NDIM, 1>(a, g, k, a.nbc[k] + a.nbx[k], loadj, body);
-      else for_each_candidate_rec<NDIM>(a, g, xi, rad, loadj, body);
+      if (!uselist) for_each_candidate_rec<NDIM, Q>(a, g, xi, rad, sub, loadj, body, flush);
+      else if constexpr (Q == 4) for_each_listed_quad<NDIM>(a, g, k, a.nbc[k] + a.nbx[k], sub, loadj, body, flush);
+      else for_each_listed_pf<NDIM, 1>(a, g, k, a.nbc[k] + a.nbx[k], loadj, body);
     }
-    st_stream(&a.f[F_FX][i], fx.value());
-    st_stream(&a.f[F_FY][i], fy.value());
-    st_stream(&a.f[F_FZ][i], fz.value());
-    st_stream(&a.f[F_DUDT][i], dudt.value());
-    st_stream(&a.f[F_DBX][i], dbx.value());
-    st_stream(&a.f[F_DBY][i], dby.value());
-    st_stream(&a.f[F_DBZ][i], dbz.value());
-    st_stream(&a.f[F_DIVB][i], divb.value());
-    st_stream(&a.f[F_CBX][i], cbx.value());
-    st_stream(&a.f[F_CBY][i], cby.value());
-    st_stream(&a.f[F_CBZ][i], cbz.value());
-    st_stream(&a.f[F_GPX][i], gpx.value());
-    st_stream(&a.f[F_GPY][i], gpy.value());
-    st_stream(&a.f[F_GPZ][i], gpz.value());
-    st_stream(&a.f[F_DEL2U][i], del2u.value());
-    st_stream(&a.f[F_DEPS][i], deps.value());
+    // (quantity, field) of every sum; the first lane of a quad stores
+    auto out = [&](int field, const PSum<PT, Q>& x, int four, int lane_) {
+      double v;
+      if constexpr (Q == 4) {
+        v = four < 0 ? 0.0
+            : lane_ == 0 ? quad_lane<0>(s[four]) : lane_ == 1 ? quad_lane<1>(s[four])
+            : lane_ == 2 ? quad_lane<2>(s[four]) : quad_lane<3>(s[four]);
+      } else {
+        v = x.value();
+      }
+      if (sub == 0) st_stream(&a.f[field][i], v);
+    };
+    out(F_FX, fx, 0, 0);
+    out(F_FY, fy, 0, 1);
+    out(F_FZ, fz, 0, 2);
+    out(F_DUDT, dudt, 0, 3);
+    out(F_DBX, dbx, mhd ? 1 : -1, 0);
+    out(F_DBY, dby, mhd ? 1 : -1, 1);
+    out(F_DBZ, dbz, mhd ? 1 : -1, 2);
+    out(F_DIVB, divb, mhd ? 1 : -1, 3);
+    out(F_CBX, cbx, mhd ? 2 : -1, 0);
+    out(F_CBY, cby, mhd ? 2 : -1, 1);
+    out(F_CBZ, cbz, mhd ? 2 : -1, 2);
+    out(F_GPX, gpx, mhd ? 3 : -1, 0);
+    out(F_GPY, gpy, mhd ? 3 : -1, 1);
+    out(F_GPZ, gpz, mhd ? 3 : -1, 2);
+    out(F_DEL2U, del2u, mhd ? 2 : 1, 3);
+    out(F_DEPS, deps, dust ? 2 : -1, 0);
     if (PHYS != 1) {
-      st_stream(&a.f[F_GDVX][i], gdx.value());
-      st_stream(&a.f[F_GDVY][i], gdy.value());
-      st_stream(&a.f[F_GDVZ][i], gdz.value());
+      out(F_GDVX, gdx, 1, 0);
+      out(F_GDVY, gdy, 1, 1);
+      out(F_GDVZ, gdz, 1, 2);
     }
   }
   if (err) atomicCAS(&a.sc->err, 0, err);
@@ -2204,9 +2308,9 @@ __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict_
     block_partials<3>(rv, rk, a.red, a.rcap, vl);
   }
 }
-template <int NDIM, typename PT, int PHYS, int TB>
+template <int NDIM, typename PT, int PHYS, int TB, int Q>
 __global__ __launch_bounds__(TB) void k_force(KArgs a, Phys p, const Grid* __restrict__ gp, int guard) {
-  b_force<NDIM, PT, PHYS, TB>(a, p, gp, guard, VL{(int)blockIdx.x, (int)gridDim.x});
+  b_force<NDIM, PT, PHYS, TB, Q>(a, p, gp, guard, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // per-particle finalisation, src/ratesND_mhd.f90:482-943 (FP64)
@@ -2960,7 +3064,7 @@ __global__ void k_nb(KArgs a, Phys p, const Grid* __restrict__ gp, int sym, cons
   int cnt = 0;
   if (!(rad < p.boxmin)) { if (!offs) out[k] = 0; return; }
   int base = offs ? offs[k] : 0;
-  for_each_candidate<NDIM>(a, g, xi, rad, [&](int kk, const double* xj, const int* flip, int icode) {
+  for_each_candidate<NDIM>(a, g, xi, rad, 0, [&](int kk, const double* xj, const int* flip, int icode) {
     double dx[3] = {0.0, 0.0, 0.0};
     for (int d = 0; d < NDIM; d++) dx[d] = xi[d] - xj[d];
     const double rij2 = rij2_exact<NDIM>(dx);
@@ -2985,7 +3089,7 @@ __global__ void k_nb(KArgs a, Phys p, const Grid* __restrict__ gp, int sym, cons
       out[3 * (base + cnt) + 2] = code;
     }
     cnt++;
-  });
+  }, [] {});
   if (!offs) out[k] = cnt;
 }
 
@@ -3067,8 +3171,11 @@ __global__ __launch_bounds__(FOLD_B) void km_pass_fold(const MArgs* __restrict__
   NDSP_MEMBER
   b_pass_fold(M.a, spec, M.nb_nr, tb, M.reflect, M.p.maxits, last ? M.out : nullptr);
 }
-NDSP_MK(km_pass_next_64) { NDSP_MEMBER b_pass_next(M.a, M.p, 64, M.list_a, M.list_b, vl); }
-NDSP_MK(km_pass_next_256) { NDSP_MEMBER b_pass_next(M.a, M.p, 256, M.list_a, M.list_b, vl); }
+__global__ __launch_bounds__(BS) void km_pass_next(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm,
+                                                   int tb) {
+  NDSP_MEMBER
+  b_pass_next(M.a, M.p, tb, M.list_a, M.list_b, vl);
+}
 __global__ __launch_bounds__(FOLD_B) void km_force_fold(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm,
                                                         RedSpec spec) {
   NDSP_MEMBER
@@ -3118,13 +3225,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void km
                                                                                          int nm) {
   NDSP_MEMBER b_nblist<NDIM>(M.a, M.p, M.gdev, vl);
 }
-template <int NDIM, typename PT, bool DUST, int TB>
+template <int NDIM, typename PT, bool DUST, int TB, int Q>
 __global__ __launch_bounds__(TB) void km_nr_pass(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm) {
-  NDSP_MEMBER b_nr_pass<NDIM, PT, DUST, TB>(M.a, M.p, M.gdev, M.list_a, M.list_b, vl);
+  NDSP_MEMBER b_nr_pass<NDIM, PT, DUST, TB, Q>(M.a, M.p, M.gdev, M.list_a, M.list_b, vl);
 }
-template <int NDIM, typename PT, int PHYS, int TB>
+template <int NDIM, typename PT, int PHYS, int TB, int Q>
 __global__ __launch_bounds__(TB) void km_force(const MArgs* __restrict__ ma, const int* __restrict__ off, int nm) {
-  NDSP_MEMBER b_force<NDIM, PT, PHYS, TB>(M.a, M.p, M.gdev, 1, vl);
+  NDSP_MEMBER b_force<NDIM, PT, PHYS, TB, Q>(M.a, M.p, M.gdev, 1, vl);
 }
 
 static int make_tables(int ikernel, int ndim, std::vector<double>& tab, double& radkern, double& dq2) {
@@ -3191,6 +3298,20 @@ static double nexp_of(const Phys& p) {
 // (33000 reals take 23 us this way and 200 with a copy command, 50000 take 250
 // and 42)
 static const size_t PIN_REALS = 40960;
+// Simulations up to this size run the h-rho passes with four lanes per particle
+// (b_nr_pass, Q = 4): with one lane they have fewer waves than the device has
+// SIMDs (1024), and a pass lasts as long as one wave walks its lists.  The
+// passes of one evaluation, one lane -> four: 800 particles 80 -> 66 us, 2D
+// 9000 86 -> 60, 3D 37^3 (50653) 193 -> 126, 203^2 quintic in FP64 245 -> 162 and
+// its force pass 338 -> 170; at four waves per SIMD and above the extra moves
+// between the lanes cost more than the shorter walks give.
+static const int64_t QUAD_MAX = 65536;
+// The force pass does too where its results are those of one lane per particle
+// bit for bit (1D, hydro, dust) or to FP64 rounding.  In mixed 2D and 3D MHD the
+// compiler contracts the pair's dot products differently in the two kernels; an
+// FP32 last bit there decides, steps later, whether single particles' h
+// iterations end at tolh, so those runs keep one lane.
+static constexpr bool quad_force_ok(int ndim, int phys, bool fp64) { return fp64 || phys != 1 || ndim == 1; }
 
 struct ndsp_ctx {
   int device = 0;           // HIP device current at creation (holds every buffer)
@@ -3198,6 +3319,8 @@ struct ndsp_ctx {
   int nfixed = 0;           // fixed boundary particles uploaded
   bool ireal_set = true;    // their partners have been given
   bool reflect = false;     // some wall reflects
+  bool quad = false;        // four lanes per particle in the h-rho passes (QUAD_MAX)
+  bool quad_force = false;  // and in the force pass (quad_force_ok)
   Grid* gdev = nullptr;     // cell grid of the last binning (device)
   int cap_bits = 0;         // Morton key-space capacity of cstart/cfill
   int maxnb_limit = 0;      // largest list capacity the lists may grow to
@@ -3472,6 +3595,22 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
   return 0;
 }
 
+// the force kernels with four lanes per particle, where they are used
+template <int ND, typename PT, int P>
+static auto quad_force() -> void (*)(KArgs, Phys, const Grid* __restrict__, int) {
+  if constexpr (quad_force_ok(ND, P, sizeof(PT) == 8)) return k_force<ND, PT, P, 256, 4>;
+  else return k_force<ND, PT, P, 256, 1>;
+}
+template <int ND, typename PT, int P>
+static auto km_quad_force() -> void (*)(const MArgs* __restrict__, const int* __restrict__, int) {
+  if constexpr (quad_force_ok(ND, P, sizeof(PT) == 8)) return km_force<ND, PT, P, 256, 4>;
+  else return km_force<ND, PT, P, 256, 1>;
+}
+
+// particles of a workgroup of the pair passes
+static int pass_tile(const ndsp_ctx* c) { return c->quad ? 64 : c->tb_nr; }
+static int force_tile(const ndsp_ctx* c) { return c->quad_force ? 64 : c->tb_force; }
+
 // K pass launches of the h-rho iteration; each reads its parameters from the
 // device-side control and does nothing once the iteration has finished
 static RedSpec spec_pass() {
@@ -3495,17 +3634,20 @@ static void launch_passes(ndsp_ctx* c, int K) {
       constexpr int ND = decltype(nd)::value;
       const bool fp64 = c->prec == NDSP_PREC_FP64, dust = c->p.idust != 0;
       const bool small = c->tb_nr == 64;
-      auto kern = fp64 ? (dust ? (small ? k_nr_pass<ND, double, true, 64> : k_nr_pass<ND, double, true, 256>)
-                               : (small ? k_nr_pass<ND, double, false, 64> : k_nr_pass<ND, double, false, 256>))
-                       : (dust ? (small ? k_nr_pass<ND, float, true, 64> : k_nr_pass<ND, float, true, 256>)
-                               : (small ? k_nr_pass<ND, float, false, 64> : k_nr_pass<ND, float, false, 256>));
-      hipLaunchKernelGGL(kern, dim3(nblk(n, c->tb_nr)), dim3(c->tb_nr), 0, c->st, a, c->p, (const Grid*)c->gdev,
-                         c->list_a, c->list_b);
+      void (*kern)(KArgs, Phys, const Grid* __restrict__, int* __restrict__, int* __restrict__);
+#define NDSP_NR(PTT, D) \
+  (c->quad ? k_nr_pass<ND, PTT, D, 256, 4> : small ? k_nr_pass<ND, PTT, D, 64, 1> : k_nr_pass<ND, PTT, D, 256, 1>)
+      if (fp64) kern = dust ? NDSP_NR(double, true) : NDSP_NR(double, false);
+      else kern = dust ? NDSP_NR(float, true) : NDSP_NR(float, false);
+#undef NDSP_NR
+      hipLaunchKernelGGL(kern, dim3(nblk(n, pass_tile(c))), dim3(c->quad ? 256 : c->tb_nr), 0, c->st, a, c->p,
+                         (const Grid*)c->gdev, c->list_a, c->list_b);
       return 0;
     });
-    hipLaunchKernelGGL(k_pass_fold, dim3(1), dim3(fold_threads(n, c->tb_nr)), 0, c->st, a, spec_pass(), (int)nblk(n, c->tb_nr), c->tb_nr,
+    hipLaunchKernelGGL(k_pass_fold, dim3(1), dim3(fold_threads(n, pass_tile(c))), 0, c->st, a, spec_pass(),
+                       (int)nblk(n, pass_tile(c)), pass_tile(c),
                        reflect ? 1 : 0, c->p.maxits, q == K - 1 ? c->hs : (DScal*)nullptr);
-    hipLaunchKernelGGL(k_pass_next, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, c->tb_nr, c->list_a, c->list_b);
+    hipLaunchKernelGGL(k_pass_next, dim3(nblk(n)), dim3(BS), 0, c->st, a, c->p, pass_tile(c), c->list_a, c->list_b);
   }
 }
 
@@ -3559,18 +3701,17 @@ static int do_rates(ndsp_ctx* c, bool with_correct = false, int guard = 0) {
       const int phys = c->p.imhd ? 1 : c->p.idust ? 2 : 0;
       void (*kern)(KArgs, Phys, const Grid* __restrict__, int);
       const bool small = c->tb_force == 64;
-      if (c->prec == NDSP_PREC_FP64) {
-        if (small) kern = phys == 1 ? k_force<ND, double, 1, 64> : phys == 2 ? k_force<ND, double, 2, 64> : k_force<ND, double, 0, 64>;
-        else kern = phys == 1 ? k_force<ND, double, 1, 256> : phys == 2 ? k_force<ND, double, 2, 256> : k_force<ND, double, 0, 256>;
-      } else {
-        if (small) kern = phys == 1 ? k_force<ND, float, 1, 64> : phys == 2 ? k_force<ND, float, 2, 64> : k_force<ND, float, 0, 64>;
-        else kern = phys == 1 ? k_force<ND, float, 1, 256> : phys == 2 ? k_force<ND, float, 2, 256> : k_force<ND, float, 0, 256>;
-      }
-      hipLaunchKernelGGL(kern, dim3(nblk(n, c->tb_force)), dim3(c->tb_force), 0, c->st, a, c->p, (const Grid*)c->gdev,
-                         guard);
+#define NDSP_F(PTT, P) \
+  (c->quad_force ? quad_force<ND, PTT, P>() : small ? k_force<ND, PTT, P, 64, 1> : k_force<ND, PTT, P, 256, 1>)
+      if (c->prec == NDSP_PREC_FP64) kern = phys == 1 ? NDSP_F(double, 1) : phys == 2 ? NDSP_F(double, 2) : NDSP_F(double, 0);
+      else kern = phys == 1 ? NDSP_F(float, 1) : phys == 2 ? NDSP_F(float, 2) : NDSP_F(float, 0);
+#undef NDSP_F
+      hipLaunchKernelGGL(kern, dim3(nblk(n, force_tile(c))), dim3(c->quad_force ? 256 : c->tb_force), 0, c->st, a, c->p,
+                         (const Grid*)c->gdev, guard);
       return 0;
     });
-    hipLaunchKernelGGL(k_force_fold, dim3(1), dim3(fold_threads(n, c->tb_force)), 0, c->st, a, spec_force(), (int)nblk(n, c->tb_force), guard);
+    hipLaunchKernelGGL(k_force_fold, dim3(1), dim3(fold_threads(n, force_tile(c))), 0, c->st, a, spec_force(),
+                       (int)nblk(n, force_tile(c)), guard);
   }
   {
     TScope t(c, "finalize");
@@ -3792,6 +3933,8 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   }
   c->g.ndim = p.ndim;
   c->reflect = nrefl > 0;
+  c->quad = npart <= QUAD_MAX;
+  c->quad_force = c->quad && quad_force_ok(p.ndim, fr_phys(p), precision == NDSP_PREC_FP64);
   c->dt = dopt[23];
   c->time = 0.0;
   auto cleanup_fail = [&](int e) { ndsp_destroy(c); return e; };
@@ -3846,8 +3989,8 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   }
   float* tabf = nullptr;
   double* tabd = nullptr;
-  ok &= hipMalloc(&tabf, sizeof(float) * tab.size()) == hipSuccess;
-  ok &= hipMalloc(&tabd, sizeof(double) * tab.size()) == hipSuccess;
+  ok &= hipMalloc(&tabf, sizeof(float) * 3 * NDSP_TAB) == hipSuccess;
+  ok &= hipMalloc(&tabd, sizeof(double) * 3 * NDSP_TAB) == hipSuccess;
   c->nb_part = 1024;
   ok &= hipMalloc(&c->part, sizeof(double) * 32 * c->nb_part) == hipSuccess;
   ok &= hipHostMalloc((void**)&c->cons_out, sizeof(double) * 32, hipHostMallocDefault) == hipSuccess;
@@ -3859,6 +4002,12 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   a.tabf = tabf;
   a.tabd = tabd;
   a.n = c->n;
+  {
+    std::vector<double> padded(3 * NDSP_TAB, 0.0);
+    for (int q = 0; q < 3; q++)
+      std::copy(tab.begin() + q * (NDSP_IKERN + 1), tab.begin() + (q + 1) * (NDSP_IKERN + 1), padded.begin() + q * NDSP_TAB);
+    tab.swap(padded);
+  }
   std::vector<float> tf(tab.begin(), tab.end());
   hipMemcpy(tabf, tf.data(), sizeof(float) * tf.size(), hipMemcpyHostToDevice);
   hipMemcpy(tabd, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice);
@@ -4220,7 +4369,7 @@ static int ensure_key_space(ndsp_ctx* c);
 // A group of batch members that share dimension, physics, neighbour-list use
 // and walls: one launch per phase covers all of them.
 struct BGroup {
-  int ndim = 0, phys = 0, dust = 0, lists = 0, reflect = 0;
+  int ndim = 0, phys = 0, dust = 0, lists = 0, reflect = 0, quad = 0, quad_force = 0;
   int fixed = 0;  // some member holds fixed particles
   std::vector<int> mem;
   MArgs* args = nullptr;
@@ -4265,7 +4414,8 @@ static int batch_build(ndsp_batch* b) {
     const int phys = c->p.imhd ? 1 : c->p.idust ? 2 : 0;
     BGroup* g = nullptr;
     for (auto& q : b->groups)
-      if (q.ndim == c->p.ndim && q.phys == phys && q.lists == c->p.use_list && q.reflect == (int)c->reflect)
+      if (q.ndim == c->p.ndim && q.phys == phys && q.lists == c->p.use_list && q.reflect == (int)c->reflect &&
+          q.quad == (int)c->quad)
         g = &q;
     if (!g) {
       b->groups.emplace_back();
@@ -4275,6 +4425,8 @@ static int batch_build(ndsp_batch* b) {
       g->dust = c->p.idust != 0;
       g->lists = c->p.use_list;
       g->reflect = c->reflect;
+      g->quad = c->quad;
+      g->quad_force = c->quad_force;
     }
     g->mem.push_back(s);
     g->fixed |= c->p.fixed_on;
@@ -4313,8 +4465,8 @@ static int batch_build(ndsp_batch* b) {
       M.cap_bits = c->cap_bits;
       M.reflect = c->reflect;
       M.nbp = (int)bin_blocks(n);
-      M.nb_nr = (int)nblk(n, b->tb);
-      M.nb_force = (int)nblk(n, b->tb);
+      M.nb_nr = (int)nblk(n, c->quad ? 64 : b->tb);
+      M.nb_force = (int)nblk(n, c->quad_force ? 64 : b->tb);
       M.nb_256 = (int)nblk(n);
       M.scratch_d = c->scratch_d;
       M.scratch_i = c->scratch_i;
@@ -4386,18 +4538,19 @@ static int batch_part_a(ndsp_batch* b) {
     for (int q = 0; q < K; q++) {
       dispatch_ndim(g.ndim, [&](auto nd) {
         constexpr int ND = decltype(nd)::value;
-        if (b->tb == 64) {
-          if (fp64) { if (g.dust) BLAUNCH((km_nr_pass<ND, double, true, 64>), g, BGroup::S_NR, 64); else BLAUNCH((km_nr_pass<ND, double, false, 64>), g, BGroup::S_NR, 64); }
-          else { if (g.dust) BLAUNCH((km_nr_pass<ND, float, true, 64>), g, BGroup::S_NR, 64); else BLAUNCH((km_nr_pass<ND, float, false, 64>), g, BGroup::S_NR, 64); }
-        } else {
-          if (fp64) { if (g.dust) BLAUNCH((km_nr_pass<ND, double, true, 256>), g, BGroup::S_NR, 256); else BLAUNCH((km_nr_pass<ND, double, false, 256>), g, BGroup::S_NR, 256); }
-          else { if (g.dust) BLAUNCH((km_nr_pass<ND, float, true, 256>), g, BGroup::S_NR, 256); else BLAUNCH((km_nr_pass<ND, float, false, 256>), g, BGroup::S_NR, 256); }
-        }
+#define NDSP_NR_B(PTT, D)                                                                      \
+  do {                                                                                         \
+    if (g.quad) BLAUNCH((km_nr_pass<ND, PTT, D, 256, 4>), g, BGroup::S_NR, 256);               \
+    else if (b->tb == 64) BLAUNCH((km_nr_pass<ND, PTT, D, 64, 1>), g, BGroup::S_NR, 64);       \
+    else BLAUNCH((km_nr_pass<ND, PTT, D, 256, 1>), g, BGroup::S_NR, 256);                      \
+  } while (0)
+        if (fp64) { if (g.dust) NDSP_NR_B(double, true); else NDSP_NR_B(double, false); }
+        else { if (g.dust) NDSP_NR_B(float, true); else NDSP_NR_B(float, false); }
+#undef NDSP_NR_B
         return 0;
       });
-      BLAUNCH(km_pass_fold, g, BGroup::S_ONE, BS, spec_pass(), b->tb, q == K - 1 ? 1 : 0);
-      if (b->tb == 64) BLAUNCH(km_pass_next_64, g, BGroup::S_256, BS);
-      else BLAUNCH(km_pass_next_256, g, BGroup::S_256, BS);
+      BLAUNCH(km_pass_fold, g, BGroup::S_ONE, BS, spec_pass(), g.quad ? 64 : b->tb, q == K - 1 ? 1 : 0);
+      BLAUNCH(km_pass_next, g, BGroup::S_256, BS, g.quad ? 64 : b->tb);
     }
   }
   if (int e = batch_join(b)) return e;
@@ -4417,14 +4570,14 @@ static int batch_part_b(ndsp_batch* b) {
     else BLAUNCH(km_pack_force<float>, g, BGroup::S_256, BS);
     dispatch_ndim(g.ndim, [&](auto nd) {
       constexpr int ND = decltype(nd)::value;
-#define NDSP_FORCE_B(PTT, TBB)                                                                        \
-  do {                                                                                                \
-    if (g.phys == 1) BLAUNCH((km_force<ND, PTT, 1, TBB>), g, BGroup::S_FORCE, TBB);                   \
-    else if (g.phys == 2) BLAUNCH((km_force<ND, PTT, 2, TBB>), g, BGroup::S_FORCE, TBB);              \
-    else BLAUNCH((km_force<ND, PTT, 0, TBB>), g, BGroup::S_FORCE, TBB);                               \
+#define NDSP_FORCE_B(PTT, P)                                                                   \
+  do {                                                                                         \
+    if (g.quad_force) BLAUNCH((km_quad_force<ND, PTT, P>()), g, BGroup::S_FORCE, 256);         \
+    else if (b->tb == 64) BLAUNCH((km_force<ND, PTT, P, 64, 1>), g, BGroup::S_FORCE, 64);      \
+    else BLAUNCH((km_force<ND, PTT, P, 256, 1>), g, BGroup::S_FORCE, 256);                     \
   } while (0)
-      if (b->tb == 64) { if (fp64) NDSP_FORCE_B(double, 64); else NDSP_FORCE_B(float, 64); }
-      else { if (fp64) NDSP_FORCE_B(double, 256); else NDSP_FORCE_B(float, 256); }
+      if (fp64) { if (g.phys == 1) NDSP_FORCE_B(double, 1); else if (g.phys == 2) NDSP_FORCE_B(double, 2); else NDSP_FORCE_B(double, 0); }
+      else { if (g.phys == 1) NDSP_FORCE_B(float, 1); else if (g.phys == 2) NDSP_FORCE_B(float, 2); else NDSP_FORCE_B(float, 0); }
 #undef NDSP_FORCE_B
       return 0;
     });

@@ -5,6 +5,9 @@
 #include <stdint.h>
 
 #define NDSP_IKERN 4000
+// a kernel table's length in memory: 4001 entries, padded so that the next one
+// starts on 16 bytes
+#define NDSP_TAB 4004
 
 // Cell grid.  Dimensions with walls (periodic or reflecting) are tiled exactly
 // by nc cells of width w = (xmax - xmin)/nc >= radkern*hmax/cell_sub, so
@@ -204,6 +207,53 @@ struct Acc {
   __device__ __forceinline__ void add(T x) { s += (double)x; }
   __device__ __forceinline__ double value() const { return s; }
 };
+
+// Sums over Q lanes per particle.  Q = 1: the lane's own accumulator.  Q = 4:
+// each lane of a quad forms the terms of one of four consecutive list entries;
+// quad_fold4 then hands lane j the four entries' terms of its quantity j, which
+// it adds in list order: the same additions, in the same order, as one lane
+// walking the list (an entry outside the kernel adds an exact zero).
+template <typename T, int Q>
+struct PSum : Acc<T> {};
+template <typename T>
+struct PSum<T, 4> {
+  T t;
+  __device__ __forceinline__ void zero() { t = T(0); }
+  __device__ __forceinline__ void add(T x) { t = x; }
+};
+template <int CTRL>
+__device__ __forceinline__ float quad_move(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ __forceinline__ int quad_move(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ double quad_move(double x) {
+  const long long b = __double_as_longlong(x);
+  const unsigned lo = (unsigned)quad_move<CTRL>((int)(unsigned)(b & 0xffffffffll));
+  const int hi = quad_move<CTRL>((int)(b >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (long long)lo);
+}
+// the value of lane L of the quad
+template <int L, typename T>
+__device__ __forceinline__ T quad_lane(T x) { return quad_move<L * 0x55>(x); }
+// quad_perm [1,0,3,2] and [2,3,0,1]
+#define QUAD_XOR1 0xB1
+#define QUAD_XOR2 0x4E
+// lane j's s += quantity j (r0..r3) of lanes 0, 1, 2, 3 in turn
+template <typename T>
+__device__ __forceinline__ void quad_fold4(int j, T r0, T r1, T r2, T r3, double& s) {
+  const bool odd = j & 1, up = j & 2;
+  const T a = quad_move<QUAD_XOR1>(odd ? r0 : r1), b = quad_move<QUAD_XOR1>(odd ? r2 : r3);
+  const T p0 = odd ? a : r0, p1 = odd ? r1 : a, q0 = odd ? b : r2, q1 = odd ? r3 : b;
+  const T c = quad_move<QUAD_XOR2>(up ? p0 : q0), d = quad_move<QUAD_XOR2>(up ? p1 : q1);
+  s += (double)(up ? c : p0);
+  s += (double)(up ? d : p1);
+  s += (double)(up ? q0 : c);
+  s += (double)(up ? q1 : d);
+}
 
 // square root, reciprocal and quotient of the pair math: FP32 uses the
 // hardware v_sqrt_f32 / v_rcp_f32 (about 1 ulp), FP64 the correctly rounded

@@ -129,7 +129,7 @@ struct KArgs {
   void* FR;
   void* GF;           // force, images only: m a0 a1 a2 (fixed particles: before the copy)
   // kernel tables (FP32 and FP64 copies of W, dW, d2W)
-  const float* tabf;  // 3 x (IKERN+1)
+  const float* tabf;  // 3 x NDSP_TAB
   const double* tabd;
   // neighbour lists, particle-major: entry m of sorted particle k at
   // nbl[k*maxnb + m] = (sorted index << 7) | image code (kinds kx + 5 ky + 25 kz)
