@@ -4370,6 +4370,7 @@ static int ensure_key_space(ndsp_ctx* c);
 // and walls: one launch per phase covers all of them.
 struct BGroup {
   int ndim = 0, phys = 0, dust = 0, lists = 0, reflect = 0, quad = 0, quad_force = 0;
+  int64_t total = 0;  // particles
   int fixed = 0;  // some member holds fixed particles
   std::vector<int> mem;
   MArgs* args = nullptr;
@@ -4430,7 +4431,15 @@ static int batch_build(ndsp_batch* b) {
     }
     g->mem.push_back(s);
     g->fixed |= c->p.fixed_on;
+    g->total += c->n;
   }
+  // four lanes per particle only where the whole group leaves the device idle
+  // (a workgroup then loads its tables for 64 particles instead of 256: the
+  // first pass of a group of 230000 takes 93 us with four lanes and 57 with
+  // one).  In FP64 a member keeps what it uses alone, where the two differ in
+  // the last bit.
+  for (auto& g : b->groups)
+    if (b->prec != NDSP_PREC_FP64 && g.total > QUAD_MAX) g.quad = g.quad_force = 0;
   while (b->gst.size() + 1 < b->groups.size()) {
     hipStream_t st = nullptr;
     HIPCHK(hipStreamCreate(&st));
@@ -4465,8 +4474,8 @@ static int batch_build(ndsp_batch* b) {
       M.cap_bits = c->cap_bits;
       M.reflect = c->reflect;
       M.nbp = (int)bin_blocks(n);
-      M.nb_nr = (int)nblk(n, c->quad ? 64 : b->tb);
-      M.nb_force = (int)nblk(n, c->quad_force ? 64 : b->tb);
+      M.nb_nr = (int)nblk(n, g.quad ? 64 : b->tb);
+      M.nb_force = (int)nblk(n, g.quad_force ? 64 : b->tb);
       M.nb_256 = (int)nblk(n);
       M.scratch_d = c->scratch_d;
       M.scratch_i = c->scratch_i;
