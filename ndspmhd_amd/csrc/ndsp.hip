@@ -2913,15 +2913,6 @@ __global__ __launch_bounds__(FOLD_T) void k_ev_final(const double* __restrict__ 
 // reorder of the particle state into cell order
 // ===========================================================================
 
-__global__ void k_fill_f(float* __restrict__ a, int n, float v) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) a[k] = v;
-}
-
-__global__ void k_gather_d(const double* __restrict__ in, double* __restrict__ out, const int* sidx, int n) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) out[k] = in[sidx[k]];
-}
 __global__ void k_fill_d(double* __restrict__ a, int n, double v) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) a[i] = v;
 }
@@ -2939,14 +2930,6 @@ __global__ void k_gather_probe(const double4* __restrict__ src, float* __restric
   const long long j = (long long)(((unsigned long long)i * mult) & (unsigned long long)(nl - 1));
   const double4 u = src[2 * j], v = src[2 * j + 1];
   out[i] = (float)(u.x + u.y + u.z + u.w + v.x + v.y + v.z + v.w);
-}
-__global__ void k_copy_i(const int* __restrict__ in, int* __restrict__ out, int n) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) out[k] = in[k];
-}
-__global__ void k_gather_i(const int* __restrict__ in, int* __restrict__ out, const int* sidx, int n) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < n) out[k] = in[sidx[k]];
 }
 
 // up to REORDER_W fields of one kind per launch: gather into the scratch
@@ -4277,7 +4260,7 @@ static int step_part_b(ndsp_ctx* c) {
       long long stride = 1000003;
       while (std::__gcd(stride, (long long)c->n) != 1) stride += 2;
       const long long off = (long long)(((unsigned long long)(c->nsteps + 1) * 2654435761ULL + it * 40503ULL) % c->n);
-      mlp_launch_grad(ml, ml.X, c->n, B, off, stride, c->st);
+      mlp_launch_grad(ml, ml.X, MLP_LDX, ml.X + MLP_COL_TARGET, MLP_LDX, c->n, B, off, stride, c->st);
       mlp_launch_adam(ml, ml.lr, c->st);
     }
   }
@@ -5181,20 +5164,20 @@ int ndsp_mlp_get_params(ndsp_ctx* c, float* params, int32_t n, int32_t* adam_ste
   return 0;
 }
 
+// a caller's batch on the device, as it is: features [B][6], then the targets;
+// the outputs follow
 static int mlp_stage(ndsp_ctx* c, const float* X, const float* T, int32_t B) {
   MlpState& m = c->mlp;
   if (B > m.xext_rows) {
     if (m.Xext) (void)hipFree(m.Xext);
     m.Xext = nullptr;
-    HIPCHK(hipMalloc(&m.Xext, sizeof(float) * MLP_LDX * (size_t)B));
+    m.xext_rows = 0;
+    HIPCHK(hipMalloc(&m.Xext, sizeof(float) * (MLP_NIN + 2) * (size_t)B));
     m.xext_rows = B;
   }
-  std::vector<float> buf((size_t)B * MLP_LDX, 0.0f);
-  for (int b = 0; b < B; b++) {
-    for (int q = 0; q < MLP_NIN; q++) buf[(size_t)b * MLP_LDX + q] = X[(size_t)b * MLP_NIN + q];
-    if (T) buf[(size_t)b * MLP_LDX + MLP_COL_TARGET] = T[b];
-  }
-  HIPCHK(hipMemcpy(m.Xext, buf.data(), sizeof(float) * buf.size(), hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpyAsync(m.Xext, X, sizeof(float) * MLP_NIN * (size_t)B, hipMemcpyHostToDevice, c->st));
+  if (T)
+    HIPCHK(hipMemcpyAsync(m.Xext + (size_t)MLP_NIN * B, T, sizeof(float) * (size_t)B, hipMemcpyHostToDevice, c->st));
   return 0;
 }
 
@@ -5202,13 +5185,11 @@ int ndsp_mlp_forward(ndsp_ctx* c, const float* X, int32_t B, float* y) {
   if (!c || !X || !y || B < 1) return set_err(NDSP_ERR_BAD_ARG, "mlp_forward: bad arguments");
   if (int e = mlp_ready(c)) return e;
   if (int e = mlp_stage(c, X, nullptr, B)) return e;
-  float* dy = nullptr;
-  HIPCHK(hipMalloc(&dy, sizeof(float) * B));
-  mlp_launch_forward(c->mlp, c->mlp.Xext, MLP_LDX, B, dy, c->st);
+  float* dy = c->mlp.Xext + (size_t)(MLP_NIN + 1) * B;
+  mlp_launch_forward(c->mlp, c->mlp.Xext, MLP_NIN, B, dy, c->st);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(y, dy, sizeof(float) * B, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipMemcpyAsync(y, dy, sizeof(float) * (size_t)B, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  (void)hipFree(dy);
   return 0;
 }
 
@@ -5216,13 +5197,11 @@ int ndsp_mlp_infer(ndsp_ctx* c, const float* X, int32_t B, float* y) {
   if (!c || !X || !y || B < 1) return set_err(NDSP_ERR_BAD_ARG, "mlp_infer: bad arguments");
   if (int e = mlp_ready(c)) return e;
   if (int e = mlp_stage(c, X, nullptr, B)) return e;
-  float* dy = nullptr;
-  HIPCHK(hipMalloc(&dy, sizeof(float) * B));
-  mlp_launch_infer(c->mlp, c->mlp.Xext, MLP_LDX, B, dy, c->st);
+  float* dy = c->mlp.Xext + (size_t)(MLP_NIN + 1) * B;
+  mlp_launch_infer(c->mlp, c->mlp.Xext, MLP_NIN, B, dy, c->st);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(y, dy, sizeof(float) * B, hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipMemcpyAsync(y, dy, sizeof(float) * (size_t)B, hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  (void)hipFree(dy);
   return 0;
 }
 
@@ -5253,15 +5232,14 @@ int ndsp_mlp_grad(ndsp_ctx* c, const float* X, const float* T, int32_t B, float*
   if (int e = mlp_ready(c)) return e;
   if (int e = mlp_stage(c, X, T, B)) return e;
   MlpState& m = c->mlp;
-  hipLaunchKernelGGL(k_fill_f, dim3(nblk(MLP_NPARAM)), dim3(BS), 0, c->st, m.grad, (int)MLP_NPARAM, 0.0f);
-  mlp_launch_grad(m, m.Xext, B, B, 0, 1, c->st);
+  mlp_launch_grad(m, m.Xext, MLP_NIN, m.Xext + (size_t)MLP_NIN * B, 1, B, B, 0, 1, c->st);
   HIPCHK(hipGetLastError());
-  float l = 0.f;
-  HIPCHK(hipMemcpyAsync(grad, m.grad, sizeof(float) * MLP_NPARAM, hipMemcpyDeviceToHost, c->st));
-  HIPCHK(hipMemcpyAsync(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost, c->st));
+  float g[MLP_NPARAM + 1];
+  HIPCHK(hipMemcpyAsync(g, m.grad, sizeof(g), hipMemcpyDeviceToHost, c->st));
+  mlp_launch_zero_grad(m, c->st);
   HIPCHK(hipStreamSynchronize(c->st));
-  hipLaunchKernelGGL(k_fill_f, dim3(nblk(MLP_NPARAM)), dim3(BS), 0, c->st, m.grad, (int)MLP_NPARAM, 0.0f);
-  if (loss) *loss = l;
+  memcpy(grad, g, sizeof(float) * MLP_NPARAM);
+  if (loss) *loss = g[MLP_NPARAM];
   return 0;
 }
 
@@ -5273,8 +5251,8 @@ int ndsp_mlp_train(ndsp_ctx* c, const float* X, const float* T, int32_t B, int32
   MlpState& m = c->mlp;
   float l = 0.f;
   for (int it = 0; it < iters; it++) {
-    mlp_launch_grad(m, m.Xext, B, B, 0, 1, c->st);
-    HIPCHK(hipMemcpyAsync(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost, c->st));
+    mlp_launch_grad(m, m.Xext, MLP_NIN, m.Xext + (size_t)MLP_NIN * B, 1, B, B, 0, 1, c->st);
+    if (it == iters - 1) HIPCHK(hipMemcpyAsync(&l, m.loss, sizeof(float), hipMemcpyDeviceToHost, c->st));
     mlp_launch_adam(m, (float)lr, c->st);
   }
   HIPCHK(hipGetLastError());

@@ -18,10 +18,10 @@ struct MlpState {
   uint16_t* wbf = nullptr;  // BF16 weights used by every forward
   float* m = nullptr;
   float* v = nullptr;
-  float* grad = nullptr;
+  float* grad = nullptr;    // gradient, then the loss
   float* loss = nullptr;
   float* X = nullptr;       // per-particle feature rows [n][MLP_LDX]
-  float* Xext = nullptr;    // staging for caller-supplied batches
+  float* Xext = nullptr;    // caller batches: 6 features, then the target, then the output of every row
   int nrows = 0;
   int xext_rows = 0;
   int adam_steps = 0;
@@ -59,6 +59,8 @@ void mlp_launch_forward(MlpState& s, const float* X, int ldx, int B, float* y, h
 // the same network on the matrix cores (BF16 inputs and activations)
 void mlp_launch_infer(MlpState& s, const float* X, int ldx, int B, float* y, hipStream_t st);
 void mlp_launch_seed_mfma(MlpState& s, const MlpSeedFields& f, hipStream_t st);
-void mlp_launch_grad(MlpState& s, const float* X, int nrows, int B, long long off, long long stride,
-                     hipStream_t st);
+// gradient over B rows of X[.][ldx], targets T[row * ldt]
+void mlp_launch_grad(MlpState& s, const float* X, int ldx, const float* T, int ldt, int nrows, int B, long long off,
+                     long long stride, hipStream_t st);
+void mlp_launch_zero_grad(MlpState& s, hipStream_t st);
 void mlp_launch_adam(MlpState& s, float lr, hipStream_t st);

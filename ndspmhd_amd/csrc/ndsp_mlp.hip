@@ -15,7 +15,8 @@
 
 #define NIN MLP_NIN
 #define NH MLP_NH
-#define WB 64  // samples per training block (one wavefront)
+#define WB 64          // samples per block of the FP32 passes (four waves, eight hidden units each)
+#define WU (NH / 4)
 
 __device__ __forceinline__ float bf16_to_f(uint16_t b) { return __uint_as_float(((uint32_t)b) << 16); }
 
@@ -42,117 +43,143 @@ __device__ __forceinline__ void load_weights(const uint16_t* __restrict__ wbf, f
   __syncthreads();
 }
 
-// forward of one sample; keeps z1, z2 (pre-activations) and a1, a2
-__device__ __forceinline__ float mlp_fwd(const float* sw, const float* x, float* z1, float* a1, float* z2,
-                                         float* a2) {
-  const float* W1 = sw;
+// The FP32 passes: a block of four waves takes WB samples; lane s of every wave
+// works on sample s, wave g on the hidden units WU g .. WU g + WU - 1 (their
+// weights are broadcast reads), and the activations pass between the waves
+// through LDS.  Each unit's sum runs in the order a single thread would take.
+// (One thread a sample left 16384 rows with 256 waves, one per CU: gradient 51 us
+// and forward 17; 24 and 9 here.)
+struct MlpTile {
+  float sw[MLP_NPARAM];
+  float a1[WB][NH + 1], a2[WB][NH + 1];
+};
+
+// forward of the block's samples: activations in t, the wave's own
+// pre-activations in z1, z2, the output of sample threadIdx % 64 returned
+__device__ __forceinline__ float mlp_fwd_tile(MlpTile& t, const float (&x)[NIN], float (&z1)[WU], float (&z2)[WU]) {
+  const int s = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const float* W1 = t.sw;
   const float* b1 = W1 + NH * NIN;
   const float* W2 = b1 + NH;
   const float* b2 = W2 + NH * NH;
   const float* W3 = b2 + NH;
-  const float b3 = W3[NH];
-  for (int o = 0; o < NH; o++) {
-    float s = b1[o];
-    for (int i = 0; i < NIN; i++) s += W1[o * NIN + i] * x[i];
-    z1[o] = s;
-    a1[o] = gelu(s);
+#pragma unroll
+  for (int u = 0; u < WU; u++) {
+    const int o = WU * g + u;
+    float v = b1[o];
+#pragma unroll
+    for (int i = 0; i < NIN; i++) v += W1[o * NIN + i] * x[i];
+    z1[u] = v;
+    t.a1[s][o] = gelu(v);
   }
-  for (int o = 0; o < NH; o++) {
-    float s = b2[o];
-    for (int i = 0; i < NH; i++) s += W2[o * NH + i] * a1[i];
-    z2[o] = s;
-    a2[o] = gelu(s);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < WU; u++) z2[u] = b2[WU * g + u];
+#pragma unroll 8
+  for (int i = 0; i < NH; i++) {
+    const float a = t.a1[s][i];
+#pragma unroll
+    for (int u = 0; u < WU; u++) z2[u] += W2[(WU * g + u) * NH + i] * a;
   }
-  float y = b3;
-  for (int i = 0; i < NH; i++) y += W3[i] * a2[i];
+#pragma unroll
+  for (int u = 0; u < WU; u++) t.a2[s][WU * g + u] = gelu(z2[u]);
+  __syncthreads();
+  float y = W3[NH];
+#pragma unroll 8
+  for (int i = 0; i < NH; i++) y += W3[i] * t.a2[s][i];
   return y;
 }
 
-// inference on a feature matrix X[B][8] (columns 0..5 are the features)
+// forward on a feature matrix X[B][ldx] (columns 0..5 are the features)
 __global__ __launch_bounds__(256) void k_mlp_forward(const uint16_t* __restrict__ wbf, const float* __restrict__ X,
                                                      int ldx, int B, float* __restrict__ y) {
-  __shared__ float sw[MLP_NPARAM];
-  load_weights(wbf, sw);
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
-  float x[NIN], z1[NH], a1[NH], z2[NH], a2[NH];
-  for (int i = 0; i < NIN; i++) x[i] = X[(size_t)b * ldx + i];
-  y[b] = mlp_fwd(sw, x, z1, a1, z2, a2);
+  __shared__ MlpTile t;
+  load_weights(wbf, t.sw);
+  const int b = blockIdx.x * WB + (threadIdx.x & 63);
+  float x[NIN], z1[WU], z2[WU];
+  for (int i = 0; i < NIN; i++) x[i] = b < B ? X[(size_t)b * ldx + i] : 0.0f;
+  const float out = mlp_fwd_tile(t, x, z1, z2);
+  if (threadIdx.x < 64 && b < B) y[b] = out;
 }
 
-// gradient of L = sum (y - t)^2 / B over the samples idx(b), b < B; sample b
-// is row (off + b * stride) mod nrows of X (target in column tcol)
-__global__ __launch_bounds__(WB) void k_mlp_grad(const uint16_t* __restrict__ wbf, const float* __restrict__ X,
-                                                 int nrows, int tcol, int B, long long off, long long stride,
-                                                 float* __restrict__ grad, float* __restrict__ loss) {
-  __shared__ float sw[MLP_NPARAM];
+// gradient of L = sum (y - t)^2 / B over the samples b < B; sample b is row
+// (off + b * stride) mod nrows of X[.][ldx], its target at T[row * ldt]
+__global__ __launch_bounds__(256) void k_mlp_grad(const uint16_t* __restrict__ wbf, const float* __restrict__ X, int ldx,
+                                                  const float* __restrict__ T, int ldt, int nrows, int B, long long off,
+                                                  long long stride, float* __restrict__ grad, float* __restrict__ loss) {
+  __shared__ MlpTile t;
   __shared__ float sX[WB][NIN + 1];
-  __shared__ float sA1[WB][NH + 1];
-  __shared__ float sA2[WB][NH + 1];
   __shared__ float sD1[WB][NH + 1];
   __shared__ float sD2[WB][NH + 1];
   __shared__ float sDy[WB];
-  load_weights(wbf, sw);
-  const int t = threadIdx.x;
-  const int b = blockIdx.x * WB + t;
+  load_weights(wbf, t.sw);
+  const int s = threadIdx.x & 63, g = threadIdx.x >> 6;
+  const int b = blockIdx.x * WB + s;
   const bool act = b < B;
-  float x[NIN], z1[NH], a1[NH], z2[NH], a2[NH];
-  float dy = 0.0f, r = 0.0f;
-  if (act) {
-    const long long row = (off + (long long)b * stride) % nrows;
-    for (int i = 0; i < NIN; i++) x[i] = X[row * MLP_LDX + i];
-    const float y = mlp_fwd(sw, x, z1, a1, z2, a2);
-    r = y - X[row * MLP_LDX + tcol];
-    dy = 2.0f * r / (float)B;
-  } else {
-    for (int i = 0; i < NIN; i++) x[i] = 0.0f;
-    for (int o = 0; o < NH; o++) { z1[o] = a1[o] = z2[o] = a2[o] = 0.0f; }
-  }
-  const float* W2 = sw + NH * NIN + NH;
+  const long long row = act ? (off + (long long)b * stride) % nrows : 0;
+  float x[NIN], z1[WU], z2[WU];
+  for (int i = 0; i < NIN; i++) x[i] = act ? X[row * ldx + i] : 0.0f;
+  const float y = mlp_fwd_tile(t, x, z1, z2);
+  const float r = act ? y - T[row * ldt] : 0.0f;
+  const float dy = act ? 2.0f * r / (float)B : 0.0f;
+  const float* W2 = t.sw + NH * NIN + NH;
   const float* W3 = W2 + NH * NH + NH;
-  float d2[NH];
-  for (int o = 0; o < NH; o++) d2[o] = dy * W3[o] * dgelu(z2[o]);
-  for (int i = 0; i < NH; i++) {
-    float s = 0.0f;
-    for (int o = 0; o < NH; o++) s += W2[o * NH + i] * d2[o];
-    sD1[t][i] = act ? s * dgelu(z1[i]) : 0.0f;
-    sA1[t][i] = a1[i];
-    sA2[t][i] = a2[i];
-    sD2[t][i] = act ? d2[i] : 0.0f;
+#pragma unroll
+  for (int u = 0; u < WU; u++) {
+    const int o = WU * g + u;
+    sD2[s][o] = act ? dy * W3[o] * dgelu(z2[u]) : 0.0f;
   }
-  for (int i = 0; i < NIN; i++) sX[t][i] = x[i];
-  sDy[t] = dy;
+  if (g == 0) {
+    for (int i = 0; i < NIN; i++) sX[s][i] = x[i];
+    sDy[s] = dy;
+  }
+  __syncthreads();
+  float d1[WU];
+#pragma unroll
+  for (int u = 0; u < WU; u++) d1[u] = 0.0f;
+#pragma unroll 8
+  for (int o = 0; o < NH; o++) {
+    const float d = sD2[s][o];
+#pragma unroll
+    for (int u = 0; u < WU; u++) d1[u] += W2[o * NH + WU * g + u] * d;
+  }
+#pragma unroll
+  for (int u = 0; u < WU; u++) sD1[s][WU * g + u] = act ? d1[u] * dgelu(z1[u]) : 0.0f;
   __syncthreads();
   // each thread sums whole parameter gradients over the block's samples
-  for (int p = t; p < MLP_NPARAM; p += WB) {
-    float s = 0.0f;
+  for (int p = threadIdx.x; p < MLP_NPARAM; p += 256) {
+    float v = 0.0f;
     int q = p;
     if (q < NH * NIN) {
       const int o = q / NIN, i = q % NIN;
-      for (int k = 0; k < WB; k++) s += sD1[k][o] * sX[k][i];
+      for (int k = 0; k < WB; k++) v += sD1[k][o] * sX[k][i];
     } else if ((q -= NH * NIN) < NH) {
-      for (int k = 0; k < WB; k++) s += sD1[k][q];
+      for (int k = 0; k < WB; k++) v += sD1[k][q];
     } else if ((q -= NH) < NH * NH) {
       const int o = q / NH, i = q % NH;
-      for (int k = 0; k < WB; k++) s += sD2[k][o] * sA1[k][i];
+      for (int k = 0; k < WB; k++) v += sD2[k][o] * t.a1[k][i];
     } else if ((q -= NH * NH) < NH) {
-      for (int k = 0; k < WB; k++) s += sD2[k][q];
+      for (int k = 0; k < WB; k++) v += sD2[k][q];
     } else if ((q -= NH) < NH) {
-      for (int k = 0; k < WB; k++) s += sDy[k] * sA2[k][q];
+      for (int k = 0; k < WB; k++) v += sDy[k] * t.a2[k][q];
     } else {
-      for (int k = 0; k < WB; k++) s += sDy[k];
+      for (int k = 0; k < WB; k++) v += sDy[k];
     }
-    atomicAdd(&grad[p], s);
+    atomicAdd(&grad[p], v);
   }
-  float l = act ? r * r / (float)B : 0.0f;
-  for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
-  if (t == 0 && loss) atomicAdd(loss, l);
+  if (g == 0) {
+    float l = act ? r * r / (float)B : 0.0f;
+    for (int o = 32; o > 0; o >>= 1) l += __shfl_xor(l, o);
+    if (s == 0) atomicAdd(loss, l);
+  }
 }
 
-// Adam update of the FP32 master weights, BF16 copy, gradient reset
+// Adam update of the FP32 master weights, BF16 copy, gradient and loss reset
 __global__ void k_mlp_adam(float* __restrict__ w, uint16_t* __restrict__ wbf, float* __restrict__ m,
-                           float* __restrict__ v, float* __restrict__ grad, float lr, float bc1, float bc2) {
+                           float* __restrict__ v, float* __restrict__ grad, float* __restrict__ loss, float lr,
+                           float bc1, float bc2) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p == 0) *loss = 0.0f;
   if (p >= MLP_NPARAM) return;
   const float g = grad[p];
   const float mm = 0.9f * m[p] + 0.1f * g;
@@ -339,21 +366,22 @@ hipError_t mlp_alloc(MlpState& s, int n) {
   if ((e = hipMalloc(&s.wbf, sizeof(uint16_t) * MLP_NPARAM))) return e;
   if ((e = hipMalloc(&s.m, sizeof(float) * MLP_NPARAM))) return e;
   if ((e = hipMalloc(&s.v, sizeof(float) * MLP_NPARAM))) return e;
-  if ((e = hipMalloc(&s.grad, sizeof(float) * MLP_NPARAM))) return e;
-  if ((e = hipMalloc(&s.loss, sizeof(float) * 4))) return e;
+  // the loss lies behind the gradient: one copy to the host takes both
+  if ((e = hipMalloc(&s.grad, sizeof(float) * (MLP_NPARAM + 1)))) return e;
+  s.loss = s.grad + MLP_NPARAM;
   if ((e = hipMalloc(&s.X, sizeof(float) * (size_t)MLP_LDX * n))) return e;
   s.nrows = n;
   hipMemset(s.w32, 0, sizeof(float) * MLP_NPARAM);
   hipMemset(s.wbf, 0, sizeof(uint16_t) * MLP_NPARAM);
   hipMemset(s.m, 0, sizeof(float) * MLP_NPARAM);
   hipMemset(s.v, 0, sizeof(float) * MLP_NPARAM);
-  hipMemset(s.grad, 0, sizeof(float) * MLP_NPARAM);
+  hipMemset(s.grad, 0, sizeof(float) * (MLP_NPARAM + 1));
   hipMemset(s.X, 0, sizeof(float) * (size_t)MLP_LDX * n);
   return hipSuccess;
 }
 
 void mlp_free(MlpState& s) {
-  void* p[] = {s.w32, s.wbf, s.m, s.v, s.grad, s.loss, s.X, s.Xext};
+  void* p[] = {s.w32, s.wbf, s.m, s.v, s.grad, s.X, s.Xext};
   for (void* q : p)
     if (q) (void)hipFree(q);
 }
@@ -364,7 +392,7 @@ hipError_t mlp_set_params(MlpState& s, const float* host, hipStream_t st) {
   hipLaunchKernelGGL(k_mlp_to_bf16, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, (const float*)s.w32, s.wbf);
   hipLaunchKernelGGL(k_mlp_fill, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, s.m, MLP_NPARAM, 0.0f);
   hipLaunchKernelGGL(k_mlp_fill, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, s.v, MLP_NPARAM, 0.0f);
-  hipLaunchKernelGGL(k_mlp_fill, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, s.grad, MLP_NPARAM, 0.0f);
+  mlp_launch_zero_grad(s, st);
   s.adam_steps = 0;
   s.have_params = 1;
   return hipGetLastError();
@@ -382,14 +410,18 @@ void mlp_launch_infer(MlpState& s, const float* X, int ldx, int B, float* y, hip
 }
 
 void mlp_launch_forward(MlpState& s, const float* X, int ldx, int B, float* y, hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_forward, dim3(nb(B, 256)), dim3(256), 0, st, (const uint16_t*)s.wbf, X, ldx, B, y);
+  hipLaunchKernelGGL(k_mlp_forward, dim3(nb(B, WB)), dim3(256), 0, st, (const uint16_t*)s.wbf, X, ldx, B, y);
 }
 
-void mlp_launch_grad(MlpState& s, const float* X, int nrows, int B, long long off, long long stride,
-                     hipStream_t st) {
-  hipLaunchKernelGGL(k_mlp_fill, dim3(1), dim3(4), 0, st, s.loss, 4, 0.0f);
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nb(B, WB)), dim3(WB), 0, st, (const uint16_t*)s.wbf, X, nrows,
-                     (int)MLP_COL_TARGET, B, off, stride, s.grad, s.loss);
+void mlp_launch_zero_grad(MlpState& s, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_fill, dim3(nb(MLP_NPARAM + 1, 256)), dim3(256), 0, st, s.grad, MLP_NPARAM + 1, 0.0f);
+}
+
+// (adds to gradient and loss: both are zero between calls)
+void mlp_launch_grad(MlpState& s, const float* X, int ldx, const float* T, int ldt, int nrows, int B, long long off,
+                     long long stride, hipStream_t st) {
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nb(B, WB)), dim3(256), 0, st, (const uint16_t*)s.wbf, X, ldx, T, ldt, nrows, B, off,
+                     stride, s.grad, s.loss);
 }
 
 void mlp_launch_adam(MlpState& s, float lr, hipStream_t st) {
@@ -397,5 +429,5 @@ void mlp_launch_adam(MlpState& s, float lr, hipStream_t st) {
   const float bc1 = 1.0f - powf(0.9f, (float)s.adam_steps);
   const float bc2 = 1.0f - powf(0.999f, (float)s.adam_steps);
   hipLaunchKernelGGL(k_mlp_adam, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, s.w32, s.wbf, s.m, s.v, s.grad,
-                     lr, bc1, bc2);
+                     s.loss, lr, bc1, bc2);
 }
