@@ -5,7 +5,7 @@
 //   k_binstats      periodic wrap / wall reflection (src/boundaryND.f90:66-160),
 //                   max h and bounding box (src/ghostND_mhd.f90:77,
 //                   linkND.f90:78-90), the cell grid
-//   k_cellid, k_scan_local, k_scatter, k_cellsort_wave
+//   k_cellid, k_scan_local, k_scatter, k_cellrank
 //                   counting sort of particles by Morton cell key, stable
 //                   by slot: replaces the head/next link lists of
 //                   set_linklist (src/linkND.f90:45-161)
@@ -439,7 +439,8 @@ __global__ __launch_bounds__(BS) void k_scan_local(KArgs a, int* bsum, const Gri
 }
 
 // the cells' starts (block offsets onto the places), their largest list radii
-// cleared (raised by k_pack_density), and every particle's slot to its place
+// cleared (raised by k_pack_density), and every particle's slot to its place in
+// the order of arrival
 __device__ __forceinline__ void b_scatter(KArgs a, const int* __restrict__ bsum, const Grid* __restrict__ gp, VL vl) {
   const long long n = gp->ncell + 1, step = (long long)vl.nb * blockDim.x;
   for (long long idx = (long long)vl.b * blockDim.x + threadIdx.x; idx < n; idx += step) {
@@ -449,7 +450,7 @@ __device__ __forceinline__ void b_scatter(KArgs a, const int* __restrict__ bsum,
   const int i = vl.b * blockDim.x + threadIdx.x;
   if (i >= a.n) return;
   const int c = a.cellid[i];
-  a.sidx[a.cpart[c] + bsum[c / (BS * 4)] + a.rank[i]] = i;
+  a.sarr[a.cpart[c] + bsum[c / (BS * 4)] + a.rank[i]] = i;
 }
 __global__ void k_scatter(KArgs a, const int* __restrict__ bsum, const Grid* __restrict__ gp) {
   b_scatter(a, bsum, gp, VL{(int)blockIdx.x, (int)gridDim.x});
@@ -474,84 +475,33 @@ __device__ __forceinline__ void sort_regs(T (&v)[N]) {
         }
       }
 }
-// cell [b, b+m) of sorted positions into ascending slot order by one lane,
-// m <= N: every entry is read before any is written back
-template <int N>
-__device__ __forceinline__ void sort_cell_lane(int* __restrict__ sidx, int b, int m) {
-  int v[N];
+// Slots of each cell into ascending order (deterministic, and a stable sort by
+// cell key overall): a particle's place is the number of smaller slots in its
+// cell, counted by its own lane.  The lanes of a cell read the same entries, so
+// the loads are broadcasts, and a wave's length follows its own cells.  The whole
+// counting sort of 128^3 with this launch takes 108 us for cells of 14 and 135 us
+// once the flow has gathered 200 to 300 particles in some; with each cell sorted
+// by a lane or by its wave in turn it took 129 us, 1.6 ms and (over 256 in a cell)
+// 14 to 42 ms.
+__device__ __forceinline__ void b_cellrank(KArgs a, VL vl) {
+  const int k = vl.b * blockDim.x + threadIdx.x;
+  if (k >= a.n) return;
+  const int i = a.sarr[k];
+  const int c = a.cellid[i];
+  const int b = a.cstart[c], e = a.cstart[c + 1];
+  int r = 0, q = b;
+  for (; q + 8 <= e; q += 8) {
+    int v[8];
 #pragma unroll
-  for (int q = 0; q < N; q++) v[q] = q < m ? sidx[b + q] : INT_MAX;
-  sort_regs<N>(v);
+    for (int u = 0; u < 8; u++) v[u] = a.sarr[q + u];
 #pragma unroll
-  for (int q = 0; q < N; q++)
-    if (q < m) sidx[b + q] = v[q];
-}
-
-// make the order inside each cell ascending in slot index (deterministic,
-// and a stable sort by cell key overall).  A lane sorts its own cell in
-// registers when the cell holds at most CS_LANE particles, or at most
-// CS_LANE2 while at least CS_LANE2_MIN cells of its wave are of that size
-// (the lanes then work side by side); the other cells are taken by the whole
-// wave in turn: a cell of at most 256 particles is ranked in registers (each
-// slot index counts the smaller ones of its cell), a larger one is
-// insertion-sorted by the first lane.
-#define CS_LANE 16
-#define CS_LANE2 64
-#define CS_LANE2_MIN 4
-__device__ __forceinline__ void b_cellsort_wave(KArgs a, const Grid* __restrict__ gp, VL vl) {
-  const long long c = (long long)vl.b * blockDim.x + threadIdx.x;
-  const int lane = threadIdx.x & 63;
-  int b = 0, m = 0;
-  if (c < gp->ncell) {
-    b = a.cstart[c];
-    m = a.cstart[c + 1] - b;
+    for (int u = 0; u < 8; u++) r += v[u] < i;
   }
-  if (m > 1 && m <= CS_LANE) sort_cell_lane<CS_LANE>(a.sidx, b, m);
-  const bool mid = m > CS_LANE && m <= CS_LANE2;
-  const bool lanes_mid = __popcll(__ballot(mid)) >= CS_LANE2_MIN;
-  if (lanes_mid && mid) sort_cell_lane<CS_LANE2>(a.sidx, b, m);
-  unsigned long long todo = __ballot(m > CS_LANE && !(lanes_mid && mid));
-  while (todo) {
-    const int src = __ffsll((long long)todo) - 1;
-    todo &= todo - 1ull;
-    const int cb = __shfl(b, src), cm = __shfl(m, src);
-    if (cm <= 256) {
-      // up to four entries per lane (positions lane + 64 q)
-      const int v0 = lane < cm ? a.sidx[cb + lane] : INT_MAX;
-      const int v1 = lane + 64 < cm ? a.sidx[cb + lane + 64] : INT_MAX;
-      const int v2 = lane + 128 < cm ? a.sidx[cb + lane + 128] : INT_MAX;
-      const int v3 = lane + 192 < cm ? a.sidx[cb + lane + 192] : INT_MAX;
-      int r0 = 0, r1 = 0, r2 = 0, r3 = 0;
-      for (int q = 0; q * 64 < cm; q++) {
-        const int vq = q == 0 ? v0 : q == 1 ? v1 : q == 2 ? v2 : v3;
-        const int nj = min(64, cm - q * 64);
-        for (int j = 0; j < nj; j++) {
-          const int u = __shfl(vq, j);
-          r0 += u < v0;
-          r1 += u < v1;
-          r2 += u < v2;
-          r3 += u < v3;
-        }
-      }
-      if (lane < cm) a.sidx[cb + r0] = v0;
-      if (lane + 64 < cm) a.sidx[cb + r1] = v1;
-      if (lane + 128 < cm) a.sidx[cb + r2] = v2;
-      if (lane + 192 < cm) a.sidx[cb + r3] = v3;
-    } else if (lane == 0) {
-      for (int k = cb + 1; k < cb + cm; k++) {
-        int v = a.sidx[k];
-        int j = k - 1;
-        while (j >= cb && a.sidx[j] > v) {
-          a.sidx[j + 1] = a.sidx[j];
-          j--;
-        }
-        a.sidx[j + 1] = v;
-      }
-    }
-  }
+  for (; q < e; q++) r += a.sarr[q] < i;
+  a.sidx[b + r] = i;
 }
-__global__ __launch_bounds__(BS) void k_cellsort_wave(KArgs a, const Grid* __restrict__ gp) {
-  b_cellsort_wave(a, gp, VL{(int)blockIdx.x, (int)gridDim.x});
+__global__ __launch_bounds__(BS) void k_cellrank(KArgs a) {
+  b_cellrank(a, VL{(int)blockIdx.x, (int)gridDim.x});
 }
 
 // ===========================================================================
@@ -3142,7 +3092,7 @@ NDSP_MK(km_predict) { NDSP_MEMBER b_predict(M.a, M.p, vl); }
 NDSP_MK(km_predict_fixed) { NDSP_MEMBER b_predict_fixed(M.a, M.p, vl); }
 NDSP_MK(km_slot_of) { NDSP_MEMBER b_slot_of(M.a, vl); }
 NDSP_MK(km_cellid) { NDSP_MEMBER b_cellid(M.a, M.gdev, vl); }
-NDSP_MK(km_cellsort) { NDSP_MEMBER b_cellsort_wave(M.a, M.gdev, vl); }
+NDSP_MK(km_cellrank) { NDSP_MEMBER b_cellrank(M.a, vl); }
 NDSP_MK(km_fixed_copy) { NDSP_MEMBER b_fixed_copy(M.a, M.p, 1, vl); }
 NDSP_MK(km_binstats) { NDSP_MEMBER b_binstats(M.a, M.p, M.box, M.gdev, 1, M.cap_bits, M.part, vl); }
 NDSP_MK(km_scan_local) { NDSP_MEMBER b_scan_local(M.a, M.bsum, M.gdev, vl); }
@@ -3549,14 +3499,13 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
     c->density_ready = true;
   }
   const long long cap = (1LL << c->cap_bits) + 1;
-  const unsigned cap_blocks = (unsigned)std::min<long long>(nblk(cap), 1 << 20);
   {
     TScope t(c, "cellsort");
     const unsigned nbs = (unsigned)((cap + BS * 4 - 1) / (BS * 4));
     hipLaunchKernelGGL(k_cellid, dim3(nblk(n)), dim3(BS), 0, c->st, a, (const Grid*)c->gdev);
     hipLaunchKernelGGL(k_scan_local, dim3(nbs), dim3(BS), 0, c->st, a, c->bsum, (const Grid*)c->gdev);
     hipLaunchKernelGGL(k_scatter, dim3(nblk(n)), dim3(BS), 0, c->st, a, (const int*)c->bsum, (const Grid*)c->gdev);
-    hipLaunchKernelGGL(k_cellsort_wave, dim3(cap_blocks), dim3(BS), 0, c->st, a, (const Grid*)c->gdev);
+    hipLaunchKernelGGL(k_cellrank, dim3(nblk(n)), dim3(BS), 0, c->st, a);
   }
   {
     TScope t(c, "pack_density");
@@ -3942,7 +3891,9 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   ok &= hipMalloc(&c->list_b, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.nrflag, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.nrcnt, sizeof(int) * (size_t)nblk(n, 64)) == hipSuccess;
-  a.rank = c->list_a;  // free during a binning: the h-rho passes come after it
+  // free during a binning: the h-rho passes come after it
+  a.rank = c->list_a;
+  a.sarr = c->list_b;
   if (ok) ok &= hipMemset(a.nrflag, 0, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.P4, sizeof(double4) * n) == hipSuccess;
   ok &= hipMalloc(&a.dxb, sizeof(double) * n) == hipSuccess;
@@ -4358,7 +4309,7 @@ struct BGroup {
   std::vector<int> mem;
   MArgs* args = nullptr;
   // workgroup offsets per launch shape (device; nm + 1 entries each)
-  enum { S_256, S_64, S_ONE, S_BIN, S_FILL, S_SCAN, S_CAP, S_NR, S_FORCE, S_HMAX, NSHAPE };
+  enum { S_256, S_64, S_ONE, S_BIN, S_SCAN, S_NR, S_FORCE, NSHAPE };
   int* off[NSHAPE] = {};
   int tot[NSHAPE] = {};
   int* due = nullptr;  // members whose periodic reorder is due (device, nm entries)
@@ -4442,7 +4393,6 @@ static int batch_build(ndsp_batch* b) {
       ndsp_ctx* c = b->sims[g.mem[q]];
       const int n = c->n;
       const long long cap = (1LL << c->cap_bits) + 1;
-      const int capb = (int)std::min<long long>(nblk(cap), 1 << 20);
       MArgs& M = ma[q];
       memset(&M, 0, sizeof(M));
       M.a = c->a;
@@ -4462,9 +4412,8 @@ static int batch_build(ndsp_batch* b) {
       M.nb_256 = (int)nblk(n);
       M.scratch_d = c->scratch_d;
       M.scratch_i = c->scratch_i;
-      const int cnt[BGroup::NSHAPE] = {(int)nblk(n), (int)nblk(n, 64), 1, M.nbp, std::min(capb, 4096),
-                                       (int)((cap + BS * 4 - 1) / (BS * 4)), capb, M.nb_nr, M.nb_force,
-                                       (int)std::min(1024u, nblk(n))};
+      const int cnt[BGroup::NSHAPE] = {(int)nblk(n), (int)nblk(n, 64), 1, M.nbp,
+                                       (int)((cap + BS * 4 - 1) / (BS * 4)), M.nb_nr, M.nb_force};
       for (int k = 0; k < BGroup::NSHAPE; k++) off[k].push_back(off[k].back() + cnt[k]);
     }
     HIPCHK(hipMalloc((void**)&g.due, sizeof(int) * nm));
@@ -4516,7 +4465,7 @@ static int batch_part_a(ndsp_batch* b) {
     BLAUNCH(km_cellid, g, BGroup::S_256, BS);
     BLAUNCH(km_scan_local, g, BGroup::S_SCAN, BS);
     BLAUNCH(km_scatter, g, BGroup::S_256, BS);
-    BLAUNCH(km_cellsort, g, BGroup::S_CAP, BS);
+    BLAUNCH(km_cellrank, g, BGroup::S_256, BS);
     if (fp64) BLAUNCH(km_pack_density<double>, g, BGroup::S_256, BS);
     else BLAUNCH(km_pack_density<float>, g, BGroup::S_256, BS);
     if (g.lists) {

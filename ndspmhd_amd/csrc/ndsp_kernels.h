@@ -111,6 +111,7 @@ struct KArgs {
   int* cfill;         // ncell
   float* cellr;       // ncell: largest list radius of a cell's particles (null without lists)
   int* rank;          // per slot: place among its cell's particles, in order of arrival
+  int* sarr;          // slots by cell, in order of arrival within each
   int* cpart;         // ncell + 1: the cells' starts within their scan block
   int* nrflag;        // unconverged after a pass, by place in the pass's list
   int* nrcnt;         // per tile of a pass: unconverged particles, then their offset
