@@ -189,7 +189,9 @@ int ndsp_autotune(ndsp_ctx *ctx, int32_t reps, int32_t *choice);
 
 /* Sets the tile shapes the autotuner chooses among (no counterpart in the
  * reference): force and h-rho workgroup sizes (64 or 256) and cells per
- * search radius (1 or 2), e.g. a choice kept from an earlier autotune. */
+ * search radius (1 or 2), e.g. a choice kept from an earlier autotune.  The h-rho
+ * passes of a simulation of at most 65536 particles, and those force passes that
+ * use four lanes per particle, keep their own workgroup of 256. */
 int ndsp_set_tile_shapes(ndsp_ctx *ctx, int32_t force_wg, int32_t density_wg,
                          int32_t cells_per_radius);
 
