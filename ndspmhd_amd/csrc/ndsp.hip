@@ -3240,10 +3240,12 @@ static const size_t PIN_REALS = 40960;
 // between the lanes cost more than the shorter walks give.
 static const int64_t QUAD_MAX = 65536;
 // The force pass does too where its results are those of one lane per particle
-// bit for bit (1D, hydro, dust) or to FP64 rounding.  In mixed 2D and 3D MHD the
-// compiler contracts the pair's dot products differently in the two kernels; an
-// FP32 last bit there decides, steps later, whether single particles' h
-// iterations end at tolh, so those runs keep one lane.
+// bit for bit (hydro, dust, 1D MHD between reflecting walls, which scans cells)
+// or to FP64 rounding.  In mixed 2D and 3D MHD, and in 1D MHD over lists, the
+// compiler contracts the pair's dot products differently in the two kernels (1D
+// tubes with fixed walls: velocities 2e-7 apart after 40 steps); an FP32 last
+// bit there decides, steps later, whether single particles' h iterations end at
+// tolh, so those runs keep one lane.
 static constexpr bool quad_force_ok(int ndim, int phys, bool fp64) { return fp64 || phys != 1 || ndim == 1; }
 
 struct ndsp_ctx {
@@ -3866,7 +3868,8 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   c->g.ndim = p.ndim;
   c->reflect = nrefl > 0;
   c->quad = npart <= QUAD_MAX;
-  c->quad_force = c->quad && quad_force_ok(p.ndim, fr_phys(p), precision == NDSP_PREC_FP64);
+  c->quad_force = c->quad && quad_force_ok(p.ndim, fr_phys(p), precision == NDSP_PREC_FP64) &&
+                  (precision == NDSP_PREC_FP64 || fr_phys(p) != 1 || !p.use_list);
   c->dt = dopt[23];
   c->time = 0.0;
   auto cleanup_fail = [&](int e) { ndsp_destroy(c); return e; };
