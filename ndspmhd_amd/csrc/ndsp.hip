@@ -3290,7 +3290,10 @@ struct ndsp_ctx {
   double* cons_out = nullptr;   // pinned host memory: the kernels write their results there
   DScal* hs = nullptr;          // pinned host copy of the scalars
   double* pin = nullptr;        // pinned staging of small downloads (PIN_REALS reals at most)
-  bool density_ready = false;   // the binning has just set the scalars of the h-rho iteration
+  // the last binning set the scalars of the h-rho iteration and nothing has
+  // iterated on them since (a recorded step does both on the device alone:
+  // its launch clears this)
+  bool density_ready = false;
   int nb_part = 0;
   Grid g;
   bool grid_valid = false;
@@ -4269,6 +4272,7 @@ int ndsp_step(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dtout) {
     // both halves at once: the second holds back while the iteration is
     // unfinished, and is then launched again once the host has finished it (one
     // wait a step instead of two)
+    c->density_ready = false;
     HIPCHK(hipGraphLaunch(c->graph_a, c->st));
     HIPCHK(hipGraphLaunch(c->graph_b, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
@@ -4657,6 +4661,7 @@ int ndsp_batch_step(ndsp_batch* b, ndsp_stats* stats, ndsp_dt* dt) {
   // both halves at once: members whose iteration needs more passes than
   // recorded hold back in the second, which is launched again once the host
   // has finished them (the others have ended their step and do nothing then)
+  for (ndsp_ctx* c : b->sims) c->density_ready = false;
   HIPCHK(hipGraphLaunch(b->ga, b->st));
   HIPCHK(hipGraphLaunch(b->gb, b->st));
   HIPCHK(hipStreamSynchronize(b->st));

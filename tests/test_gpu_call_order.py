@@ -1,0 +1,48 @@
+"""The library's calls in orders a host may use them in: what one call leaves
+behind on the host must not stand in for what another has done on the device
+since.  Each sequence runs against the launch-by-launch path."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ("x", "vel", "Bevol", "en", "hh", "rho", "force", "dBevoldt", "dudt", "numneigh", "nits", "slot")
+
+
+def _same(a, b, where):
+    for k in FIELDS:
+        assert np.array_equal(a.get(k), b.get(k)), (where, k)
+
+
+@pytest.mark.parametrize("setup", ["box", "tube"])
+@pytest.mark.parametrize("batch", [False, True])
+def test_density_after_binning_and_recorded_step(setup, batch):
+    """set_linklist, a recorded step, then iterate_density and get_rates: the
+    step has used up the binning's scalars, so the iteration sets them anew and
+    works on the corrected state, as it does after a launch-by-launch step"""
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import brio_wu_1d, periodic_mhd_box
+    o, st = periodic_mhd_box(11, seed=3, vel_seed=4, vrms=0.5) if setup == "box" else brio_wu_1d(300)
+    print("density after a recorded step:", setup, "batch" if batch else "alone", flush=True)
+    eager, sim = nd.Simulation(o, st, precision=1), nd.Simulation(o, st, precision=1)
+    if batch:
+        b = nd.Batch([sim])
+        step = b.step
+    else:
+        sim.set_graph(True)
+        step = sim.step
+    for s in range(3):
+        eager.step()
+        step()
+    eager.set_linklist()
+    sim.set_linklist()
+    eager.step()
+    step()
+    _same(eager, sim, "step")
+    before = sim.get("rho")
+    assert eager.iterate_density() == sim.iterate_density()
+    assert sim.stats["itsdensity"] >= 1 and not np.array_equal(before, sim.get("rho"))
+    assert eager.get_rates() == sim.get_rates()
+    _same(eager, sim, "rates")
+    if batch:
+        b.close()
