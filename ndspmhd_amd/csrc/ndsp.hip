@@ -3692,9 +3692,11 @@ static void fill_outputs(ndsp_ctx* c, const DScal& h, ndsp_stats* stats, ndsp_dt
 
 // Permutes the persistent per-particle state into the cell order of the last
 // binning (slot k <- sorted position k), so that per-particle accesses of the
-// pair kernels stay spatially coherent.  Each field is gathered into scratch
-// and copied back: the field pointers never change, so launch parameters
-// recorded earlier (a captured step graph) stay valid.
+// pair kernels stay spatially coherent.  Each field is gathered into its array
+// of the second set and the sets trade places, recorded steps with them (each
+// set has its own); where that set is not there, and for members of a batch,
+// whose argument tables hold the addresses, it is gathered into scratch and
+// copied back.
 static int reorder(ndsp_ctx* c) {
   KArgs& a = c->a;
   const int n = c->n;
@@ -4274,6 +4276,7 @@ int ndsp_step(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dtout) {
     // wait a step instead of two)
     c->density_ready = false;
     HIPCHK(hipGraphLaunch(c->graph_a, c->st));
+    c->grid_valid = true;  // binned, as do_linklist leaves it (a reorder before the step took it back)
     HIPCHK(hipGraphLaunch(c->graph_b, c->st));
     HIPCHK(hipStreamSynchronize(c->st));
     if (!c->hs->pc_done) {
