@@ -3273,6 +3273,7 @@ struct ndsp_ctx {
   bool falt_failed = false;
   bool in_batch = false;
   bool alt_graph_valid = false;
+  unsigned generation = 0;  // counts what makes recorded launches stale (invalidate_graphs)
   hipGraphExec_t alt_graph_a = nullptr, alt_graph_b = nullptr;
   Phys p;
   int prec;
@@ -3314,8 +3315,10 @@ struct ndsp_ctx {
   int nev = 0;
 };
 
-// recorded steps hold field addresses and launch shapes: both sets' go stale
+// recorded steps hold field addresses and launch shapes: both sets' go stale,
+// and so do the recorded steps of the batches this context is a member of
 static void invalidate_graphs(ndsp_ctx* c) {
+  c->generation++;
   c->graph_valid = false;
   c->alt_graph_valid = false;
 }
@@ -3439,6 +3442,9 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
   bits = std::min(28, bits);
   if (bits == c->cap_bits) return 0;
   const long long cap = (1LL << bits) + 1;
+  // from here on nothing is sized: a failed allocation leaves it so
+  c->cap_bits = 0;
+  invalidate_graphs(c);
   if (c->a.cstart) hipFree(c->a.cstart);
   if (c->a.cfill) hipFree(c->a.cfill);
   if (c->bsum) hipFree(c->bsum);
@@ -3454,7 +3460,6 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
   HIPCHK(hipMalloc(&c->bsum, sizeof(int) * (cap / (BS * 4) + 2)));
   if (c->p.use_list) HIPCHK(hipMalloc(&c->a.cellr, sizeof(float) * cap));
   c->cap_bits = bits;
-  invalidate_graphs(c);
   return 0;
 }
 
@@ -4331,8 +4336,7 @@ struct ndsp_batch {
   hipGraphExec_t ga = nullptr, gb = nullptr;
   bool valid = false;
   DScal* hs = nullptr;               // pinned host copies of every member's scalars
-  std::vector<int> caps;             // members' key-space sizes at recording
-  std::vector<int> nbcaps;           // members' list capacities at recording
+  std::vector<unsigned> gens;        // members' generations at recording
   std::vector<hipStream_t> gst;      // streams of the groups after the first (recording only)
   std::vector<hipEvent_t> gev;       // fork event, then one join event per further group
   std::vector<BGroup> groups;
@@ -4644,19 +4648,17 @@ int ndsp_batch_step(ndsp_batch* b, ndsp_stats* stats, ndsp_dt* dt) {
     if (int e = ensure_key_space(c)) return e;
     due[s] = c->grid_valid && c->reorder_every > 0 && (c->nsteps % c->reorder_every == 0 || c->reorder_next);
     if (due[s]) c->reorder_next = false;
-    if (b->caps.size() != (size_t)ns || b->caps[s] != c->cap_bits || b->nbcaps[s] != c->a.maxnb) b->valid = false;
+    // (sizes alone do not tell: arrays allocated again may have the old size
+    // at another address, and the argument tables hold addresses)
+    if (b->gens.size() != (size_t)ns || b->gens[s] != c->generation) b->valid = false;
   }
   for (int s = 0; s < ns; s++) HIPCHK(hipStreamSynchronize(b->sims[s]->st));
   if (!b->valid) {
     if (int e = batch_build(b)) return e;
     if (int e = batch_capture(b, b->ga, batch_part_a)) return e;
     if (int e = batch_capture(b, b->gb, batch_part_b)) return e;
-    b->caps.resize(ns);
-    b->nbcaps.resize(ns);
-    for (int s = 0; s < ns; s++) {
-      b->caps[s] = b->sims[s]->cap_bits;
-      b->nbcaps[s] = b->sims[s]->a.maxnb;
-    }
+    b->gens.resize(ns);
+    for (int s = 0; s < ns; s++) b->gens[s] = b->sims[s]->generation;
     b->valid = true;
   }
   if (std::find(due.begin(), due.end(), 1) != due.end())

@@ -73,3 +73,34 @@ def test_recorded_steps_keep_reordering(setup, prec):
     if setup == "box":
         # (the flow moves particles between cells, so the orders differ)
         assert all(not np.array_equal(a, b) for a, b in zip(slots[1:], slots[2:]))
+
+
+@pytest.mark.parametrize("how", ["tile shapes", "autotune"])
+def test_batch_after_member_reallocates(how):
+    """a member's cell arrays are allocated again between batch steps, at the
+    size they had: the batch records its steps anew and the members stay those
+    stepped one by one bit for bit"""
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import brio_wu_1d, periodic_mhd_box, shock_tube_2d
+    cfg = [brio_wu_1d(300), shock_tube_2d(600), periodic_mhd_box(9, seed=3, vel_seed=4), brio_wu_1d(500)]
+    members = [nd.Simulation(o, st, precision=1) for o, st in cfg]
+    alone = [nd.Simulation(o, st, precision=1) for o, st in cfg]
+    batch = nd.Batch(members)
+    for s in range(9):
+        if s in (2, 5, 7):
+            print("member arrays again:", how, "before step", s, flush=True)
+            for k in ((0, 1, 2, 3) if s == 7 else (s % 4, (s + 1) % 4)):
+                if how == "tile shapes":
+                    shapes = (64, 256, 2)
+                else:
+                    c = members[k].autotune(reps=1)
+                    shapes = (c["force_workgroup"], c["density_workgroup"], c["cells_per_radius"])
+                    alone[k].autotune(reps=1)
+                members[k].set_tile_shapes(*shapes)
+                alone[k].set_tile_shapes(*shapes)
+        batch.step()
+        for k, (m, a) in enumerate(zip(members, alone)):
+            a.step()
+            _same(a, m, (s, k))
+            assert m.stats == a.stats and m.dt_info == a.dt_info
+    batch.close()
