@@ -3291,6 +3291,12 @@ struct ndsp_ctx {
   double* cons_out = nullptr;   // pinned host memory: the kernels write their results there
   DScal* hs = nullptr;          // pinned host copy of the scalars
   double* pin = nullptr;        // pinned staging of small downloads (PIN_REALS reals at most)
+  // what a step's binning had too little room for, made before the next
+  // binning: until then the grid, its cells and the lists stay for the calls
+  // that read them (iterate_density, get_rates, neighbours)
+  bool grow_key = false;   // key space, from the statistics in grow_from
+  bool grow_nbl = false;   // list rows
+  DScal grow_from;
   // the last binning set the scalars of the h-rho iteration and nothing has
   // iterated on them since (a recorded step does both on the device alone:
   // its launch clears this)
@@ -3466,8 +3472,7 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
 // List capacity after a binning in which some rows overflowed (those
 // particles scanned cells, the slowest part of their launch): 1.5 times the
 // present one, up to four times the initial capacity; the old lists are
-// dropped (the next binning rebuilds them) and recorded steps are recorded
-// again.  A failed allocation keeps the present capacity for good.
+// dropped (a binning follows) and recorded steps are recorded again.  A failed allocation keeps the present capacity for good.
 static int grow_lists(ndsp_ctx* c) {
   if (!c->p.use_list || c->a.maxnb >= c->maxnb_limit) return 0;
   const int m = std::min(c->maxnb_limit, (c->a.maxnb * 3 / 2 + 31) / 32 * 32);
@@ -3485,6 +3490,23 @@ static int grow_lists(ndsp_ctx* c) {
   return 0;
 }
 
+// notes what the step that left the scalars h lacked room for
+static void note_growth(ndsp_ctx* c, const DScal& h) {
+  if (h.grid_clamped && c->cap_bits < 28) {
+    c->grow_key = true;
+    c->grow_from = h;
+  }
+  if (h.list_overflow) c->grow_nbl = true;
+}
+// makes that room; the caller bins next
+static int apply_growth(ndsp_ctx* c) {
+  const bool key = c->grow_key && c->cap_bits > 0, nbl = c->grow_nbl;
+  c->grow_key = c->grow_nbl = false;
+  if (key)
+    if (int e = size_key_space(c, c->grow_from, 2)) return e;
+  return nbl ? grow_lists(c) : 0;
+}
+
 // Binning (set_linklist, src/linkND.f90:45): wrap, statistics, device-side
 // grid, counting sort by Morton cell key, packed views, neighbour lists.
 // No host round trip except the first call, which sizes the key space.
@@ -3492,6 +3514,8 @@ static int do_linklist(ndsp_ctx* c, int in_step) {
   KArgs& a = c->a;
   const int n = c->n;
   if (!c->ireal_set) return set_err(NDSP_ERR_BAD_ARG, "fixed particles need their partners: call ndsp_set_ireal");
+  if (!c->capturing)
+    if (int e = apply_growth(c)) return e;
   {
     // wrap, statistics, grid and the iteration's scalars in one launch; the
     // first binning sizes the key space from the statistics in between
@@ -4268,6 +4292,7 @@ int ndsp_step(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dtout) {
     if (int e = reorder(c)) return e;
     c->reorder_next = false;
   }
+  if (int e = apply_growth(c)) return e;
   if (graph_usable(c) && c->cap_bits > 0) {
     // the step as two recorded graphs; the h-rho iteration is completed on
     // the host path in between when it needs more passes than recorded
@@ -4299,10 +4324,7 @@ int ndsp_step(ndsp_ctx* c, ndsp_stats* stats, ndsp_dt* dtout) {
   c->time = hs.time;
   c->dt = hs.dt_cur;
   c->nsteps++;
-  if (hs.grid_clamped && c->cap_bits < 28)
-    if (int e = size_key_space(c, hs, 2)) return e;
-  if (hs.list_overflow)
-    if (int e = grow_lists(c)) return e;
+  note_growth(c, hs);
   if (c->mlp.enabled) c->mlp.steps_seen++;
   fill_outputs(c, hs, stats, dtout);
   return check_err(c, hs);
@@ -4645,6 +4667,7 @@ int ndsp_batch_step(ndsp_batch* b, ndsp_stats* stats, ndsp_dt* dt) {
       return set_err(NDSP_ERR_BAD_OPTION, "batch_step: members may not time kernels or use the h predictor");
     if (!c->have_rates)
       if (int e = ndsp_derivs(c, nullptr, nullptr)) return e;
+    if (int e = apply_growth(c)) return e;
     if (int e = ensure_key_space(c)) return e;
     due[s] = c->grid_valid && c->reorder_every > 0 && (c->nsteps % c->reorder_every == 0 || c->reorder_next);
     if (due[s]) c->reorder_next = false;
@@ -4691,10 +4714,7 @@ int ndsp_batch_step(ndsp_batch* b, ndsp_stats* stats, ndsp_dt* dt) {
     c->time = hs.time;
     c->dt = hs.dt_cur;
     c->nsteps++;
-    if (hs.grid_clamped && c->cap_bits < 28)
-      if (int e = size_key_space(c, hs, 2)) return e;
-    if (hs.list_overflow)
-      if (int e = grow_lists(c)) return e;
+    note_growth(c, hs);
     fill_outputs(c, hs, stats ? stats + s : nullptr, dt ? dt + s : nullptr);
     const int e = check_err(c, hs);
     if (e && !first_err) first_err = e;

@@ -104,3 +104,69 @@ def test_batch_after_member_reallocates(how):
             _same(a, m, (s, k))
             assert m.stats == a.stats and m.dt_info == a.dt_info
     batch.close()
+
+
+def _rows(a):
+    return a[np.lexsort(a.T[::-1])]
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_lists_usable_after_a_step_that_overflowed(graph):
+    """a step in which list rows overflowed makes longer ones before the next
+    binning, not at once: its grid and lists still serve iterate_density,
+    get_rates and neighbours, which equal the cell scan's to round-off (1e-12,
+    as the other list tests)"""
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import periodic_mhd_box
+    o, st = periodic_mhd_box(12, seed=7, vel_seed=8, vrms=0.3)
+    st["hh"][np.random.default_rng(9).choice(st["hh"].size, 30, replace=False)] *= 2.5
+    o = o.replace(maxdensits=0)
+    print("calls after a step with overflowed rows, graph", graph, flush=True)
+    sim, scan = nd.Simulation(o, st, precision=1), nd.Simulation(o.replace(cellscan=1), st, precision=1)
+    for s in (sim, scan):
+        s.set_graph(graph)
+        for k in range(3):
+            s.step()
+            if s is sim and k == 0:
+                over = int((s.get("nblist_len") < 0).sum())
+                print("overflowed rows", over, flush=True)
+                assert over
+            s.iterate_density()
+            s.get_rates()
+    assert np.array_equal(_rows(sim.neighbours()), _rows(scan.neighbours()))
+    for k in ("rho", "force", "dBevoldt", "dudt"):
+        a, b = sim.get(k), scan.get(k)
+        assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b)), k
+
+
+@pytest.mark.parametrize("graph", [False, True])
+def test_grid_usable_after_a_step_that_clamped_it(graph):
+    """a state with much smaller h than the key space was sized for: the first
+    step widens the cells and the key space grows before the next binning; the
+    step's grid serves the calls in between, and neighbours and rates equal
+    those of a context sized for the state (1e-12: other cells, other order)"""
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import periodic_mhd_box
+    o, st = periodic_mhd_box(12, seed=7, vel_seed=8, vrms=0.3)
+    o = o.replace(maxdensits=0)
+    wide = dict(st, hh=st["hh"] * 4.0)
+    narrow = dict(st, hh=st["hh"] * 0.7)
+    print("calls after a step with widened cells, graph", graph, flush=True)
+    sim, ref = nd.Simulation(o, wide, precision=1), nd.Simulation(o, narrow, precision=1)
+    for s in (sim, ref):
+        s.set_tile_shapes(256, 256, 1)
+        s.set_graph(graph)
+        s.derivs()
+    sim.upload(narrow)
+    sim.derivs()
+    for _ in range(3):
+        for s in (sim, ref):
+            s.set_dt(1e-3)
+            s.step()
+        assert np.array_equal(_rows(sim.neighbours(sym=True)), _rows(ref.neighbours(sym=True)))
+        for s in (sim, ref):
+            s.iterate_density()
+            s.get_rates()
+        for k in ("rho", "force", "dBevoldt", "dudt"):
+            a, b = sim.get(k), ref.get(k)
+            assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b)), k
