@@ -2941,6 +2941,21 @@ __global__ void k_split3(const double* __restrict__ in, double* __restrict__ o0,
   o1[i] = w > 1 ? r[1] : 0.0;
   o2[i] = w > 2 ? r[2] : 0.0;
 }
+// a context before its first upload: every index that a download follows
+// stays within the particles (slots in caller order, no lists yet)
+__global__ void k_init_ids(KArgs a) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= a.n) return;
+  a.uid[i] = i;
+  a.slot_of[i] = i;
+  a.sidx[i] = i;
+  a.ireal[i] = -1;
+  a.itype[i] = 0;
+  if (a.nbc) {
+    a.nbc[i] = -1;
+    a.nbx[i] = 0;
+  }
+}
 // what an upload leaves besides the caller's arrays: slots in caller order,
 // no partners yet, Bfield and the dust fraction of the evolved state, every
 // derived field and rate zero
@@ -3990,6 +4005,7 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   hipMemcpy(a.sc, &hs, sizeof(DScal), hipMemcpyHostToDevice);
   hipMemset(a.numneigh, 0, sizeof(int) * n);
   hipMemset(a.nits, 0, sizeof(int) * n);
+  hipLaunchKernelGGL(k_init_ids, dim3(nblk(n)), dim3(BS), 0, c->st, a);
   if (hipDeviceSynchronize() != hipSuccess) return cleanup_fail(set_err(NDSP_ERR_HIP, "init sync"));
   *out = c;
   return 0;

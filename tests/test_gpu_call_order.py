@@ -170,3 +170,30 @@ def test_grid_usable_after_a_step_that_clamped_it(graph):
         for k in ("rho", "force", "dBevoldt", "dudt"):
             a, b = sim.get(k), ref.get(k)
             assert np.max(np.abs(a - b)) <= 1e-12 * np.max(np.abs(b)), k
+
+
+@pytest.mark.parametrize("n", [1, 65, 40000])
+def test_download_before_upload(n):
+    """a context that holds no state yet gives fields of zeros in the caller's
+    order (small ones through pinned memory, large ones through device memory)
+    and no lists"""
+    import ctypes
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import periodic_mhd_box
+    o, _ = periodic_mhd_box(4)
+    L = nd.load_library()
+    iopt, dopt = np.ascontiguousarray(o.iopt(), dtype=np.int32), np.ascontiguousarray(o.dopt(), dtype=np.float64)
+    h, w = ctypes.c_void_p(), ctypes.c_int32()
+    as_p = lambda a, t: a.ctypes.data_as(ctypes.POINTER(t))
+    assert L.ndsp_create(as_p(iopt, ctypes.c_int32), as_p(dopt, ctypes.c_double), n, 1, ctypes.byref(h)) == 0
+    print("download before upload", n, flush=True)
+    want = {"x": 0.0, "vel": 0.0, "rho": 0.0, "numneigh": 0.0, "nblist_len": -1.0, "slot": np.arange(n)}
+    for k, v in want.items():
+        out = np.full(3 * n, 7.0)
+        assert L.ndsp_download(h, k.encode(), as_p(out, ctypes.c_double), ctypes.byref(w)) == 0
+        assert w.value == (3 if k in ("x", "vel") else 1)
+        assert np.array_equal(out[:w.value * n], np.broadcast_to(v, w.value * n)), k
+        assert np.all(out[w.value * n:] == 7.0)
+    # what needs a state says so
+    assert L.ndsp_iterate_density(h, None) != 0 and L.ndsp_get_rates(h, None) != 0
+    assert L.ndsp_destroy(h) == 0
