@@ -20,6 +20,7 @@ struct MlpState {
   float* v = nullptr;
   float* grad = nullptr;    // gradient, then the loss
   float* loss = nullptr;
+  bool grad_zero = false;   // both are zero on the device (in stream order)
   float* X = nullptr;       // per-particle feature rows [n][MLP_LDX]
   float* Xext = nullptr;    // caller batches: 6 features, then the target, then the output of every row
   int nrows = 0;

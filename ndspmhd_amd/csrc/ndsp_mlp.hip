@@ -415,11 +415,15 @@ void mlp_launch_forward(MlpState& s, const float* X, int ldx, int B, float* y, h
 
 void mlp_launch_zero_grad(MlpState& s, hipStream_t st) {
   hipLaunchKernelGGL(k_mlp_fill, dim3(nb(MLP_NPARAM + 1, 256)), dim3(256), 0, st, s.grad, MLP_NPARAM + 1, 0.0f);
+  s.grad_zero = true;
 }
 
-// (adds to gradient and loss: both are zero between calls)
+// (adds to gradient and loss, which a training step or mlp_launch_zero_grad
+// leaves zero; a caller that returned early, on an error, left its sums)
 void mlp_launch_grad(MlpState& s, const float* X, int ldx, const float* T, int ldt, int nrows, int B, long long off,
                      long long stride, hipStream_t st) {
+  if (!s.grad_zero) mlp_launch_zero_grad(s, st);
+  s.grad_zero = false;
   hipLaunchKernelGGL(k_mlp_grad, dim3(nb(B, WB)), dim3(256), 0, st, (const uint16_t*)s.wbf, X, ldx, T, ldt, nrows, B, off,
                      stride, s.grad, s.loss);
 }
@@ -430,4 +434,5 @@ void mlp_launch_adam(MlpState& s, float lr, hipStream_t st) {
   const float bc2 = 1.0f - powf(0.999f, (float)s.adam_steps);
   hipLaunchKernelGGL(k_mlp_adam, dim3(nb(MLP_NPARAM, 256)), dim3(256), 0, st, s.w32, s.wbf, s.m, s.v, s.grad,
                      s.loss, lr, bc1, bc2);
+  s.grad_zero = true;
 }

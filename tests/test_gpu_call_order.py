@@ -197,3 +197,45 @@ def test_download_before_upload(n):
     # what needs a state says so
     assert L.ndsp_iterate_density(h, None) != 0 and L.ndsp_get_rates(h, None) != 0
     assert L.ndsp_destroy(h) == 0
+
+
+def _leave_hip_error():
+    """an invalid device number, refused by the HIP runtime, leaves its error
+    for the next hipGetLastError of this thread"""
+    import ctypes
+    with open("/proc/self/maps") as f:
+        path = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    assert ctypes.CDLL(path).hipSetDevice(99999) != 0
+
+
+def test_gradient_after_an_early_return():
+    """a gradient call that returned on an error after its launch (here one
+    that another HIP call had left) leaves sums on the device; the next
+    gradient or training call starts from zero all the same (gradients of one
+    block of rows: one atomic per parameter, so equal bit for bit)"""
+    import ndspmhd_amd as nd
+    from ndspmhd_amd.setups import periodic_mhd_box
+    o, st = periodic_mhd_box(6)
+    rng = np.random.default_rng(5)
+    X, T = rng.standard_normal((64, 6)).astype(np.float32), rng.standard_normal(64).astype(np.float32)
+    p = (0.3 * rng.uniform(-1, 1, nd.MLP_NPARAM)).astype(np.float32)
+    sim, ref = nd.Simulation(o, st), nd.Simulation(o, st)
+    for s in (sim, ref):
+        s.mlp_set_params(p)
+    want = ref.mlp_grad(X, T)
+    print("gradient after an early return", flush=True)
+    for call in (lambda: sim.mlp_grad(X, T), lambda: sim.mlp_train(X, T, 1, 1e-3)):
+        _leave_hip_error()
+        with pytest.raises(nd.NdspError):
+            call()
+        sim.mlp_set_params(p)
+    _leave_hip_error()
+    with pytest.raises(nd.NdspError):
+        sim.mlp_grad(X, T)
+    got = sim.mlp_grad(X, T)
+    assert got[0] == want[0] and np.array_equal(got[1], want[1])
+    _leave_hip_error()
+    with pytest.raises(nd.NdspError):
+        sim.mlp_grad(X, T)
+    assert sim.mlp_train(X, T, 1, 1e-3) == ref.mlp_train(X, T, 1, 1e-3)
+    assert np.array_equal(sim.mlp_get_params()[0], ref.mlp_get_params()[0])
