@@ -183,8 +183,10 @@ int ndsp_kernel_times(ndsp_ctx *ctx, double *ms, int32_t cap, int32_t *n,
 /* Autotuner (no counterpart in the reference): times `reps` derivs
  * evaluations for each tile shape -- workgroup size of the force and h-rho
  * kernels (64 or 256) and cells per search radius of the binning (1 or 2) --
- * and keeps the fastest; choice[3] (may be NULL) receives them.  The evolved
- * state is restored afterwards, so results do not change. */
+ * and keeps the fastest; choice[3] (may be NULL) receives them.  Kernels with
+ * one workgroup size (see ndsp_set_tile_shapes) are not tried at another; 256
+ * is reported for them.  The evolved state is restored afterwards, so results
+ * do not change. */
 int ndsp_autotune(ndsp_ctx *ctx, int32_t reps, int32_t *choice);
 
 /* Sets the tile shapes the autotuner chooses among (no counterpart in the

@@ -4399,8 +4399,8 @@ static void batch_free_groups(ndsp_batch* b) {
   b->groups.clear();
 }
 
-// groups, per-member launch arguments and workgroup offsets of every shape
-static int batch_build(ndsp_batch* b) {
+// the members' groups
+static void batch_group(ndsp_batch* b) {
   batch_free_groups(b);
   const int ns = (int)b->sims.size();
   for (int s = 0; s < ns; s++) {
@@ -4433,6 +4433,11 @@ static int batch_build(ndsp_batch* b) {
   // the last bit.
   for (auto& g : b->groups)
     if (b->prec != NDSP_PREC_FP64 && g.total > QUAD_MAX) g.quad = g.quad_force = 0;
+}
+
+// groups, per-member launch arguments and workgroup offsets of every shape
+static int batch_build(ndsp_batch* b) {
+  batch_group(b);
   while (b->gst.size() + 1 < b->groups.size()) {
     hipStream_t st = nullptr;
     HIPCHK(hipStreamCreate(&st));
@@ -4843,12 +4848,14 @@ int ndsp_autotune(ndsp_ctx* c, int32_t reps, int32_t* choice) {
   hipEvent_t e0, e1;
   hipEventCreate(&e0);
   hipEventCreate(&e1);
+  // (kernels with four lanes per particle have one workgroup size, 256: where
+  // they run there is nothing to choose)
   const int tbs[2] = {64, 256}, subs[2] = {1, 2};
   double best = 1e300;
   int bf = c->tb_force, bn = c->tb_nr, bc = c->p.cell_sub;
   int err = 0;
-  for (int a = 0; a < 2 && !err; a++)
-    for (int b = 0; b < 2 && !err; b++)
+  for (int a = c->quad_force ? 1 : 0; a < 2 && !err; a++)
+    for (int b = c->quad ? 1 : 0; b < 2 && !err; b++)
       for (int q = 0; q < 2 && !err; q++) {
         c->tb_force = tbs[a];
         c->tb_nr = tbs[b];
@@ -4908,6 +4915,12 @@ int ndsp_batch_autotune(ndsp_batch* b, int32_t reps, int32_t* choice) {
   std::vector<SavedState> S(ns);
   int err = 0;
   for (int s = 0; s < ns && !err; s++) err = save_state(b->sims[s], S[s]);
+  // the workgroup size is a choice where some group has kernels with one lane
+  // per particle
+  b->valid = false;
+  batch_group(b);
+  bool sized = false;
+  for (const auto& g : b->groups) sized = sized || !g.quad || !g.quad_force;
   const int tbs[2] = {64, 256}, subs[2] = {1, 2};
   int bt = b->tb, bc = b->sims[0]->p.cell_sub;
   double best = 1e300;
@@ -4917,7 +4930,7 @@ int ndsp_batch_autotune(ndsp_batch* b, int32_t reps, int32_t* choice) {
       if (int r = restore_state(b->sims[s], S[s])) e = e ? e : r;
     return e;
   };
-  for (int a = 0; a < 2 && !err; a++)
+  for (int a = sized ? 0 : 1; a < 2 && !err; a++)
     for (int q = 0; q < 2 && !err; q++) {
       b->tb = tbs[a];
       for (int s = 0; s < ns; s++) {
