@@ -735,16 +735,14 @@ __device__ __forceinline__ bool list_image(const Grid& g, int code, double* xj) 
 // calling body(kk, r, xj_img, flip, code) with r = load(kk) (a struct holding
 // the FP64 position and 1/h in r.p and whatever the pair sum reads) and the
 // image coordinates of the ghost arithmetic (so the exact FP64 tests see the
-// values of the cell scan).  Entries come four per load; the record of entry
-// m + PF (PF 1 or 2) is fetched while entry m is processed, so a wavefront's
-// gathers overlap its arithmetic (the pair passes use one ahead: a second
-// record in flight costs them a wave per SIMD).  The loop is unrolled over
-// the PF + 1 record buffers, which take turns as the current one, so no
-// record is copied.
-template <int NDIM, int PF = 1, typename LOAD, typename F>
+// values of the cell scan).  Entries come four per load; the next entry's
+// record is fetched while an entry is processed, so a wavefront's gathers
+// overlap its arithmetic (a second record in flight costs the pair passes a
+// wave per SIMD).  The loop is unrolled over the two record buffers, which
+// take turns as the current one, so no record is copied.
+template <int NDIM, typename LOAD, typename F>
 __device__ __forceinline__ void for_each_listed_pf(const KArgs& a, const Grid& g, int k, int cnt, LOAD&& load,
                                                    F&& body) {
-  static_assert(PF == 1 || PF == 2, "prefetch distance 1 or 2");
   if (cnt <= 0) return;
   const uint4* L4 = (const uint4*)(a.nbl + (size_t)k * a.maxnb);
   const int ng = (cnt + 3) >> 2;
@@ -756,10 +754,10 @@ __device__ __forceinline__ void for_each_listed_pf(const KArgs& a, const Grid& g
   const uint4 g1 = ng > 1 ? L4[1] : make_uint4(0u, 0u, 0u, 0u);
   unsigned c0 = g0.x, c1 = g0.y, c2 = g0.z, c3 = g0.w, n0 = g1.x, n1 = g1.y, n2 = g1.z, n3 = g1.w;
   int m = 0;
-  // entry m, its record in cur; the record of entry m + PF goes into nxt
+  // entry m, its record in cur; the next entry's record goes into nxt
   auto visit = [&](const auto& cur, auto& nxt) {
     const unsigned e = c0;
-    const unsigned en = m + PF < cnt ? (PF == 2 ? c2 : c1) : e;
+    const unsigned en = m + 1 < cnt ? c1 : e;
     nxt = load((int)(en >> 7));
     const int kk = (int)(e >> 7);
     const int code = (int)(e & 63u);
@@ -776,26 +774,12 @@ __device__ __forceinline__ void for_each_listed_pf(const KArgs& a, const Grid& g
     m++;
   };
   using R = decltype(load(0));
-  R rA = load((int)(c0 >> 7));
-  if constexpr (PF == 1) {
-    R rB;
-    for (;;) {
-      if (m >= cnt) break;
-      visit(rA, rB);
-      if (m >= cnt) break;
-      visit(rB, rA);
-    }
-  } else {
-    R rB = load((int)((cnt > 1 ? c1 : c0) >> 7));
-    R rC;
-    for (;;) {
-      if (m >= cnt) break;
-      visit(rA, rC);
-      if (m >= cnt) break;
-      visit(rB, rA);
-      if (m >= cnt) break;
-      visit(rC, rB);
-    }
+  R rA = load((int)(c0 >> 7)), rB;
+  for (;;) {
+    if (m >= cnt) break;
+    visit(rA, rB);
+    if (m >= cnt) break;
+    visit(rB, rA);
   }
 }
 
@@ -1466,8 +1450,9 @@ static RedSpec red_spec(std::initializer_list<std::pair<int, int>> q) {
 // current h (P4.w), and psi is left alone unless MHD is off.  sym = 0 is
 // density_partial (src/density_sums.f90:396): gather count, psi zeroed when
 // MHD is on (:630-635).  With persistent = 1 each particle keeps iterating
-// (partial passes) until it converges; otherwise an unconverged particle is
-// appended to next_list for the next launch.  Sums depend only on the
+// (partial passes) until it converges; otherwise the unconverged particles
+// are flagged, and k_pass_fold and k_pass_next make the next launch's list of
+// them, in order.  Sums depend only on the
 // particle's own h, so the per-particle sequence of h is the reference's.
 // ===========================================================================
 
@@ -1654,7 +1639,7 @@ __device__ __forceinline__ void b_nr_pass(KArgs a, Phys p, const Grid* __restric
       };
       if (!uselist) for_each_candidate_rec<NDIM, Q>(a, g, xi, rad, sub, loadj, body, flush);
       else if constexpr (Q == 4) for_each_listed_quad<NDIM>(a, g, k, nlisted, sub, loadj, body, flush);
-      else for_each_listed_pf<NDIM, 1>(a, g, k, nlisted, loadj, body);
+      else for_each_listed_pf<NDIM>(a, g, k, nlisted, loadj, body);
       npairs += (unsigned long long)ngat;
       nn = symp ? nsym : ngat;
       double sum[6];
@@ -2221,7 +2206,7 @@ __device__ __forceinline__ void b_force(KArgs a, Phys p, const Grid* __restrict_
       // third wave per SIMD (162 registers with one, 180 with two)
       if (!uselist) for_each_candidate_rec<NDIM, Q>(a, g, xi, rad, sub, loadj, body, flush);
       else if constexpr (Q == 4) for_each_listed_quad<NDIM>(a, g, k, a.nbc[k] + a.nbx[k], sub, loadj, body, flush);
-      else for_each_listed_pf<NDIM, 1>(a, g, k, a.nbc[k] + a.nbx[k], loadj, body);
+      else for_each_listed_pf<NDIM>(a, g, k, a.nbc[k] + a.nbx[k], loadj, body);
     }
     // (quantity, field) of every sum; the first lane of a quad stores
     auto out = [&](int field, const PSum<PT, Q>& x, int four, int lane_) {
@@ -3091,7 +3076,6 @@ struct MArgs {
   int nbp;        // binning-statistics blocks
   int nb_nr, nb_force, nb_256;  // blocks of the h-rho, force and elementwise launches
   double* scratch_d;  // REORDER_W fields of n doubles (or the five int fields) for reorders
-  int* scratch_i;
 };
 
 __device__ __forceinline__ int member_of(const int* __restrict__ off, int nm, int b) {
@@ -3250,8 +3234,12 @@ static double nexp_of(const Phys& p) {
   return 4.0 / 3.0 * M_PI * r * r * r;
 }
 
-// (33000 reals take 23 us this way and 200 with a copy command, 50000 take 250
-// and 42)
+// Downloads of at most this many reals are written into pinned memory by the
+// kernel and copied from there by the host: no copy command, 12 to 20 us less
+// at any size (medians of 30 into memory in use: 800 reals 14 us against 28,
+// 40000 26 against 38, 200000 91 against 109, 500000 220 against 240).  The
+// line lies where a context's pinned memory is 320 KB: a sweep keeps hundreds
+// of contexts, and from there on the copy itself is most of the time.
 static const size_t PIN_REALS = 40960;
 // Simulations up to this size run the h-rho passes with four lanes per particle
 // (b_nr_pass, Q = 4): with one lane they have fewer waves than the device has
@@ -3305,7 +3293,6 @@ struct ndsp_ctx {
   hipStream_t st = nullptr;
   KArgs a;
   double* scratch_d = nullptr;  // REORDER_W fields of n doubles for reorders
-  int* scratch_i = nullptr;
   int* bsum = nullptr;
   int* list_a = nullptr;        // active lists of the h-rho passes
   int* list_b = nullptr;
@@ -3937,7 +3924,6 @@ int ndsp_create(const int32_t* iopt, const double* dopt, int64_t npart, int32_t 
   hipMemset(c->fields, 0, field_stride(n) * F_NFIELDS);
   bool ok = true;
   ok &= hipMalloc(&c->scratch_d, sizeof(double) * n * REORDER_W) == hipSuccess;
-  ok &= hipMalloc(&c->scratch_i, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.itype, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.ireal, sizeof(int) * n) == hipSuccess;
   ok &= hipMalloc(&a.slot_of, sizeof(int) * n) == hipSuccess;
@@ -4022,7 +4008,7 @@ int ndsp_destroy(ndsp_ctx* c) {
   if (!c) return 0;
   if (c->st) hipStreamSynchronize(c->st);
   KArgs& a = c->a;
-  void* ptrs[] = {c->fields, c->fields_alt, c->scratch_d, c->scratch_i, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
+  void* ptrs[] = {c->fields, c->fields_alt, c->scratch_d, a.numneigh, a.nits, a.uid, a.itype, a.ireal, a.slot_of, a.cellid, a.sidx, a.P4, a.dxb,
                   a.DR, a.FR, a.GF, a.sc, (void*)a.tabf, (void*)a.tabd,
                   c->part, a.cstart, a.cfill, a.cpart, a.cellr, c->bsum, c->list_a, c->list_b, a.nrflag, a.nrcnt,
                   a.nbl, a.nbc, a.nbx, a.hcap, a.red, c->gdev};
@@ -4144,8 +4130,8 @@ int ndsp_download(ndsp_ctx* c, const char* name, double* out, int32_t* width) {
     }
   }
   if (w) {
-    // small fields straight into pinned host memory (no copy command), larger
-    // ones through the scratch (800 particles: 15 us instead of 29)
+    // small fields straight into pinned host memory, larger ones through the
+    // scratch (PIN_REALS)
     const size_t len = (size_t)n * w;
     const bool direct = len <= PIN_REALS;
     hipLaunchKernelGGL(k_to_caller, dim3(nblk(n)), dim3(BS), 0, c->st, cf, (const int*)c->a.slot_of,
@@ -4475,7 +4461,6 @@ static int batch_build(ndsp_batch* b) {
       M.nb_force = (int)nblk(n, g.quad_force ? 64 : b->tb);
       M.nb_256 = (int)nblk(n);
       M.scratch_d = c->scratch_d;
-      M.scratch_i = c->scratch_i;
       const int cnt[BGroup::NSHAPE] = {(int)nblk(n), (int)nblk(n, 64), 1, M.nbp,
                                        (int)((cap + BS * 4 - 1) / (BS * 4)), M.nb_nr, M.nb_force};
       for (int k = 0; k < BGroup::NSHAPE; k++) off[k].push_back(off[k].back() + cnt[k]);
