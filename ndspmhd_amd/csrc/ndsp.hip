@@ -964,7 +964,7 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
   // the widest search: the largest h of the binning
   const double rmax = p.radkern * s1 * (1.0 + 1.0e-6) * a.sc->hmax_bin;
   const int ue = __builtin_amdgcn_readfirstlane(ilogb(rmax));
-  const double us = ldexp(1.0, -ue), ui = ldexp(1.0, ue);
+  const float us = wave_uniform(ldexpf(1.0f, -ue)), limu = wave_uniform(limf * us);
   const int maxnb = a.maxnb;
   unsigned* const L = a.nbl + (size_t)(act ? k : 0) * maxnb;
   int cnt = 0, nx = 0;
@@ -994,7 +994,7 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
     const bool in = (seg >> lane) & 1ull;
     const double4 pk = a.P4[act ? k : a.n - 1];
     const double pk_x[3] = {pk.x, pk.y, pk.z};
-    const double wk = pk.w * ui;
+    const double wk = ldexp(pk.w, ue);
     const float rl2 = (float)(lim2 / (wk * wk));
     double lo[3] = {0.0, 0.0, 0.0}, hi[3] = {0.0, 0.0, 0.0};
     const float rw2 = wave_max_pos(in ? rl2 : 0.0f) * (1.0f + 1.0e-5f);
@@ -1006,7 +1006,7 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
       lo[d] = wave_extreme<false>(in ? pk_x[d] : DBL_MAX);
       hi[d] = wave_extreme<true>(in ? pk_x[d] : -DBL_MAX);
       org[d] = wave_uniform(0.5 * (lo[d] + hi[d]));
-      half[d] = wave_uniform((float)(0.5 * (hi[d] - lo[d]) * us) * (1.0f + 1.0e-6f));
+      half[d] = wave_uniform((float)(0.5 * (hi[d] - lo[d])) * us * (1.0f + 1.0e-6f));
       diag2 += half[d] * half[d];
       int c1, q;
       cell_range(g, d, lo[d], rmax, clo[d], q);
@@ -1025,7 +1025,7 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
     {
       float xr[3] = {0.0f, 0.0f, 0.0f}, p2 = 0.0f;
       for (int d = 0; d < NDIM; d++) {
-        xr[d] = in ? (float)((pk_x[d] - org[d]) * us) : 0.0f;
+        xr[d] = in ? (float)(pk_x[d] - org[d]) * us : 0.0f;
         p2 += xr[d] * xr[d];
       }
       const float pg = in ? p2 - rl2 : 1.0e30f, px = in ? p2 : 1.0e30f;
@@ -1108,10 +1108,10 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
         const double4 pi = a.P4[act ? k : a.n - 1];
         const double xi[3] = {pi.x, pi.y, pi.z};
         const double hi21 = pi.w * pi.w;
-        const double wi = pi.w * ui;
+        const double wi = ldexp(pi.w, ue);
         const float rl2 = (float)(lim2 / (wi * wi));
         float xr[3] = {0.0f, 0.0f, 0.0f};
-        for (int d = 0; d < NDIM; d++) xr[d] = (float)((xi[d] - org[d]) * us);
+        for (int d = 0; d < NDIM; d++) xr[d] = (float)(xi[d] - org[d]) * us;
         for (int t = 0; t < m; t++) {
           float r2 = 0.0f;
           for (int d = 0; d < NDIM; d++) {
@@ -1195,8 +1195,8 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
           ok = ok && src[d] >= 0;
           // distance of the cell (widened a little: a particle may be binned
           // next door by rounding) from the box
-          const float mid = (float)((g.lo[d] + (cc[d] + 0.5) * g.w[d] - org[d]) * us);
-          const float e = fmaxf(fabsf(mid) - half[d] - 0.50001f * (float)(g.w[d] * us), 0.0f);
+          const float mid = (float)(g.lo[d] + (cc[d] + 0.5) * g.w[d] - org[d]) * us;
+          const float e = fmaxf(fabsf(mid) - half[d] - 0.50001f * ((float)g.w[d] * us), 0.0f);
           d2 += e * e;
         }
         if (ok) {
@@ -1205,7 +1205,7 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
           if (NDIM >= 3) key |= key_part(g, 2, src[2]);
           cb = a.cstart[key];
           cn = a.cstart[key + 1] - cb;
-          const float cr = a.cellr[key] * (float)us;
+          const float cr = a.cellr[key] * us;
           cr2 = cr * cr * (1.0f + 1.0e-5f);
           if (d2 * (1.0f - 1.0e-4f) > fmaxf(rw2, cr2)) cn = 0;
           if (cn == 0) cr2 = 0.0f;
@@ -1238,11 +1238,11 @@ __device__ __forceinline__ void b_nblist(KArgs a, Phys p, const Grid* __restrict
             // kind 1: the image left of xmin; kind 2: right of xmax
             const unsigned kd = (ent >> (2 * d)) & 3u;
             const double Ld = g.xmax[d] - g.xmin[d];
-            rel[d] = (float)((xj[d] + (kd == 1u ? -Ld : kd == 2u ? Ld : 0.0) - org[d]) * us);
+            rel[d] = (float)(xj[d] + (kd == 1u ? -Ld : kd == 2u ? Ld : 0.0) - org[d]) * us;
             const float e = fmaxf(fabsf(rel[d]) - half[d], 0.0f);
             d2 += e * e;
           }
-          const float rj = limf * __builtin_amdgcn_rcpf((float)(pj.w * ui));
+          const float rj = limu * __builtin_amdgcn_rcpf((float)pj.w);
           const float rj2 = rj * rj;
           const bool keep = lane < nq - q && d2 * (1.0f - 1.0e-4f) <= fmaxf(rw2, rj2);
           const unsigned long long bal = __ballot(keep);
