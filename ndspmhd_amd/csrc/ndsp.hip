@@ -3481,7 +3481,8 @@ static int size_key_space(ndsp_ctx* c, const DScal& hs, int extra_bits) {
 // List capacity after a binning in which some rows overflowed (those
 // particles scanned cells, the slowest part of their launch): 1.5 times the
 // present one, up to four times the initial capacity; the old lists are
-// dropped (a binning follows) and recorded steps are recorded again.  A failed allocation keeps the present capacity for good.
+// dropped (a binning follows) and recorded steps are recorded again.  A failed
+// allocation keeps the present capacity for good.
 static int grow_lists(ndsp_ctx* c) {
   if (!c->p.use_list || c->a.maxnb >= c->maxnb_limit) return 0;
   const int m = std::min(c->maxnb_limit, (c->a.maxnb * 3 / 2 + 31) / 32 * 32);
